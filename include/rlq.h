@@ -191,7 +191,9 @@ void rlq_weights_stack(const rlq_weights *w, uint64_t *n2, uint64_t *n3);
  * x[b*cols ..] is quantized to the weights' activation type on the GPU, then
  * y[b*rows + r] = dot_packed(weights row r, activation b).  x and y are
  * device pointers (x 16-byte aligned).  Up to 8 columns share one pass over
- * the weights.  A call takes at most 8388606 columns (the error keys carry
+ * the weights; more run a GEMM over an image of the quantized columns in the
+ * context's scratch (while `stream` is being captured, types other than Q4_K
+ * run passes of 8 columns, which need none).  A call takes at most 8388606 columns (the error keys carry
  * the column): more return RLQ_UNIMPLEMENTED (a = batch, b = the limit), as
  * do rlq_matmul_argmax, rlq_matmul_noalloc and rlq_quantize_device. */
 int32_t rlq_matmul(rlq_context *ctx, const rlq_weights *w, const float *x, uint64_t batch, float *y,
@@ -218,11 +220,12 @@ int32_t rlq_matmul_argmax(rlq_context *ctx, const rlq_weights *w, const float *x
  * memory (code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc).  rlq_matmul (argmax null) or rlq_matmul_argmax (argmax
  * non-null) on the same kernels, with the same results, that allocates and
- * frees nothing: the argmax keys and the prefill GEMM's activation image
- * (batches above 8 of Q4_K weights) live in a static 32 MiB device array
- * that each GPU holds until the process ends.  A call whose workspace
- * exceeds it returns RLQ_SCRATCH_LIMIT (a = bytes needed, b = 33554432); for
- * 4096 columns that is a batch of about 3,700.  Every call on one GPU, from
+ * frees nothing: the argmax keys and the GEMMs' activation images (batches
+ * above 8) live in a static 32 MiB device array that each GPU holds until the
+ * process ends.  A call with Q4_K weights whose workspace exceeds it returns
+ * RLQ_SCRATCH_LIMIT (a = bytes needed, b = 33554432); for 4096 columns that is
+ * a batch of about 3,700.  With other weights such a call runs passes of 8
+ * columns.  Every call on one GPU, from
  * any context, shares that GPU's array: calls that overlap on one GPU (other
  * streams, other threads) race and must be ordered by the caller. */
 int32_t rlq_matmul_noalloc(rlq_context *ctx, const rlq_weights *w, const float *x, uint64_t batch, float *y,

@@ -80,7 +80,7 @@ bool path_weight(uint32_t t) {
 }
 
 // Batches up to this size run the decode kernels (one pass over the weights
-// per 8 columns); larger Q4_K batches run the prefill GEMM.
+// per 8 columns); larger ones a GEMM (matmul_route).
 constexpr uint64_t kDecodeMaxBatch = 8;
 
 // ---- device buffers ---------------------------------------------------------
@@ -598,6 +598,54 @@ static hipError_t decode_launch(rlq_context* ctx, const rlq_weights* w, const fl
 // model runtime's field 0x7fffff (rlq_device.hpp).
 constexpr uint64_t kMaxKeyColumns = (1ull << 23) - 2;
 
+// How a product of `batch` f32 columns runs: the decode kernels (passes of up to
+// 8 columns), the 128-column Q4_K GEMM, or the int8 GEMM of every format.
+enum class Route { kDecode, kGemm, kIgemm };
+
+// The Q4_K GEMM's workgroups take 128 columns x 256 rows and one CU each: from
+// three quarters of the CUs on it is the faster one (14336x4096, 512 columns =
+// 224 workgroups: 73 us against 95), below that the int8 GEMM's smaller tiles
+// are (4096x4096, 512 columns = 64 workgroups: 37 us).  Q8_0 and Q2_K cannot
+// split K (their sums have one order), so few columns of a long row are faster
+// in decode passes, which do (4096x14336 Q8_0, 16 columns: 60 us against 137).
+static Route matmul_route(uint32_t dtype, uint64_t rows, uint64_t batch) {
+    if (batch <= kDecodeMaxBatch) return Route::kDecode;
+    if (dtype == kQ4_K) return (rows + 255) / 256 * ((batch + 127) / 128) >= 192 ? Route::kGemm : Route::kIgemm;
+    return (dtype == kQ8_0 || dtype == kQ2_K) && batch <= 32 ? Route::kDecode : Route::kIgemm;
+}
+
+static size_t route_bytes(Route r, uint32_t dtype, uint64_t batch, uint64_t cols) {
+    return r == Route::kGemm ? gemm_planes_bytes(batch, cols) : r == Route::kIgemm ? igemm_bytes(dtype, batch, cols) : 0;
+}
+
+// The GEMM of a route other than kDecode over `scratch` (route_bytes), then the
+// argmax over the stored rows (keys: one u64 per column, or null).
+static int32_t gemm_launch(rlq_context* ctx, const rlq_weights* w, Route r, const float* x, uint64_t batch, float* y,
+                           void* scratch, unsigned long long* keys, uint32_t* argmax, hipStream_t s, rlq_error* err) {
+    if (r == Route::kGemm)
+        HIP_TRY(launch_gemm_q4k(w->dev, w->rows, w->cols, x, batch, y, w->rows, scratch, ctx->err_words, nullptr, nullptr,
+                                s));
+    else
+        HIP_TRY(launch_igemm(w->dtype, w->dev, w->rows, w->cols, x, batch, y, w->rows, scratch, ctx->err_words, s));
+    if (argmax) {
+        HIP_TRY(launch_fill_u64(keys, batch, 0ull, s));
+        HIP_TRY(launch_argmax_rows(y, batch, w->rows, keys, s));
+        HIP_TRY(launch_argmax_finish(keys, batch, y, w->rows, argmax, s));
+    }
+    return ok(err);
+}
+
+// Whether the stream records a graph (or HIP will not say).
+static bool capturing(hipStream_t s) {
+    if (!s) return false;  // the null stream cannot be captured
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &st) != hipSuccess) {
+        (void)hipGetLastError();
+        return true;
+    }
+    return st != hipStreamCaptureStatusNone;
+}
+
 static int32_t matmul_impl(rlq_context* ctx, const rlq_weights* w, const float* x, uint64_t batch, float* y,
                            uint32_t* argmax, void* stream, rlq_error* err) {
     if (!ctx || !w || !x || !y) return fail(err, RLQ_INVALID_ARGUMENT);
@@ -606,26 +654,25 @@ static int32_t matmul_impl(rlq_context* ctx, const rlq_weights* w, const float* 
     if (batch > kMaxKeyColumns) return fail(err, RLQ_UNIMPLEMENTED, w->dtype, batch, kMaxKeyColumns);
     DeviceGuard g(ctx->device);
     const hipStream_t s = pick(ctx, stream);
-    const bool gemm = w->dtype == kQ4_K && batch > kDecodeMaxBatch;
+    Route route = matmul_route(w->dtype, w->rows, batch);
+    // A graph keeps the addresses it was captured with, and the context's
+    // scratch may be replaced by a later, larger call: what needs no scratch
+    // (every type but Q4_K) is recorded as decode passes.
+    if (route == Route::kIgemm && w->dtype != kQ4_K && capturing(s)) route = Route::kDecode;
     if (argmax) {
         bool grown = false;
-        HIP_TRY(ensure(ctx, ctx->keys, kArgmaxStateBytes + (gemm ? batch * sizeof(unsigned long long) : 0), &grown));
+        HIP_TRY(ensure(ctx, ctx->keys,
+                       kArgmaxStateBytes + (route != Route::kDecode ? batch * sizeof(unsigned long long) : 0), &grown));
         if (grown) HIP_TRY(launch_fill_u64((unsigned long long*)ctx->keys.p, 1, 0ull, s));  // the arrival counter
     }
-    if (gemm) {  // prefill: the MFMA GEMM, then the argmax over the stored rows
-        HIP_TRY(ensure(ctx, ctx->planes, gemm_planes_bytes(batch, w->cols)));
-        HIP_TRY(launch_gemm_q4k(w->dev, w->rows, w->cols, x, batch, y, w->rows, ctx->planes.p, ctx->err_words, nullptr,
-                                nullptr, s));
-        if (argmax) {
-            unsigned long long* keys = (unsigned long long*)((uint8_t*)ctx->keys.p + kArgmaxStateBytes);
-            HIP_TRY(launch_fill_u64(keys, batch, 0ull, s));
-            HIP_TRY(launch_argmax_rows(y, batch, w->rows, keys, s));
-            HIP_TRY(launch_argmax_finish(keys, batch, y, w->rows, argmax, s));
-        }
-    } else {  // decode: the argmax is finished inside each launch
-        const MvArgmax am = argmax_state(ctx->keys.p, argmax);
-        HIP_TRY(decode_launch(ctx, w, x, batch, y, argmax ? &am : nullptr, nullptr, nullptr, MvExtra{}, s));
+    if (route != Route::kDecode) {
+        HIP_TRY(ensure(ctx, ctx->planes, route_bytes(route, w->dtype, batch, w->cols)));
+        return gemm_launch(ctx, w, route, x, batch, y, ctx->planes.p,
+                           (unsigned long long*)((uint8_t*)ctx->keys.p + kArgmaxStateBytes), argmax, s, err);
     }
+    // decode: the argmax is finished inside each launch
+    const MvArgmax am = argmax_state(ctx->keys.p, argmax);
+    HIP_TRY(decode_launch(ctx, w, x, batch, y, argmax ? &am : nullptr, nullptr, nullptr, MvExtra{}, s));
     return ok(err);
 }
 
@@ -664,30 +711,30 @@ int32_t rlq_matmul_noalloc(rlq_context* ctx, const rlq_weights* w, const float* 
     if (((uintptr_t)x & 15) || ((uintptr_t)y & 3)) return fail(err, RLQ_INVALID_ARGUMENT, w->dtype);
     if (batch == 0) return ok(err);
     if (batch > kMaxKeyColumns) return fail(err, RLQ_UNIMPLEMENTED, w->dtype, batch, kMaxKeyColumns);
-    const bool gemm = w->dtype == kQ4_K && batch > kDecodeMaxBatch;
+    Route route = matmul_route(w->dtype, w->rows, batch);
     const uint64_t state_bytes = argmax ? kArgmaxStateBytes : 0;
-    const uint64_t keys_bytes = argmax && gemm ? (batch * 8 + 255) / 256 * 256 : 0;
-    const uint64_t need = state_bytes + keys_bytes + (gemm ? gemm_planes_bytes(batch, w->cols) : 0);
+    uint64_t keys_bytes = argmax && route != Route::kDecode ? (batch * 8 + 255) / 256 * 256 : 0;
+    // the limit of Q4_K stays that of the larger image, whichever GEMM runs
+    uint64_t need = state_bytes + keys_bytes +
+                    (w->dtype == kQ4_K && route != Route::kDecode ? gemm_planes_bytes(batch, w->cols)
+                                                                  : route_bytes(route, w->dtype, batch, w->cols));
+    if (need > kScratchBytes && w->dtype != kQ4_K) {  // decode passes need no image
+        route = Route::kDecode;
+        keys_bytes = 0;
+        need = state_bytes;
+    }
     if (need > kScratchBytes) return fail(err, RLQ_SCRATCH_LIMIT, w->dtype, need, kScratchBytes);
     if (!ctx->scratch) return fail(err, RLQ_INVALID_ARGUMENT, w->dtype);
     DeviceGuard g(ctx->device);
     const hipStream_t s = pick(ctx, stream);
     // the scratch keeps the last call's contents: what must start at 0 is cleared
     if (argmax) HIP_TRY(launch_fill_u64((unsigned long long*)ctx->scratch, 1, 0ull, s));  // the arrival counter
-    if (gemm) {
-        HIP_TRY(launch_gemm_q4k(w->dev, w->rows, w->cols, x, batch, y, w->rows, ctx->scratch + state_bytes + keys_bytes,
-                                ctx->err_words, nullptr, nullptr, s));
-        if (argmax) {
-            unsigned long long* keys = (unsigned long long*)(ctx->scratch + state_bytes);
-            HIP_TRY(launch_fill_u64(keys, batch, 0ull, s));
-            HIP_TRY(launch_argmax_rows(y, batch, w->rows, keys, s));
-            HIP_TRY(launch_argmax_finish(keys, batch, y, w->rows, argmax, s));
-        }
-    } else {
-        const MvArgmax am = argmax_state(ctx->scratch, argmax);
-        HIP_TRY(launch_matvec(w->dtype, w->dev, w->rows, w->cols, x, nullptr, batch, y, w->rows,
-                              argmax ? &am : nullptr, ctx->err_words, nullptr, nullptr, s));
-    }
+    if (route != Route::kDecode)
+        return gemm_launch(ctx, w, route, x, batch, y, ctx->scratch + state_bytes + keys_bytes,
+                           (unsigned long long*)(ctx->scratch + state_bytes), argmax, s, err);
+    const MvArgmax am = argmax_state(ctx->scratch, argmax);
+    HIP_TRY(launch_matvec(w->dtype, w->dev, w->rows, w->cols, x, nullptr, batch, y, w->rows, argmax ? &am : nullptr,
+                          ctx->err_words, nullptr, nullptr, s));
     return ok(err);
 }
 

@@ -141,6 +141,14 @@ hipError_t launch_gemm_q4k(const uint8_t* w, uint64_t rows, uint64_t cols, const
                            uint64_t ldy, void* scratch, unsigned long long* err_word, int32_t* dbg_isum,
                            int32_t* dbg_imin, hipStream_t s);
 
+// ---- igemm.hip ----
+// The int8 GEMM of every weight format: y[m*ldy + r] = dot(row r, column m) for
+// m < M, x [M][cols] f32 quantized into `scratch` (igemm_bytes) first.  A data
+// error in any column goes to `err_word` and suppresses every output.
+size_t igemm_bytes(uint32_t t, uint64_t M, uint64_t cols);
+hipError_t launch_igemm(uint32_t t, const uint8_t* w, uint64_t rows, uint64_t cols, const float* x, uint64_t M, float* y,
+                        uint64_t ldy, void* scratch, unsigned long long* err_word, hipStream_t s);
+
 // ---- llama.hip ----
 // The dense Llama decode step (crates/model-runtime/src/llama.rs:222-392)
 // over resident weights.  Dimensions are validated by the caller.

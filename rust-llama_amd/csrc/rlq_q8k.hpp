@@ -117,6 +117,41 @@ __device__ __forceinline__ Q8KRow q8k_row16(const float (&v)[16], uint32_t r16) 
     return o;
 }
 
+// Half a Q8_0 block (encode.rs:115-126, 151-192), 16 values per lane; the lanes
+// of a quad pair hold the two halves of one block (odd: the second).  q: the
+// lane's 16 int8; d: the f32 of the stored f16 scale.  Returns -1, or the kind
+// of the block's data error (q and d then 0; index: the first non-finite value
+// within the block).
+__device__ __forceinline__ int q8_0_pair16(const float (&v)[16], uint32_t odd, uint32_t (&q)[4], float& d,
+                                           uint32_t& index) {
+    q[0] = q[1] = q[2] = q[3] = 0;
+    d = 0.0f;
+    uint32_t nf = 0xffffffffu;
+#pragma unroll
+    for (int k = 15; k >= 0; --k)
+        if (!finite(v[k])) nf = odd * 16 + k;
+    index = umin_(nf, (uint32_t)dpp_i<kQuadXor1>((int32_t)nf));
+    float am = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) am = fmaxf(am, fabsf(v[k]));
+    am = fmaxf(am, dpp_f<kQuadXor1>(am));
+    if (index != 0xffffffffu) return kKindNonFinite;
+    const float df = am / 127.0f;
+    const uint32_t dh = float_to_half_bits(df);
+    // preflight (encode.rs:80-90): d, 1/d and the stored half must be finite
+    if (!finite(df) || (df != 0.0f && !finite(1.0f / df)) || (dh & 0x7c00u) == 0x7c00u) return kKindScale;
+    const float inv = df != 0.0f ? 1.0f / df : 0.0f;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+        // `(x * inv).round() as i8`: half away from zero, saturating
+        float r = __builtin_roundf(v[k] * inv);
+        r = r > 127.0f ? 127.0f : (r < -128.0f ? -128.0f : r);
+        q[k / 4] |= ((uint32_t)(int32_t)r & 0xffu) << (8 * (k % 4));
+    }
+    d = half_bits_to_float_exact(dh);
+    return -1;
+}
+
 // The Q4_K / Q5_K slot order of an activation image (rlq_layout.hpp,
 // q45_pos_of_slot): the two lanes of a quad pair hold the 16 values of one
 // sub-block half each (lane bit 0 = half h'), q their natural bytes.  Slot
