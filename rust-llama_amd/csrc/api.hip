@@ -462,6 +462,37 @@ int32_t mm_stage(rlq_context* ctx, const rlq_weights* w, uint32_t at, uint32_t x
     return ok(err);
 }
 
+// Q4_K / Q5_K columns from this many per launch on are quantized once by the
+// planes kernel instead of in every workgroup's prologue (with one workgroup
+// per CU; 14336x4096 batch 8: 12.6 us for both launches against 12.9 us
+// fused, batch 6: 12.5 against 11.8; 6144x4096 batch 8: 9.8 against 10.9).
+constexpr uint64_t kPlanesMinBatch = 7;
+
+// The decode launch of `batch` (<= 8) f32 columns: the fused kernels, or the
+// Q8_K planes kernel and then the matvec over the planes.
+hipError_t decode_launch(rlq_context* ctx, const rlq_weights* w, const float* x, uint64_t batch, float* y,
+                         const MvArgmax* am, int32_t* isum, int32_t* imin, const MvExtra& ex, hipStream_t s) {
+    if ((w->dtype == kQ4_K || w->dtype == kQ5_K) && batch >= kPlanesMinBatch && ex.epilogue == 0) {
+        hipError_t e = ensure(ctx, ctx->planes, act_planes_bytes(kQ8_K, w->cols, batch));
+        if (e != hipSuccess) return e;
+        const ActPlanes pl = act_planes_carve(ctx->planes.p, kQ8_K, w->cols, batch);
+        e = launch_quantize_q8k(x, w->cols, batch, &pl, nullptr, ctx->err_words, s);
+        if (e != hipSuccess) return e;
+        return launch_matvec_ex(w->dtype, w->dev, w->rows, w->cols, nullptr, &pl, batch, y, w->rows, am,
+                                ctx->err_words, isum, imin, ex, s);
+    }
+    return launch_matvec_ex(w->dtype, w->dev, w->rows, w->cols, x, nullptr, batch, y, w->rows, am, ctx->err_words,
+                            isum, imin, ex, s);
+}
+
+// Whether several matrices' products may run on the int8 GEMM.  Packed Q8_K
+// columns bring their own 16-value sums, which the GEMM takes as f16 and so
+// only from its own quantizer: formats with mins keep the decode kernels then.
+// (The GEMM reads packed blocks in words, the decode path's unpacker in bytes.)
+bool mm_igemm_takes(uint32_t dtype, uint32_t x_dtype, const void* x) {
+    return x_dtype == 0 || (!(dtype == kQ2_K || dtype == kQ4_K || dtype == kQ5_K) && ((uintptr_t)x & 3) == 0);
+}
+
 // Common argument checks: (x_dtype, x alignment, column count).
 int32_t mm_check_rhs(const rlq_weights* w, uint32_t at, uint32_t x_dtype, const void* x, const float* y,
                      uint64_t columns, rlq_error* err) {
@@ -496,6 +527,26 @@ int32_t rlq_mul_mat(rlq_context* ctx, const rlq_weights* w, uint32_t x_dtype, co
     if (columns == 1 && x_dtype == 0) {  // one f32 column: one launch that quantizes it in every workgroup
         HIP_TRY(launch_matvec_ex(w->dtype, w->dev, w->rows, w->cols, (const float*)x, nullptr, 1, y, w->rows,
                                  nullptr, ctx->err_words, nullptr, nullptr, MvExtra{}, s));
+        return ok(err);
+    }
+    // the columns of one matrix are contiguous over the r2 slices it serves
+    const IgStack st{n3 * w->n2, n2 / w->n2 * ncols, w->n2, n3 / w->n3, w->mat_bytes};
+    // two to eight f32 columns of one matrix: the one launch of rlq_matmul
+    if (columns <= kDecodeMaxBatch && st.groups == 1 && x_dtype == 0 && ncols > 1) {
+        HIP_TRY(decode_launch(ctx, w, (const float*)x, columns, y, nullptr, nullptr, nullptr, MvExtra{}, s));
+        return ok(err);
+    }
+    // The GEMM's two launches against one decode launch per slice after the
+    // quantizer and the gate: always fewer (Q4_K 4096x4096, 4 matrices of 2
+    // slices of 4 columns: 25 us against 66; one matrix, 100 columns: 25 against
+    // 103).  Single columns keep the decode kernels, whose sums are in the
+    // reference's order; Q8_0 and Q2_K, whose sums are so in both, take the GEMM
+    // for more than 32 columns a matrix (matmul_route).
+    const bool ordered = w->dtype == kQ8_0 || w->dtype == kQ2_K;
+    if (mm_igemm_takes(w->dtype, x_dtype, x) && (ordered ? st.cpg > 32 : ncols > 1)) {
+        HIP_TRY(ensure(ctx, ctx->planes, igemm_bytes(w->dtype, st.groups, st.cpg, w->cols)));
+        HIP_TRY(launch_igemm(w->dtype, w->dev, w->rows, w->cols, x, x_dtype != 0, st, y, w->rows, ctx->planes.p,
+                             ctx->err_words, s));
         return ok(err);
     }
     ActPlanes planes;
@@ -559,6 +610,19 @@ int32_t rlq_mul_mat_id(rlq_context* ctx, const rlq_weights* w, uint32_t x_dtype,
                                  nullptr, ctx->err_words, nullptr, nullptr, ex, s));
         return ok(err);
     }
+    // The decode launch reads a matrix per pair, the GEMM every matrix in use
+    // once, with one launch and the padding of its tiles on top: from 80 MB of
+    // matrices read again on it is the faster one (8 Q4_K experts of 14336x4096:
+    // 8 pairs 50 us against 55, 16 pairs 95 against 71, 90 pairs 526 against 72;
+    // of 4096x2048: 16 pairs 20 against 26, 32 pairs 32 against 26).
+    const uint64_t again = (pairs - (pairs < w->n2 ? pairs : w->n2)) * w->mat_bytes;
+    if (again >= (80ull << 20) && w->n2 <= kIgMaxMats && pairs <= 0x7fffffull && mm_igemm_takes(w->dtype, x_dtype, x)) {
+        const IgRoute r{ids, (uint32_t)pairs, (uint32_t)w->n2, (uint32_t)columns, (uint32_t)slots, (uint32_t)ncols};
+        HIP_TRY(ensure(ctx, ctx->planes, igemm_ids_bytes(w->dtype, w->cols, r)));
+        HIP_TRY(launch_igemm_ids(w->dtype, w->dev, w->rows, w->cols, w->mat_bytes, x, x_dtype != 0, r, y, w->rows,
+                                 ctx->planes.p, ctx->err_words, s));
+        return ok(err);
+    }
     ActPlanes planes;
     uint32_t* gate;
     rc = mm_stage(ctx, w, at, x_dtype, x, columns, ids, pairs, y, s, &planes, &gate, err);
@@ -570,29 +634,6 @@ int32_t rlq_mul_mat_id(rlq_context* ctx, const rlq_weights* w, uint32_t x_dtype,
 }
 
 // ---- device matmul --------------------------------------------------------------
-
-// Q4_K / Q5_K columns from this many per launch on are quantized once by the
-// planes kernel instead of in every workgroup's prologue (with one workgroup
-// per CU; 14336x4096 batch 8: 12.6 us for both launches against 12.9 us
-// fused, batch 6: 12.5 against 11.8; 6144x4096 batch 8: 9.8 against 10.9).
-constexpr uint64_t kPlanesMinBatch = 7;
-
-// The decode launch of `batch` (<= 8) f32 columns: the fused kernels, or the
-// Q8_K planes kernel and then the matvec over the planes.
-static hipError_t decode_launch(rlq_context* ctx, const rlq_weights* w, const float* x, uint64_t batch, float* y,
-                                const MvArgmax* am, int32_t* isum, int32_t* imin, const MvExtra& ex, hipStream_t s) {
-    if ((w->dtype == kQ4_K || w->dtype == kQ5_K) && batch >= kPlanesMinBatch && ex.epilogue == 0) {
-        hipError_t e = ensure(ctx, ctx->planes, act_planes_bytes(kQ8_K, w->cols, batch));
-        if (e != hipSuccess) return e;
-        const ActPlanes pl = act_planes_carve(ctx->planes.p, kQ8_K, w->cols, batch);
-        e = launch_quantize_q8k(x, w->cols, batch, &pl, nullptr, ctx->err_words, s);
-        if (e != hipSuccess) return e;
-        return launch_matvec_ex(w->dtype, w->dev, w->rows, w->cols, nullptr, &pl, batch, y, w->rows, am,
-                                ctx->err_words, isum, imin, ex, s);
-    }
-    return launch_matvec_ex(w->dtype, w->dev, w->rows, w->cols, x, nullptr, batch, y, w->rows, am, ctx->err_words,
-                            isum, imin, ex, s);
-}
 
 // Columns per call: an error key holds column + 1 in 23 bits below the
 // model runtime's field 0x7fffff (rlq_device.hpp).
@@ -615,7 +656,7 @@ static Route matmul_route(uint32_t dtype, uint64_t rows, uint64_t batch) {
 }
 
 static size_t route_bytes(Route r, uint32_t dtype, uint64_t batch, uint64_t cols) {
-    return r == Route::kGemm ? gemm_planes_bytes(batch, cols) : r == Route::kIgemm ? igemm_bytes(dtype, batch, cols) : 0;
+    return r == Route::kGemm ? gemm_planes_bytes(batch, cols) : r == Route::kIgemm ? igemm_bytes(dtype, 1, batch, cols) : 0;
 }
 
 // The GEMM of a route other than kDecode over `scratch` (route_bytes), then the
@@ -626,7 +667,8 @@ static int32_t gemm_launch(rlq_context* ctx, const rlq_weights* w, Route r, cons
         HIP_TRY(launch_gemm_q4k(w->dev, w->rows, w->cols, x, batch, y, w->rows, scratch, ctx->err_words, nullptr, nullptr,
                                 s));
     else
-        HIP_TRY(launch_igemm(w->dtype, w->dev, w->rows, w->cols, x, batch, y, w->rows, scratch, ctx->err_words, s));
+        HIP_TRY(launch_igemm(w->dtype, w->dev, w->rows, w->cols, x, false, IgStack{1, batch, 1, 1, 0}, y, w->rows, scratch,
+                             ctx->err_words, s));
     if (argmax) {
         HIP_TRY(launch_fill_u64(keys, batch, 0ull, s));
         HIP_TRY(launch_argmax_rows(y, batch, w->rows, keys, s));

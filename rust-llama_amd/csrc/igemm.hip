@@ -77,19 +77,42 @@ static IgImage ig_carve(void* base, uint32_t t, uint64_t tiles, uint64_t cols) {
     return IgImage{(uint8_t*)base, (uint32_t*)((uint8_t*)base + n * ig_pieces(t) * 1024), (uint32_t)ig_chunks(cols)};
 }
 
+// Which matrix and column an image column stands for.  Products of one or more
+// matrices whose columns are contiguous: `groups` of cpg columns, tpg tiles
+// each; group k uses matrix k / wn2 / r3 * wn2 + k % wn2 (MUL_MAT broadcast).
+// Or dealt by igemm_route_kernel (tile_mat non-null): the matrix of each tile,
+// kIgZero for products without one (their rows are 0) and columns no product
+// uses, kIgNone for unused tiles; per image column its source and its output
+// row (-1: none).
+constexpr uint32_t kIgNone = ~0u, kIgZero = ~0u - 1;
+struct IgMap {
+    uint32_t cpg, tpg, wn2, r3;
+    const uint32_t* tile_mat;
+    const int32_t *src, *row;
+};
+
 // Columns of one (tile, chunk): 16 lanes per column, lane r16 holding positions
-// 16 r16 .. +15.  From f32 (x) or from the quantized planes; `map` (may be
-// null: the identity below M) gives each image column's source, -1 for none.
-template <uint32_t T>
-__global__ __launch_bounds__(512) void igemm_act_kernel(const float* __restrict__ x, ActPlanes pl,
-                                                        const int32_t* __restrict__ map, uint32_t M, uint32_t K,
+// 16 r16 .. +15, from f32 rows (x) or from rows of packed Q8_K / Q8_0 blocks
+// (taken as given).
+template <uint32_t T, bool PACKED>
+__global__ __launch_bounds__(512) void igemm_act_kernel(const void* __restrict__ xsrc, IgMap map, uint32_t K,
                                                         uint32_t nchunk, uint8_t* __restrict__ img,
                                                         uint32_t* __restrict__ flags, unsigned long long* err_word,
                                                         const uint32_t* gate) {
     if (gate && *gate) return;
     const uint32_t c = blockIdx.x % nchunk, tile = blockIdx.x / nchunk;
-    const uint32_t r16 = threadIdx.x & 15, tok = threadIdx.x >> 4, slot = tile * kIgTok + tok;
-    const int64_t m = map ? (int64_t)map[slot] : (slot < M ? (int64_t)slot : -1);
+    const uint32_t r16 = threadIdx.x & 15, tok = threadIdx.x >> 4;
+    int64_t m = -1;
+    if (map.tile_mat) {
+        if (map.tile_mat[tile] == kIgNone) {
+            if (threadIdx.x == 0) flags[blockIdx.x] = 0;
+            return;
+        }
+        m = map.src[tile * kIgTok + tok];
+    } else {
+        const uint32_t g = tile / map.tpg, j = tile % map.tpg * kIgTok + tok;
+        if (j < map.cpg) m = (int64_t)g * map.cpg + j;
+    }
     const uint32_t e0 = c * 256 + r16 * 16;
     const bool live = m >= 0 && e0 < K;
     uint8_t* out = img + (uint64_t)blockIdx.x * (ig_pieces(T) * 1024);
@@ -97,12 +120,27 @@ __global__ __launch_bounds__(512) void igemm_act_kernel(const float* __restrict_
     float d = 0.0f;
     int32_t bsum = 0;
     int bad = 0;
-    if (x) {
+    if constexpr (PACKED) {
+        if (live) {
+            if constexpr (T == kQ8_0) {
+                const uint16_t* b = (const uint16_t*)((const uint8_t*)xsrc + ((uint64_t)m * (K / 32) + e0 / 32) * 34);
+                d = half_bits_to_float_exact(b[0]);
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+                    q[k] = (uint32_t)b[1 + 8 * (r16 & 1) + 2 * k] | (uint32_t)b[2 + 8 * (r16 & 1) + 2 * k] << 16;
+            } else {
+                const uint32_t* b = (const uint32_t*)((const uint8_t*)xsrc + ((uint64_t)m * (K / 256) + c) * 292);
+                d = __uint_as_float(b[0]);
+#pragma unroll
+                for (int k = 0; k < 4; ++k) q[k] = b[1 + 4 * r16 + k];
+            }
+        }
+    } else {
         float v[16];
 #pragma unroll
         for (int k = 0; k < 16; ++k) v[k] = 0.0f;
         if (live) {
-            const float4* src = (const float4*)(x + (uint64_t)m * K + e0);
+            const float4* src = (const float4*)((const float*)xsrc + (uint64_t)m * K + e0);
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
                 const float4 f = src[k];
@@ -132,11 +170,6 @@ __global__ __launch_bounds__(512) void igemm_act_kernel(const float* __restrict_
                                                : error_key((uint64_t)m, kKindScale, c));
             }
         }
-    } else if (live) {  // the planes were checked before the gate was written
-        const uint4 w = *(const uint4*)(pl.q + (uint64_t)m * K + e0);
-        q[0] = w.x, q[1] = w.y, q[2] = w.z, q[3] = w.w;
-        d = T == kQ8_0 ? pl.d[(uint64_t)m * (K / 32) + e0 / 32] : pl.d[(uint64_t)m * (K / 256) + c];
-        if (ig_mins(T)) bsum = pl.bsum[((uint64_t)m * K + e0) / 16];
     }
     const uint4 w = ig_slots(T) ? q45_slots(q, r16 & 1) : make_uint4(q[0], q[1], q[2], q[3]);
     *(uint4*)(out + (r16 >> 1) * 1024 + (r16 & 1) * 512 + tok * 16) = w;
@@ -147,7 +180,7 @@ __global__ __launch_bounds__(512) void igemm_act_kernel(const float* __restrict_
     }
     if constexpr (ig_mins(T))
         *(_Float16*)(out + kIgBsum + (r16 >> 3) * 512 + tok * 16 + (r16 & 7) * 2) = (_Float16)bsum;
-    bad = __syncthreads_or(bad);
+    if (!PACKED) bad = __syncthreads_or(bad);
     if (threadIdx.x == 0) flags[blockIdx.x] = (uint32_t)bad;
 }
 
@@ -441,16 +474,12 @@ struct IgArgs {
     const uint8_t* img;
     const uint32_t* flags;
     uint32_t nflags;
-    uint32_t M;       // columns
     uint32_t NT, MT;  // workgroup tiles along rows and columns
     float* y;
     uint64_t ldy;
-    const uint32_t* gate;
-    // MUL_MAT_ID: the expert of each image tile (~0u: none) and the output row
-    // of each image column (-1: none)
-    const uint32_t* tile_expert;
-    const int32_t* slot_row;
-    uint64_t expert_bytes;
+    const uint32_t* gate;  // nonzero: the call was refused (igemm_route_kernel)
+    IgMap map;
+    uint64_t mat_bytes;  // between the stack's matrices
 };
 
 __device__ __forceinline__ i32x16 ig_mfma(i32x4 a, i32x4 b, i32x16 c) {
@@ -497,11 +526,16 @@ __global__ __launch_bounds__(256, TT == 1 ? 3 : 2) void igemm_kernel(IgArgs g) {
     const uint32_t id = xcd * per + (xcd < rest ? xcd : rest) + blockIdx.x / 8;
     const uint32_t nt = id / g.MT, mt = id % g.MT;
     const uint8_t* w = g.w;
-    if (g.tile_expert) {
-        const uint32_t e = g.tile_expert[mt * TT];
-        if (e == ~0u) return;
-        w += (uint64_t)e * g.expert_bytes;
+    uint32_t mat = 0;
+    if (g.map.tile_mat) {
+        mat = g.map.tile_mat[mt * TT];
+        if (mat == kIgNone) return;
+    } else {
+        const uint32_t k = mt * TT / g.map.tpg;
+        if (mt * TT % g.map.tpg * kIgTok >= g.map.cpg) return;  // a tile of padding
+        mat = k / g.map.wn2 / g.map.r3 * g.map.wn2 + k % g.map.wn2;
     }
+    if (mat != kIgZero) w += (uint64_t)mat * g.mat_bytes;
     const uint32_t nchunk = g.nchunk, steps = (nchunk + KS - 1) / KS;
     uint32_t t16 = (nt * RW + rw) * 2 + (ln >> 4);
     t16 = t16 < g.ntiles16 ? t16 : g.ntiles16 - 1;  // (rows past the end are never stored)
@@ -559,7 +593,7 @@ __global__ __launch_bounds__(256, TT == 1 ? 3 : 2) void igemm_kernel(IgArgs g) {
 #pragma unroll
         for (int i = 0; i < 16; ++i) y[t][i] = 0.0f;
 
-    for (uint32_t it = 0; it < steps; ++it) {
+    for (uint32_t it = 0; it < (mat == kIgZero ? 0 : steps); ++it) {
         ig_barrier();  // stage `it` has landed for every wave; the other one is free
         if (it + 1 < steps) {
             issue(it + 1);
@@ -652,6 +686,7 @@ __global__ __launch_bounds__(256, TT == 1 ? 3 : 2) void igemm_kernel(IgArgs g) {
         cur = nxt;
     }
 
+    if (mat == kIgZero) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // its first stage must land before LDS is reused
     if constexpr (KS > 1) {  // the groups' partial sums, added in group order
         __syncthreads();
         float* red = (float*)smem;
@@ -673,17 +708,20 @@ __global__ __launch_bounds__(256, TT == 1 ? 3 : 2) void igemm_kernel(IgArgs g) {
     const uint32_t row = (nt * RW + rw) * 32 + ln;
     if (row >= g.rows) return;
 #pragma unroll
-    for (int t = 0; t < TT; ++t)
+    for (int t = 0; t < TT; ++t) {
+        const uint32_t tile = mt * TT + t;
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
-            const uint32_t slot = (mt * TT + t) * kIgTok + 8 * (i / 4) + 4 * kh + (i % 4);
-            if (g.slot_row) {
-                const int32_t r = g.slot_row[slot];
+            const uint32_t tok = 8 * (i / 4) + 4 * kh + (i % 4);
+            if (g.map.tile_mat) {
+                const int32_t r = g.map.row[tile * kIgTok + tok];
                 if (r >= 0) g.y[(uint64_t)r * g.ldy + row] = y[t][i];
-            } else if (slot < g.M) {
-                g.y[(uint64_t)slot * g.ldy + row] = y[t][i];
+            } else {
+                const uint32_t k = tile / g.map.tpg, j = tile % g.map.tpg * kIgTok + tok;
+                if (j < g.map.cpg) g.y[((uint64_t)k * g.map.cpg + j) * g.ldy + row] = y[t][i];
             }
         }
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -693,7 +731,7 @@ template <uint32_t T, int TT, int KS>
 static hipError_t ig_launch_one(IgArgs g, uint32_t tiles, hipStream_t s) {
     constexpr int RW = 4 / KS;
     g.NT = (g.rows + 32 * RW - 1) / (32 * RW);
-    g.MT = TT == 1 ? (g.M + kIgTok - 1) / kIgTok : tiles / TT;
+    g.MT = tiles / TT;
     const uint64_t grid = (uint64_t)g.NT * g.MT;
     if (grid == 0 || grid > 0x7fffffffull) return hipErrorInvalidValue;
     static LdsLimit lim;
@@ -702,13 +740,6 @@ static hipError_t ig_launch_one(IgArgs g, uint32_t tiles, hipStream_t s) {
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL((igemm_kernel<T, TT, KS>), dim3((unsigned)grid), dim3(256), lds, s, g);
     return hipGetLastError();
-}
-
-// Column tiles of the image of M columns: padded so that a pair of tiles per
-// workgroup (TT = 2) always lies inside it.
-static uint32_t ig_tiles(uint64_t M) {
-    const uint64_t t = (M + kIgTok - 1) / kIgTok;
-    return (uint32_t)(t > 1 ? (t + 1) & ~1ull : t);
 }
 
 // Shape of the workgroups, by the number of (32 rows x 32 columns) tiles.
@@ -722,40 +753,46 @@ static uint32_t ig_tiles(uint64_t M) {
 // against 42.1).  Q4_K unpacks in fewest steps and keeps one column tile up to
 // 4000 tiles (37 us against 45); Q8_0 and Q2_K cannot split K, and Q8_0, whose
 // work is the f32 terms, keeps one column tile throughout (124 us against 137).
+// pairs: two neighbouring column tiles may share a wave.
 template <uint32_t T>
-static hipError_t ig_launch(const IgArgs& g, uint32_t tiles, hipStream_t s) {
-    const uint64_t n = (uint64_t)((g.rows + 31) / 32) * ((g.M + kIgTok - 1) / kIgTok);
+static hipError_t ig_launch(const IgArgs& g, uint32_t tiles, bool pairs, hipStream_t s) {
+    const uint64_t live = g.map.tile_mat ? tiles : (uint64_t)tiles / g.map.tpg * ((g.map.cpg + kIgTok - 1) / kIgTok);
+    const uint64_t n = (uint64_t)((g.rows + 31) / 32) * live;
     if constexpr (T == kQ8_0) {
         return ig_launch_one<T, 1, 1>(g, tiles, s);
     } else {
         if constexpr (T != kQ2_K) {
             if (n <= 512) return ig_launch_one<T, 1, 4>(g, tiles, s);
             if (n <= 1100) return ig_launch_one<T, 1, 2>(g, tiles, s);
-            if (T != kQ4_K && n <= 3000 && tiles > 1) return ig_launch_one<T, 2, T == kQ4_K ? 1 : 2>(g, tiles, s);
+            if (T != kQ4_K && n <= 3000 && pairs) return ig_launch_one<T, 2, T == kQ4_K ? 1 : 2>(g, tiles, s);
         }
-        if (tiles == 1 || n <= (T == kQ2_K || T == kQ4_K ? 4000 : 0)) return ig_launch_one<T, 1, 1>(g, tiles, s);
+        if (!pairs || n <= (T == kQ2_K || T == kQ4_K ? 4000 : 0)) return ig_launch_one<T, 1, 1>(g, tiles, s);
         return ig_launch_one<T, 2, 1>(g, tiles, s);
     }
 }
 
 template <uint32_t T>
-static hipError_t ig_act(const float* x, const ActPlanes& pl, const int32_t* map, uint32_t M, uint32_t K, uint32_t tiles,
-                         const IgImage& im, unsigned long long* err, const uint32_t* gate, hipStream_t s) {
-    hipLaunchKernelGGL((igemm_act_kernel<T>), dim3(tiles * im.nchunk), dim3(512), 0, s, x, pl, map, M, K, im.nchunk, im.img,
-                       im.flags, err, gate);
+static hipError_t ig_act(const void* x, bool packed, const IgMap& map, uint32_t K, uint32_t tiles, const IgImage& im,
+                         unsigned long long* err, const uint32_t* gate, hipStream_t s) {
+    const dim3 grid(tiles * im.nchunk);
+    if (!packed)
+        hipLaunchKernelGGL((igemm_act_kernel<T, false>), grid, dim3(512), 0, s, x, map, K, im.nchunk, im.img, im.flags, err,
+                           gate);
+    else if constexpr (!ig_mins(T))
+        hipLaunchKernelGGL((igemm_act_kernel<T, true>), grid, dim3(512), 0, s, x, map, K, im.nchunk, im.img, im.flags, err,
+                           gate);
+    else
+        return hipErrorInvalidValue;
     return hipGetLastError();
 }
 
-size_t igemm_bytes(uint32_t t, uint64_t M, uint64_t cols) { return igemm_image_bytes(t, ig_tiles(M), cols); }
-
-hipError_t launch_igemm(uint32_t t, const uint8_t* w, uint64_t rows, uint64_t cols, const float* x, uint64_t M, float* y,
-                        uint64_t ldy, void* scratch, unsigned long long* err_word, hipStream_t s) {
-    if (rows == 0 || cols == 0 || cols % (t == kQ8_0 ? 32 : 256) || M == 0 || rows > 0x7fffffffull ||
-        cols > (1u << 30) || M > (1u << 24))
+// The image of the columns, then the product.
+static hipError_t ig_run(uint32_t t, const uint8_t* w, uint64_t rows, uint64_t cols, uint64_t mat_bytes, const void* x,
+                         bool packed, const IgMap& map, uint32_t tiles, bool pairs, const IgImage& im, float* y, uint64_t ldy,
+                         const uint32_t* gate, unsigned long long* err, hipStream_t s) {
+    if (rows == 0 || cols == 0 || cols % (t == kQ8_0 ? 32 : 256) || tiles == 0 || rows > 0x7fffffffull ||
+        cols > (1u << 30) || tiles > (1u << 20) || (uint64_t)tiles * im.nchunk > 0x7fffffffull)
         return hipErrorInvalidValue;
-    const uint32_t tiles = ig_tiles(M);
-    const IgImage im = ig_carve(scratch, t, tiles, cols);
-    if ((uint64_t)tiles * im.nchunk > 0x7fffffffull) return hipErrorInvalidValue;
     IgArgs g{};
     g.w = w;
     g.rows = (uint32_t)rows;
@@ -765,15 +802,16 @@ hipError_t launch_igemm(uint32_t t, const uint8_t* w, uint64_t rows, uint64_t co
     g.img = im.img;
     g.flags = im.flags;
     g.nflags = tiles * im.nchunk;
-    g.M = (uint32_t)M;
     g.y = y;
     g.ldy = ldy;
-    const ActPlanes none{};
+    g.gate = gate;
+    g.map = map;
+    g.mat_bytes = mat_bytes;
     hipError_t e;
-#define RLQ_IG(TYPE)                                                                                       \
-    case TYPE:                                                                                             \
-        e = ig_act<TYPE>(x, none, nullptr, g.M, (uint32_t)cols, tiles, im, err_word, nullptr, s);          \
-        return e != hipSuccess ? e : ig_launch<TYPE>(g, tiles, s);
+#define RLQ_IG(TYPE)                                                                        \
+    case TYPE:                                                                              \
+        e = ig_act<TYPE>(x, packed, map, (uint32_t)cols, tiles, im, err, gate, s);          \
+        return e != hipSuccess ? e : ig_launch<TYPE>(g, tiles, pairs, s);
     switch (t) {
         RLQ_IG(kQ8_0)
         RLQ_IG(kQ2_K)
@@ -784,6 +822,132 @@ hipError_t launch_igemm(uint32_t t, const uint8_t* w, uint64_t rows, uint64_t co
         default: return hipErrorInvalidValue;
     }
 #undef RLQ_IG
+}
+
+// Column tiles of one group: from three on an even number, so that pairs of them
+// can share a wave.
+static uint64_t ig_group_tiles(uint64_t cpg) {
+    const uint64_t t = (cpg + kIgTok - 1) / kIgTok;
+    return t > 2 ? (t + 1) & ~1ull : t;
+}
+
+size_t igemm_bytes(uint32_t t, uint64_t groups, uint64_t cpg, uint64_t cols) {
+    return igemm_image_bytes(t, groups * ig_group_tiles(cpg), cols);
+}
+
+hipError_t launch_igemm(uint32_t t, const uint8_t* w, uint64_t rows, uint64_t cols, const void* x, bool packed,
+                        const IgStack& st, float* y, uint64_t ldy, void* scratch, unsigned long long* err_word,
+                        hipStream_t s) {
+    const uint64_t tpg = ig_group_tiles(st.cpg), tiles = tpg * st.groups;
+    if (st.cpg == 0 || st.groups == 0 || tiles > (1u << 20)) return hipErrorInvalidValue;
+    IgMap map{};
+    map.cpg = (uint32_t)st.cpg, map.tpg = (uint32_t)tpg, map.wn2 = (uint32_t)st.wn2, map.r3 = (uint32_t)st.r3;
+    return ig_run(t, w, rows, cols, st.mat_bytes, x, packed, map, (uint32_t)tiles, tpg % 2 == 0,
+                  ig_carve(scratch, t, tiles, cols), y, ldy, nullptr, err_word, s);
+}
+
+// ---------------------------------------------------------------------------
+// MUL_MAT_ID
+// ---------------------------------------------------------------------------
+
+// Checks the ids (the first one outside [-1, mats) refuses the call) and deals
+// the products to image columns, matrix after matrix, each from a whole group
+// of `unit` tiles on (one workgroup); then the products without a matrix (id
+// -1) and the columns that no product uses, which are quantized for their
+// errors only.  Where inside its run a product lands depends on the order of
+// the LDS atomics; its result does not.  One workgroup: the counts stay in LDS,
+// and a launch of its own costs less than a grid-wide sum.
+__global__ __launch_bounds__(1024) void igemm_route_kernel(IgRoute r, uint32_t tiles, uint32_t unit,
+                                                           uint32_t* __restrict__ tile_mat, int32_t* __restrict__ src,
+                                                           int32_t* __restrict__ row, uint32_t* __restrict__ gate,
+                                                           unsigned long long* err_word) {
+    __shared__ uint32_t count[kIgMaxMats + 1], first[kIgMaxMats + 2], used[kIgMaxColumns / 32];
+    __shared__ unsigned long long bad;
+    const uint32_t tid = threadIdx.x, group = unit * kIgTok;
+    if (tid == 0) bad = ~0ull;
+    for (uint32_t i = tid; i <= r.mats; i += 1024) count[i] = 0;
+    for (uint32_t i = tid; i < (r.columns + 31) / 32; i += 1024) used[i] = 0;
+    for (uint32_t i = tid; i < tiles * kIgTok; i += 1024) src[i] = row[i] = -1;
+    __syncthreads();
+    auto column_of = [&](uint32_t i) { return i / r.slots * r.ncols + i % r.slots % r.ncols; };
+    for (uint32_t i = tid; i < r.products; i += 1024) {
+        const int32_t id = r.ids[i];
+        if (id < -1 || id >= (int32_t)r.mats) {
+            atomicMin(&bad, (unsigned long long)i);
+        } else {
+            atomicAdd(&count[id < 0 ? r.mats : (uint32_t)id], 1u);
+            if (id >= 0) atomicOr(&used[column_of(i) / 32], 1u << (column_of(i) % 32));
+        }
+    }
+    __syncthreads();
+    if (tid == 0) {
+        *gate = bad != ~0ull;
+        if (bad != ~0ull) report_error(err_word, bounds_key(bad));
+    }
+    if (bad != ~0ull) return;
+    auto is_used = [&](uint32_t c) { return (used[c / 32] >> (c % 32)) & 1u; };
+    for (uint32_t c = tid; c < r.columns; c += 1024)
+        if (!is_used(c)) atomicAdd(&count[r.mats], 1u);
+    __syncthreads();
+    if (tid == 0) {
+        uint32_t t = 0;
+        for (uint32_t m = 0; m <= r.mats; ++m) {
+            first[m] = t;
+            t += (count[m] + group - 1) / group * unit;
+        }
+        first[r.mats + 1] = t;
+    }
+    __syncthreads();
+    for (uint32_t t = tid; t < tiles; t += 1024) {
+        uint32_t m = 0;
+        while (m <= r.mats && first[m + 1] <= t) ++m;
+        tile_mat[t] = m > r.mats ? kIgNone : (m == r.mats ? kIgZero : m);
+    }
+    __syncthreads();
+    for (uint32_t i = tid; i <= r.mats; i += 1024) count[i] = 0;
+    __syncthreads();
+    for (uint32_t i = tid; i < r.products; i += 1024) {
+        const int32_t id = r.ids[i];
+        const uint32_t m = id < 0 ? r.mats : (uint32_t)id;
+        const uint32_t at = first[m] * kIgTok + atomicAdd(&count[m], 1u);
+        row[at] = (int32_t)i;
+        if (id >= 0) src[at] = (int32_t)column_of(i);
+    }
+    for (uint32_t c = tid; c < r.columns; c += 1024)
+        if (!is_used(c)) src[first[r.mats] * kIgTok + atomicAdd(&count[r.mats], 1u)] = (int32_t)c;
+}
+
+// From 128 products a matrix on, two column tiles of one matrix share a wave.
+static uint32_t ig_unit(const IgRoute& r) { return r.products / r.mats >= 128 ? 2 : 1; }
+// Upper bound of the tiles: every run in use may leave its last group short.
+static uint64_t ig_route_tiles(const IgRoute& r) {
+    const uint64_t u = ig_unit(r), n = (uint64_t)r.products + r.columns;
+    return (n / (u * kIgTok) + (r.products < r.mats ? r.products : r.mats) + 1) * u;
+}
+
+size_t igemm_ids_bytes(uint32_t t, uint64_t cols, const IgRoute& r) {
+    const uint64_t tiles = ig_route_tiles(r);
+    return igemm_image_bytes(t, tiles, cols) + 4 + tiles * (4 + kIgTok * 8);
+}
+
+hipError_t launch_igemm_ids(uint32_t t, const uint8_t* w, uint64_t rows, uint64_t cols, uint64_t mat_bytes, const void* x,
+                            bool packed, const IgRoute& r, float* y, uint64_t ldy, void* scratch,
+                            unsigned long long* err_word, hipStream_t s) {
+    const uint64_t tiles = ig_route_tiles(r);
+    if (r.products == 0 || r.mats == 0 || r.mats > kIgMaxMats || r.columns > kIgMaxColumns || tiles > (1u << 20))
+        return hipErrorInvalidValue;
+    const IgImage im = ig_carve(scratch, t, tiles, cols);
+    uint32_t* gate = im.flags + tiles * im.nchunk;
+    uint32_t* tile_mat = gate + 1;
+    int32_t *src = (int32_t*)(tile_mat + tiles), *row = src + tiles * kIgTok;
+    const uint32_t unit = ig_unit(r);
+    hipLaunchKernelGGL(igemm_route_kernel, dim3(1), dim3(1024), 0, s, r, (uint32_t)tiles, unit, tile_mat, src, row, gate,
+                       err_word);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    IgMap map{};
+    map.tile_mat = tile_mat, map.src = src, map.row = row;
+    return ig_run(t, w, rows, cols, mat_bytes, x, packed, map, (uint32_t)tiles, unit == 2, im, y, ldy, gate, err_word, s);
 }
 
 }  // namespace rlq

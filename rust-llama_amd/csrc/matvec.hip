@@ -3425,38 +3425,46 @@ hipError_t launch_matvec_ex(uint32_t wtype, const uint8_t* w, uint64_t rows, uin
 // otherwise the outputs of the pairs with id -1 are zeroed (the reference's
 // `zeros` output, cpu_index.rs:204) and the gate is 0.
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void mm_prepare_kernel(const int32_t* __restrict__ ids, uint64_t pairs,
-                                                         int32_t experts, const uint8_t* __restrict__ bad,
-                                                         uint64_t nbad, float* __restrict__ y, uint64_t rows,
-                                                         uint32_t* gate, unsigned long long* err_word) {
+__global__ __launch_bounds__(1024) void mm_prepare_kernel(const int32_t* __restrict__ ids, uint64_t pairs,
+                                                          int32_t experts, const uint8_t* __restrict__ bad,
+                                                          uint64_t nbad, float* __restrict__ y, uint64_t rows,
+                                                          uint32_t* gate, unsigned long long* err_word) {
     __shared__ unsigned long long first_s;
-    __shared__ int flag_s;
-    if (threadIdx.x == 0) first_s = ~0ull, flag_s = 0;
+    __shared__ int flag_s, none_s;
+    if (threadIdx.x == 0) first_s = ~0ull, flag_s = none_s = 0;
     __syncthreads();
     unsigned long long first = ~0ull;
-    for (uint64_t i = threadIdx.x; i < pairs; i += 256) {
+    int any_bad = 0, any_none = 0;
+    for (uint64_t i = threadIdx.x; i < pairs; i += 1024) {
         const int32_t id = ids[i];
         if ((id < -1 || id >= experts) && i < first) first = i;
+        any_none |= id == -1;
     }
-    int any_bad = 0;
-    for (uint64_t i = threadIdx.x; i < nbad; i += 256) any_bad |= bad[i];
+    // the flag bytes, sixteen at a time (planes.bad is 16-byte aligned): 1024
+    // columns of 16 blocks took 64 dependent loads a thread one by one
+    for (uint64_t i = threadIdx.x; i < nbad / 16; i += 1024) {
+        const uint4 v = ((const uint4*)bad)[i];
+        any_bad |= (int)((v.x | v.y | v.z | v.w) != 0);
+    }
+    for (uint64_t i = nbad / 16 * 16 + threadIdx.x; i < nbad; i += 1024) any_bad |= bad[i];
     if (first != ~0ull) atomicMin(&first_s, first);
     if (any_bad) atomicOr(&flag_s, 1);
+    if (any_none) atomicOr(&none_s, 1);
     __syncthreads();
     const bool refused = first_s != ~0ull || flag_s != 0;
     if (threadIdx.x == 0) {
         *gate = refused ? 1u : 0u;
         if (first_s != ~0ull) report_error(err_word, bounds_key(first_s));
     }
-    if (refused || !ids) return;
+    if (refused || !none_s) return;
     for (uint64_t p = 0; p < pairs; ++p)
         if (ids[p] == -1)
-            for (uint64_t r = threadIdx.x; r < rows; r += 256) y[p * rows + r] = 0.0f;
+            for (uint64_t r = threadIdx.x; r < rows; r += 1024) y[p * rows + r] = 0.0f;
 }
 
 hipError_t launch_mm_prepare(const int32_t* ids, uint64_t pairs, uint32_t experts, const uint8_t* bad, uint64_t nbad,
                              float* y, uint64_t rows, uint32_t* gate, unsigned long long* err_word, hipStream_t s) {
-    hipLaunchKernelGGL(mm_prepare_kernel, dim3(1), dim3(256), 0, s, ids, ids ? pairs : 0, (int32_t)experts, bad, nbad,
+    hipLaunchKernelGGL(mm_prepare_kernel, dim3(1), dim3(1024), 0, s, ids, ids ? pairs : 0, (int32_t)experts, bad, nbad,
                        y, rows, gate, err_word);
     return hipGetLastError();
 }

@@ -142,12 +142,32 @@ hipError_t launch_gemm_q4k(const uint8_t* w, uint64_t rows, uint64_t cols, const
                            int32_t* dbg_imin, hipStream_t s);
 
 // ---- igemm.hip ----
-// The int8 GEMM of every weight format: y[m*ldy + r] = dot(row r, column m) for
-// m < M, x [M][cols] f32 quantized into `scratch` (igemm_bytes) first.  A data
-// error in any column goes to `err_word` and suppresses every output.
-size_t igemm_bytes(uint32_t t, uint64_t M, uint64_t cols);
-hipError_t launch_igemm(uint32_t t, const uint8_t* w, uint64_t rows, uint64_t cols, const float* x, uint64_t M, float* y,
-                        uint64_t ldy, void* scratch, unsigned long long* err_word, hipStream_t s);
+// The int8 GEMM of every weight format.  The columns, `groups` of cpg
+// contiguous ones, are f32 rows of x or (packed; Q3_K, Q6_K and Q8_0 weights)
+// rows of activation blocks taken as given; group k takes matrix
+// k / wn2 / r3 * wn2 + k % wn2 of a stack, mat_bytes apart, and
+// y[c*ldy + r] = dot(row r of its matrix, column c).  `scratch`: igemm_bytes.  A
+// data error in any column goes to `err_word` and suppresses every output.
+struct IgStack {
+    uint64_t groups, cpg, wn2, r3, mat_bytes;
+};
+size_t igemm_bytes(uint32_t t, uint64_t groups, uint64_t cpg, uint64_t cols);
+hipError_t launch_igemm(uint32_t t, const uint8_t* w, uint64_t rows, uint64_t cols, const void* x, bool packed,
+                        const IgStack& st, float* y, uint64_t ldy, void* scratch, unsigned long long* err_word,
+                        hipStream_t s);
+// MUL_MAT_ID: product i takes matrix ids[i] of `mats` (-1: its row is 0) and
+// column i / slots * ncols + i % slots % ncols, and writes y + i * ldy.  An id
+// out of range is reported and suppresses every output, as a data error in
+// any of the `columns` columns does.
+struct IgRoute {
+    const int32_t* ids;
+    uint32_t products, mats, columns, slots, ncols;
+};
+constexpr uint32_t kIgMaxMats = 1024, kIgMaxColumns = 65536;
+size_t igemm_ids_bytes(uint32_t t, uint64_t cols, const IgRoute& r);
+hipError_t launch_igemm_ids(uint32_t t, const uint8_t* w, uint64_t rows, uint64_t cols, uint64_t mat_bytes, const void* x,
+                            bool packed, const IgRoute& r, float* y, uint64_t ldy, void* scratch,
+                            unsigned long long* err_word, hipStream_t s);
 
 // ---- llama.hip ----
 // The dense Llama decode step (crates/model-runtime/src/llama.rs:222-392)

@@ -67,3 +67,85 @@ def test_many_columns(t, rows, cols, batch):
         W.close()
     finally:
         ctx.close()
+
+
+# ---- several matrices -------------------------------------------------------------
+
+def check(t, y, want):
+    """y, want [products, rows]."""
+    for i in range(len(want)):
+        assert rel_l2(y[i], want[i]) <= REL_L2, i
+    if t in EXACT_ALWAYS:
+        assert np.array_equal(y.view(np.uint32), want.view(np.uint32))
+
+
+def packed_rows(t, x):
+    return np.concatenate([O.quantize(O.matvec_activation_dtype(int(t)), r) for r in x])
+
+
+@pytest.mark.parametrize("packed", [False, True])
+@pytest.mark.parametrize("t", TYPES, ids=lambda t: DT(t).name)
+def test_mul_mat_id_many_pairs(t, packed):
+    """Enough pairs for the grouped products: experts without a token, tokens
+    and slots without an expert, one expert with most tokens, and refusals by an
+    id and by a column that no product uses."""
+    rows, cols, experts, tokens, slots = 520, 2048, 6, 130, 2
+    say("igemm ids", DT(t).name, "packed" if packed else "f32")
+    w = _weights(t, experts * rows, cols, 7)
+    rng = np.random.default_rng(8)
+    ids = rng.integers(0, experts - 1, (tokens, slots)).astype(np.int32)  # the last expert unused
+    ids[3:80, 0] = 2
+    ids[5] = -1
+    ids[9, 1] = -1
+    x = rng.standard_normal((tokens, cols)).astype(np.float32)
+    a = packed_rows(t, x) if packed else x
+    xd = torch.from_numpy(a).cuda().reshape(tokens, 1, -1)
+    at = O.matvec_activation_dtype(int(t)) if packed else O.F32
+    ctx = rlq.Context(0)
+    try:
+        W = rlq.Weights(ctx, t, w, rows, cols, experts)
+        y = ctx.mul_mat_id(W, xd, torch.from_numpy(ids).cuda(), x_dtype=at)
+        ctx.sync()
+        want = O.mul_mat_id(int(t), w, rows, cols, experts, at, a, 1, tokens, ids)
+        check(t, y.cpu().numpy().reshape(-1, rows), np.asarray(want).reshape(-1, rows))
+        z = torch.full((tokens, slots, rows), 7.0, device="cuda")
+        bad = ids.copy()
+        bad[100, 1], bad[101, 0] = experts, -2
+        ctx.mul_mat_id(W, xd, torch.from_numpy(bad).cuda(), x_dtype=at, y=z)
+        with pytest.raises(rlq.QuantError) as e:
+            ctx.sync()
+        assert (e.value.name, e.value.a) == ("Bounds", 201) and bool((z == 7.0).all())
+        if not packed:
+            xd[5, 0, 77] = float("nan")
+            ctx.mul_mat_id(W, xd, torch.from_numpy(ids).cuda(), y=z)
+            with pytest.raises(rlq.QuantError) as e:
+                ctx.sync()
+            assert (e.value.name, e.value.index, e.value.b) == ("NonFiniteInput", 77, 5) and bool((z == 7.0).all())
+        W.close()
+    finally:
+        ctx.close()
+
+
+@pytest.mark.parametrize("packed", [False, True])
+@pytest.mark.parametrize("ncols", [2, 17, 33])
+@pytest.mark.parametrize("t", TYPES, ids=lambda t: DT(t).name)
+def test_mul_mat_broadcast_many_columns(t, ncols, packed):
+    """Both broadcast directions: 2 matrices along n2 for 4 slices, along n3 for
+    2, so that a matrix serves several runs of columns."""
+    rows, cols, wn2, wn3, n2, n3 = 47, 768, 2, 1, 4, 2
+    say("igemm broadcast", DT(t).name, ncols, "packed" if packed else "f32")
+    w = _weights(t, wn2 * wn3 * rows, cols, 17)
+    x = np.random.default_rng(18).standard_normal((n3 * n2 * ncols, cols)).astype(np.float32)
+    a = packed_rows(t, x) if packed else x
+    at = O.matvec_activation_dtype(int(t)) if packed else O.F32
+    ctx = rlq.Context(0)
+    try:
+        W = rlq.Weights(ctx, t, w, rows, cols, wn2, wn3)
+        xd = torch.from_numpy(a).cuda().reshape(n3, n2, ncols, -1)
+        y = ctx.mul_mat(W, xd, x_dtype=at)
+        ctx.sync()
+        want = O.mul_mat(int(t), w, rows, cols, wn2, wn3, at, a, ncols, n2, n3)
+        check(t, y.cpu().numpy().reshape(-1, rows), np.asarray(want).reshape(-1, rows))
+        W.close()
+    finally:
+        ctx.close()
