@@ -191,9 +191,10 @@ void rlq_weights_stack(const rlq_weights *w, uint64_t *n2, uint64_t *n3);
  * x[b*cols ..] is quantized to the weights' activation type on the GPU, then
  * y[b*rows + r] = dot_packed(weights row r, activation b).  x and y are
  * device pointers (x 16-byte aligned).  Up to 8 columns share one pass over
- * the weights; more run a GEMM over an image of the quantized columns in the
- * context's scratch (while `stream` is being captured, types other than Q4_K
- * run passes of 8 columns, which need none).  A call takes at most 8388606 columns (the error keys carry
+ * the weights; more (and, of some types and shapes, two to eight) run a GEMM
+ * over an image of the quantized columns in the context's scratch (while
+ * `stream` is being captured, types other than Q4_K run passes of 8 columns,
+ * which need none).  A call takes at most 8388606 columns (the error keys carry
  * the column): more return RLQ_UNIMPLEMENTED (a = batch, b = the limit), as
  * do rlq_matmul_argmax, rlq_matmul_noalloc and rlq_quantize_device. */
 int32_t rlq_matmul(rlq_context *ctx, const rlq_weights *w, const float *x, uint64_t batch, float *y,
@@ -220,8 +221,7 @@ int32_t rlq_matmul_argmax(rlq_context *ctx, const rlq_weights *w, const float *x
  * memory (code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc).  rlq_matmul (argmax null) or rlq_matmul_argmax (argmax
  * non-null) on the same kernels, with the same results, that allocates and
- * frees nothing: the argmax keys and the GEMMs' activation images (batches
- * above 8) live in a static 32 MiB device array that each GPU holds until the
+ * frees nothing: the argmax keys and the GEMMs' activation images live in a static 32 MiB device array that each GPU holds until the
  * process ends.  A call with Q4_K weights whose workspace exceeds it returns
  * RLQ_SCRATCH_LIMIT (a = bytes needed, b = 33554432); for 4096 columns that is
  * a batch of about 3,700.  With other weights such a call runs passes of 8
@@ -276,8 +276,8 @@ int32_t rlq_sync(rlq_context *ctx, void *stream, rlq_error *err);
 
 /* Exact integer part of every (row, block) dot of the weights against
  * activation column 0 of x (device f32, `batch` columns of cols values, 1 <=
- * batch <= 8), computed inside the kernel rlq_matmul runs for that batch size
- * (the columns are quantized on the GPU as rlq_matmul does):
+ * batch <= 8), computed inside the decode kernel of that batch size (the
+ * columns are quantized on the GPU as rlq_matmul does):
  * isum[r*nb + k] and imin[r*nb + k] for block k are the integers of
  * crates/quant/src/matvec_extra.rs:174-283 (the eight lanes added; imin is
  * the mins sum of Q2_K, Q4_K and Q5_K, 0 otherwise) and matvec.rs:124-127.

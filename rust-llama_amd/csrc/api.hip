@@ -485,6 +485,40 @@ hipError_t decode_launch(rlq_context* ctx, const rlq_weights* w, const float* x,
                             isum, imin, ex, s);
 }
 
+// How a product of `batch` f32 columns runs: the decode kernels (passes of up to
+// 8 columns), the 128-column Q4_K GEMM, or the int8 GEMM of every format.
+enum class Route { kDecode, kGemm, kIgemm };
+
+// The Q4_K GEMM's workgroups take 128 columns x 256 rows and one CU each: from
+// three quarters of the CUs on it is the faster one (14336x4096, 512 columns =
+// 224 workgroups: 73 us against 95), below that the int8 GEMM's smaller tiles
+// are (4096x4096, 512 columns = 64 workgroups: 36 us).
+//
+// Up to 8 columns the decode kernels read the weights once, with no launch
+// before them.  The int8 GEMM's two launches are faster where those kernels
+// take several passes or lose their K split (us, decode against GEMM):
+//  - Q6_K two columns (two passes: 4096x14336 30.5 / 22.7, 1024x1024 10.2 / 7.9), and
+//    three or more of 2048 or more values (4096x4096 17.4 / 12.0, 14336x4096 20.8 /
+//    18.5; 1024x1024 7.3 / 7.9);
+//  - Q2_K and Q3_K from five columns (a second group of columns) of 2048 or more
+//    values (4096x4096 17.4 / 9.1 and 17.7 / 10.4; 1024x1024 7.2 / 7.4 and 7.5 / 7.8),
+//    Q3_K below the balanced deal's 6144 rows (14336x4096 14.1 / 15.8);
+//  - Q8_0 whose parked terms no longer fit LDS (4096x14336: three columns 29.6 /
+//    40, five 80 / 40; 4096x4096, eight columns 13.5 / 16.6).
+// Not with an argmax, which the decode kernels finish in the same launch, and
+// not for the output head's row counts, where they are near the memory rate.
+Route matmul_route(uint32_t dtype, uint64_t rows, uint64_t cols, uint64_t batch, bool argmax) {
+    if (batch > kDecodeMaxBatch)
+        return dtype == kQ4_K && (rows + 255) / 256 * ((batch + 127) / 128) >= 192 ? Route::kGemm : Route::kIgemm;
+    if (batch < 2 || argmax || rows > 32768) return Route::kDecode;
+    const bool igemm = dtype == kQ6_K   ? batch == 2 || cols >= 2048
+                       : dtype == kQ2_K ? batch >= 5 && cols >= 2048
+                       : dtype == kQ3_K ? batch >= 5 && cols >= 2048 && rows < 6144
+                       : dtype == kQ8_0 ? batch * (cols / 32) > 1600
+                                        : false;
+    return igemm ? Route::kIgemm : Route::kDecode;
+}
+
 // Whether several matrices' products may run on the int8 GEMM.  Packed Q8_K
 // columns bring their own 16-value sums, which the GEMM takes as f16 and so
 // only from its own quantizer: formats with mins keep the decode kernels then.
@@ -531,8 +565,9 @@ int32_t rlq_mul_mat(rlq_context* ctx, const rlq_weights* w, uint32_t x_dtype, co
     }
     // the columns of one matrix are contiguous over the r2 slices it serves
     const IgStack st{n3 * w->n2, n2 / w->n2 * ncols, w->n2, n3 / w->n3, w->mat_bytes};
-    // two to eight f32 columns of one matrix: the one launch of rlq_matmul
-    if (columns <= kDecodeMaxBatch && st.groups == 1 && x_dtype == 0 && ncols > 1) {
+    const bool plain = columns <= kDecodeMaxBatch && st.groups == 1 && x_dtype == 0 && ncols > 1;
+    // two to eight f32 columns of one matrix: the launch of rlq_matmul
+    if (plain && matmul_route(w->dtype, w->rows, w->cols, columns, false) == Route::kDecode) {
         HIP_TRY(decode_launch(ctx, w, (const float*)x, columns, y, nullptr, nullptr, nullptr, MvExtra{}, s));
         return ok(err);
     }
@@ -540,10 +575,8 @@ int32_t rlq_mul_mat(rlq_context* ctx, const rlq_weights* w, uint32_t x_dtype, co
     // quantizer and the gate: always fewer (Q4_K 4096x4096, 4 matrices of 2
     // slices of 4 columns: 25 us against 66; one matrix, 100 columns: 25 against
     // 103).  Single columns keep the decode kernels, whose sums are in the
-    // reference's order; Q8_0 and Q2_K, whose sums are so in both, take the GEMM
-    // for more than 32 columns a matrix (matmul_route).
-    const bool ordered = w->dtype == kQ8_0 || w->dtype == kQ2_K;
-    if (mm_igemm_takes(w->dtype, x_dtype, x) && (ordered ? st.cpg > 32 : ncols > 1)) {
+    // reference's order.
+    if (mm_igemm_takes(w->dtype, x_dtype, x) && ncols > 1) {
         HIP_TRY(ensure(ctx, ctx->planes, igemm_bytes(w->dtype, st.groups, st.cpg, w->cols)));
         HIP_TRY(launch_igemm(w->dtype, w->dev, w->rows, w->cols, x, x_dtype != 0, st, y, w->rows, ctx->planes.p,
                              ctx->err_words, s));
@@ -639,22 +672,6 @@ int32_t rlq_mul_mat_id(rlq_context* ctx, const rlq_weights* w, uint32_t x_dtype,
 // model runtime's field 0x7fffff (rlq_device.hpp).
 constexpr uint64_t kMaxKeyColumns = (1ull << 23) - 2;
 
-// How a product of `batch` f32 columns runs: the decode kernels (passes of up to
-// 8 columns), the 128-column Q4_K GEMM, or the int8 GEMM of every format.
-enum class Route { kDecode, kGemm, kIgemm };
-
-// The Q4_K GEMM's workgroups take 128 columns x 256 rows and one CU each: from
-// three quarters of the CUs on it is the faster one (14336x4096, 512 columns =
-// 224 workgroups: 73 us against 95), below that the int8 GEMM's smaller tiles
-// are (4096x4096, 512 columns = 64 workgroups: 37 us).  Q8_0 and Q2_K cannot
-// split K (their sums have one order), so few columns of a long row are faster
-// in decode passes, which do (4096x14336 Q8_0, 16 columns: 60 us against 137).
-static Route matmul_route(uint32_t dtype, uint64_t rows, uint64_t batch) {
-    if (batch <= kDecodeMaxBatch) return Route::kDecode;
-    if (dtype == kQ4_K) return (rows + 255) / 256 * ((batch + 127) / 128) >= 192 ? Route::kGemm : Route::kIgemm;
-    return (dtype == kQ8_0 || dtype == kQ2_K) && batch <= 32 ? Route::kDecode : Route::kIgemm;
-}
-
 static size_t route_bytes(Route r, uint32_t dtype, uint64_t batch, uint64_t cols) {
     return r == Route::kGemm ? gemm_planes_bytes(batch, cols) : r == Route::kIgemm ? igemm_bytes(dtype, 1, batch, cols) : 0;
 }
@@ -696,7 +713,7 @@ static int32_t matmul_impl(rlq_context* ctx, const rlq_weights* w, const float* 
     if (batch > kMaxKeyColumns) return fail(err, RLQ_UNIMPLEMENTED, w->dtype, batch, kMaxKeyColumns);
     DeviceGuard g(ctx->device);
     const hipStream_t s = pick(ctx, stream);
-    Route route = matmul_route(w->dtype, w->rows, batch);
+    Route route = matmul_route(w->dtype, w->rows, w->cols, batch, argmax != nullptr);
     // A graph keeps the addresses it was captured with, and the context's
     // scratch may be replaced by a later, larger call: what needs no scratch
     // (every type but Q4_K) is recorded as decode passes.
@@ -753,7 +770,7 @@ int32_t rlq_matmul_noalloc(rlq_context* ctx, const rlq_weights* w, const float* 
     if (((uintptr_t)x & 15) || ((uintptr_t)y & 3)) return fail(err, RLQ_INVALID_ARGUMENT, w->dtype);
     if (batch == 0) return ok(err);
     if (batch > kMaxKeyColumns) return fail(err, RLQ_UNIMPLEMENTED, w->dtype, batch, kMaxKeyColumns);
-    Route route = matmul_route(w->dtype, w->rows, batch);
+    Route route = matmul_route(w->dtype, w->rows, w->cols, batch, argmax != nullptr);
     const uint64_t state_bytes = argmax ? kArgmaxStateBytes : 0;
     uint64_t keys_bytes = argmax && route != Route::kDecode ? (batch * 8 + 255) / 256 * 256 : 0;
     // the limit of Q4_K stays that of the larger image, whichever GEMM runs

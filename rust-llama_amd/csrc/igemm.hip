@@ -79,14 +79,16 @@ static IgImage ig_carve(void* base, uint32_t t, uint64_t tiles, uint64_t cols) {
 
 // Which matrix and column an image column stands for.  Products of one or more
 // matrices whose columns are contiguous: `groups` of cpg columns, tpg tiles
-// each; group k uses matrix k / wn2 / r3 * wn2 + k % wn2 (MUL_MAT broadcast).
-// Or dealt by igemm_route_kernel (tile_mat non-null): the matrix of each tile,
-// kIgZero for products without one (their rows are 0) and columns no product
-// uses, kIgNone for unused tiles; per image column its source and its output
+// each; group k uses matrix k / wn2 / r3 * wn2 + k % wn2 (MUL_MAT broadcast; one:
+// a single group, which needs no divisions).
+// Or dealt by igemm_route_kernel (tile_mat non-null): the matrix of each tile
+// (low half; high half: its live columns, which come first), kIgZero for
+// products without one (their rows are 0) and columns no product uses, kIgNone
+// for unused tiles; per image column its source and its output
 // row (-1: none).
 constexpr uint32_t kIgNone = ~0u, kIgZero = ~0u - 1;
 struct IgMap {
-    uint32_t cpg, tpg, wn2, r3;
+    uint32_t cpg, tpg, wn2, r3, one;
     const uint32_t* tile_mat;
     const int32_t *src, *row;
 };
@@ -110,7 +112,7 @@ __global__ __launch_bounds__(512) void igemm_act_kernel(const void* __restrict__
         }
         m = map.src[tile * kIgTok + tok];
     } else {
-        const uint32_t g = tile / map.tpg, j = tile % map.tpg * kIgTok + tok;
+        const uint32_t g = map.one ? 0 : tile / map.tpg, j = (tile - g * map.tpg) * kIgTok + tok;
         if (j < map.cpg) m = (int64_t)g * map.cpg + j;
     }
     const uint32_t e0 = c * 256 + r16 * 16;
@@ -220,8 +222,9 @@ __device__ __forceinline__ f16x2 ig_byte_half2(uint32_t w, uint32_t sel) {
            (f16x2){(_Float16)1024.0f, (_Float16)1024.0f};
 }
 
-// One format: Raw holds a lane's loaded bytes of one (16-row tile, chunk) pair;
-// Pre what a chunk's k-steps share; ops<S> the weight operand of k-step S.
+// One format: Raw holds a lane's loaded bytes of one (16-row tile, chunk) pair:
+// head loads the scales, refill<S> the pieces that no k-step after S uses; Pre is
+// what a chunk's k-steps share; ops<S> makes the weight operand of k-step S.
 // Lane (ln, kh) of a wave works on row ln % 16 = n of layout tile ln / 16 and k
 // half kh.
 template <uint32_t T>
@@ -238,11 +241,13 @@ struct Ig<kQ2_K> {
     struct Pre {
         uint32_t c[4];
     };
-    __device__ static void load(Raw& r, const uint8_t* p, uint32_t n, uint32_t kh) {
-#pragma unroll
-        for (uint32_t g = 0; g < 2; ++g) r.q[g] = ig_ld16(p + (16 * (2 * g + kh) + n) * 16);
+    __device__ static void head(Raw& r, const uint8_t* p, uint32_t n) {
         r.sc = ig_ld16(p + 1024 + n * 16);
         r.dd = *(const uint32_t*)(p + 1280 + n * 4);
+    }
+    template <int S>
+    __device__ static void refill(Raw& r, const uint8_t* p, uint32_t n, uint32_t kh) {
+        if (S % 4 == 3) r.q[S / 4] = ig_ld16(p + (16 * (2 * (S / 4) + kh) + n) * 16);
     }
     __device__ static Pre pre(const Raw& r, uint32_t kh) {
         Pre o;
@@ -282,10 +287,12 @@ struct Ig<kQ3_K> {
     struct Pre {
         uint32_t c[4];
     };
-    __device__ static void load(Raw& r, const uint8_t* p, uint32_t n, uint32_t kh) {
-#pragma unroll
-        for (uint32_t g = 0; g < 2; ++g) r.q[g] = ig_ld16(p + (16 * (2 * g + kh) + n) * 16);
-        r.hm = ig_ld16(p + 1024 + n * 32 + 16 * kh);
+    template <int S>
+    __device__ static void refill(Raw& r, const uint8_t* p, uint32_t n, uint32_t kh) {
+        if (S % 4 == 3) r.q[S / 4] = ig_ld16(p + (16 * (2 * (S / 4) + kh) + n) * 16);
+        if (S == 7) r.hm = ig_ld16(p + 1024 + n * 32 + 16 * kh);
+    }
+    __device__ static void head(Raw& r, const uint8_t* p, uint32_t n) {
         const uint32_t* s = (const uint32_t*)(p + 1536 + n * 12);
         r.s0 = s[0], r.s1 = s[1], r.s2 = s[2];
         r.d = *(const uint16_t*)(p + 1728 + n * 2);
@@ -352,10 +359,10 @@ struct Ig<kQ4_K> {
     struct Pre {
         uint32_t hi[2], lo[2];
     };
-    __device__ static void load(Raw& r, const uint8_t* p, uint32_t n, uint32_t kh) {
-#pragma unroll
-        for (uint32_t g = 0; g < 4; ++g) r.q[g] = ig_ld16(p + (g / 2) * 1024 + (16 * (2 * (g % 2) + kh) + n) * 16);
-        r.h = ig_ld16(p + 2048 + n * 16);
+    __device__ static void head(Raw& r, const uint8_t* p, uint32_t n) { r.h = ig_ld16(p + 2048 + n * 16); }
+    template <int S>
+    __device__ static void refill(Raw& r, const uint8_t* p, uint32_t n, uint32_t kh) {
+        if (S & 1) r.q[S / 2] = ig_ld16(p + (S / 4) * 1024 + (16 * (2 * (S / 2 % 2) + kh) + n) * 16);
     }
     __device__ static Pre pre(const Raw& r, uint32_t) {
         const IgHead q = ig_head(r.h);
@@ -386,11 +393,11 @@ struct Ig<kQ5_K> {
     struct Pre {
         uint32_t sc[2];
     };
-    __device__ static void load(Raw& r, const uint8_t* p, uint32_t n, uint32_t kh) {
-#pragma unroll
-        for (uint32_t g = 0; g < 4; ++g) r.q[g] = ig_ld16(p + (g / 2) * 1024 + (16 * (2 * (g % 2) + kh) + n) * 16);
-        r.qh = ig_ld16(p + 2048 + n * 32 + 16 * kh);
-        r.h = ig_ld16(p + 2560 + n * 16);
+    __device__ static void head(Raw& r, const uint8_t* p, uint32_t n) { r.h = ig_ld16(p + 2560 + n * 16); }
+    template <int S>
+    __device__ static void refill(Raw& r, const uint8_t* p, uint32_t n, uint32_t kh) {
+        if (S & 1) r.q[S / 2] = ig_ld16(p + (S / 4) * 1024 + (16 * (2 * (S / 2 % 2) + kh) + n) * 16);
+        if (S == 7) r.qh = ig_ld16(p + 2048 + n * 32 + 16 * kh);
     }
     __device__ static Pre pre(const Raw& r, uint32_t) {
         const IgHead q = ig_head(r.h);
@@ -425,13 +432,14 @@ struct Ig<kQ6_K> {
     struct Pre {
         uint32_t c[4];
     };
-    __device__ static void load(Raw& r, const uint8_t* p, uint32_t n, uint32_t kh) {
-#pragma unroll
-        for (uint32_t k = 0; k < 4; ++k) r.ql[k] = ig_ld16(p + kh * 1024 + (16 * k + n) * 16);
-#pragma unroll
-        for (uint32_t g = 0; g < 2; ++g) r.qh[g] = ig_ld16(p + 2048 + n * 64 + 32 * g + 16 * kh);
+    __device__ static void head(Raw& r, const uint8_t* p, uint32_t n) {
         r.sc = ig_ld16(p + 3072 + n * 16);
         r.d = *(const uint16_t*)(p + 3328 + n * 2);
+    }
+    template <int S>
+    __device__ static void refill(Raw& r, const uint8_t* p, uint32_t n, uint32_t kh) {
+        if (S % 4 >= 2) r.ql[2 * (S / 4) + S % 2] = ig_ld16(p + kh * 1024 + (16 * (2 * (S / 4) + S % 2) + n) * 16);
+        if (S % 4 == 3) r.qh[S / 4] = ig_ld16(p + 2048 + n * 64 + 32 * (S / 4) + 16 * kh);
     }
     __device__ static Pre pre(const Raw& r, uint32_t kh) {
         Pre o;
@@ -458,6 +466,20 @@ struct Ig<kQ6_K> {
     }
     __device__ static float d(const Raw& r) { return half_to_float(r.d); }
 };
+
+template <int S>
+using IgStep = std::integral_constant<int, S>;
+// f(IgStep<0>), ..., f(IgStep<7>)
+template <typename F>
+__device__ __forceinline__ void ig_steps(F&& f) {
+    f(IgStep<0>{}), f(IgStep<1>{}), f(IgStep<2>{}), f(IgStep<3>{});
+    f(IgStep<4>{}), f(IgStep<5>{}), f(IgStep<6>{}), f(IgStep<7>{});
+}
+template <uint32_t T>
+__device__ __forceinline__ void ig_load(typename Ig<T>::Raw& r, const uint8_t* p, uint32_t n, uint32_t kh) {
+    ig_steps([&](auto s) { Ig<T>::template refill<decltype(s)::value>(r, p, n, kh); });
+    Ig<T>::head(r, p, n);
+}
 
 // Q8_0: a chunk of four layout pairs (eight blocks of 32)
 struct IgQ8Raw {
@@ -496,9 +518,63 @@ __device__ __forceinline__ void ig_barrier() {
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
+// LDS writes of every wave are visible after it; loads to registers stay in flight.
+__device__ __forceinline__ void ig_lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
 template <uint32_t T, int TT, int KS>
 constexpr uint32_t ig_lds() {
     return 2u * KS * TT * ig_pieces(T) * 1024u;
+}
+
+// One block's term before the activation scale, from its integers.
+template <uint32_t T>
+__device__ __forceinline__ float ig_term(int32_t A, int32_t B, float mn, float d, float dmin) {
+    const int32_t I = Ig<T>::kPlanes == 2 ? (int32_t)(((uint32_t)A << Ig<T>::kShift) + (uint32_t)B) : A;
+    const float t = d * (float)I;
+    return ig_mins(T) ? __builtin_fmaf(-dmin, mn, t) : t;
+}
+// Q2_K's whole term, in the reference's operations (matvec_extra.rs:193-195).
+__device__ __forceinline__ float ig_q2_term(int32_t I, float mn, float da, float d, float dmin) {
+    return (da * d) * (float)I - (da * dmin) * mn;
+}
+
+// The matrix of column tile `tile` (kIgNone: nothing to do), and how many of its
+// columns are live.
+__device__ __forceinline__ uint32_t ig_matrix(const IgMap& map, uint32_t tile, uint32_t& live) {
+    if (map.tile_mat) {
+        const uint32_t v = map.tile_mat[tile];
+        live = kIgTok;
+        if (v >= kIgZero) return v;
+        live = v >> 16;
+        return v & 0xffffu;
+    }
+    const uint32_t k = map.one ? 0 : tile / map.tpg, j = (tile - k * map.tpg) * kIgTok;
+    if (j >= map.cpg) return kIgNone;  // a tile of padding
+    live = map.cpg - j < kIgTok ? map.cpg - j : kIgTok;
+    if (map.one) return 0;
+    return k / map.wn2 / map.r3 * map.wn2 + k % map.wn2;
+}
+// Stores value i of a lane's sixteen (column 8 (i / 4) + 4 kh + i % 4 of the tile) of
+// weight row `row`: the live columns of a group follow each other.
+struct IgStore {
+    float* y;             // column 0 of the tile, or output row 0
+    uint32_t live;
+    const int32_t* rows;  // the output row of each column (-1: none), or null
+};
+__device__ __forceinline__ IgStore ig_store(const IgArgs& g, uint32_t tile, uint32_t row) {
+    const IgMap& map = g.map;
+    if (map.tile_mat) return IgStore{g.y + row, 0, map.row + tile * kIgTok};
+    const uint32_t k = map.one ? 0 : tile / map.tpg, j = (tile - k * map.tpg) * kIgTok;
+    return IgStore{g.y + ((uint64_t)k * map.cpg + j) * g.ldy + row, map.cpg > j ? map.cpg - j : 0, nullptr};
+}
+__device__ __forceinline__ void ig_put(const IgStore& o, uint64_t ldy, uint32_t i, uint32_t kh, float v) {
+    const uint32_t tok = 8 * (i / 4) + 4 * kh + (i % 4);
+    if (o.rows) {
+        const int32_t r = o.rows[tok];
+        if (r >= 0) o.y[(uint64_t)r * ldy] = v;
+    } else if (tok < o.live) {
+        o.y[tok * ldy] = v;
+    }
 }
 
 // A workgroup of four waves: RW = 4 / KS waves side by side along the rows (32
@@ -510,8 +586,8 @@ constexpr uint32_t ig_lds() {
 // Bound: many columns, the VALU (unpacking the weights, about 11 operations
 // per four Q5_K / Q6_K values and wave, and three to five per output and block)
 // beside the MFMAs: Q6_K 4096x14336, 1000 columns, 193 us = 610 TOP/s (8.24 ms
-// in passes of 8 columns); Q3_K 14336x4096, 512 columns, 87 us.  Few columns:
-// the memory latency of each wave's steps, about 1.4 us.
+// in passes of 8 columns); Q3_K 14336x4096, 512 columns, 87 us.  A step takes at
+// least the memory latency, about 1.4 us: few tiles have a kernel of their own.
 template <uint32_t T, int TT, int KS>
 __global__ __launch_bounds__(256, TT == 1 ? 3 : 2) void igemm_kernel(IgArgs g) {
     constexpr int RW = 4 / KS;
@@ -526,15 +602,9 @@ __global__ __launch_bounds__(256, TT == 1 ? 3 : 2) void igemm_kernel(IgArgs g) {
     const uint32_t id = xcd * per + (xcd < rest ? xcd : rest) + blockIdx.x / 8;
     const uint32_t nt = id / g.MT, mt = id % g.MT;
     const uint8_t* w = g.w;
-    uint32_t mat = 0;
-    if (g.map.tile_mat) {
-        mat = g.map.tile_mat[mt * TT];
-        if (mat == kIgNone) return;
-    } else {
-        const uint32_t k = mt * TT / g.map.tpg;
-        if (mt * TT % g.map.tpg * kIgTok >= g.map.cpg) return;  // a tile of padding
-        mat = k / g.map.wn2 / g.map.r3 * g.map.wn2 + k % g.map.wn2;
-    }
+    uint32_t live;  // (every column is multiplied)
+    const uint32_t mat = ig_matrix(g.map, mt * TT, live);
+    if (mat == kIgNone) return;
     if (mat != kIgZero) w += (uint64_t)mat * g.mat_bytes;
     const uint32_t nchunk = g.nchunk, steps = (nchunk + KS - 1) / KS;
     uint32_t t16 = (nt * RW + rw) * 2 + (ln >> 4);
@@ -573,7 +643,7 @@ __global__ __launch_bounds__(256, TT == 1 ? 3 : 2) void igemm_kernel(IgArgs g) {
                 r.d[j] = *(const uint32_t*)(p + 1024 + n * 4);
             }
         } else {
-            Ig<T>::load(r, w + ((uint64_t)t16 * nchunk + c) * Ig<T>::kChunk, n, kh);
+            ig_load<T>(r, w + ((uint64_t)t16 * nchunk + c) * Ig<T>::kChunk, n, kh);
         }
     };
 
@@ -631,7 +701,7 @@ __global__ __launch_bounds__(256, TT == 1 ? 3 : 2) void igemm_kernel(IgArgs g) {
                 i32x16 A[TT], B[TT];
 #pragma unroll
                 for (int t = 0; t < TT; ++t) A[t] = (i32x16){}, B[t] = (i32x16){};
-                auto kstep = [&](auto s_) {
+                ig_steps([&](auto s_) {
                     constexpr int S = decltype(s_)::value;
                     i32x4 wa, wb;
                     W::template ops<S>(cur, pre, wa, wb);
@@ -641,15 +711,7 @@ __global__ __launch_bounds__(256, TT == 1 ? 3 : 2) void igemm_kernel(IgArgs g) {
                         A[t] = ig_mfma(a, wa, A[t]);
                         if (W::kPlanes == 2) B[t] = ig_mfma(a, wb, B[t]);
                     }
-                };
-                kstep(std::integral_constant<int, 0>{});
-                kstep(std::integral_constant<int, 1>{});
-                kstep(std::integral_constant<int, 2>{});
-                kstep(std::integral_constant<int, 3>{});
-                kstep(std::integral_constant<int, 4>{});
-                kstep(std::integral_constant<int, 5>{});
-                kstep(std::integral_constant<int, 6>{});
-                kstep(std::integral_constant<int, 7>{});
+                });
                 const float d = W::d(cur);
                 float dmin = 0.0f;
                 f16x8 mins = {};
@@ -668,16 +730,10 @@ __global__ __launch_bounds__(256, TT == 1 ? 3 : 2) void igemm_kernel(IgArgs g) {
 #pragma unroll
                         for (int k = 0; k < 4; ++k) {
                             const int i = 4 * q + k;
-                            const int32_t I = W::kPlanes == 2 ? (int32_t)(((uint32_t)A[t][i] << W::kShift) + (uint32_t)B[t][i])
-                                                              : A[t][i];
-                            if constexpr (T == kQ2_K) {  // matvec_extra.rs:193-195
-                                const float term = (dv[k] * d) * (float)I - (dv[k] * dmin) * mn[i];
-                                y[t][i] = y[t][i] + term;
-                            } else {
-                                float term = d * (float)I;
-                                if constexpr (ig_mins(T)) term = __builtin_fmaf(-dmin, mn[i], term);
-                                y[t][i] = __builtin_fmaf(dv[k], term, y[t][i]);
-                            }
+                            if constexpr (T == kQ2_K)
+                                y[t][i] = y[t][i] + ig_q2_term(A[t][i], mn[i], dv[k], d, dmin);
+                            else
+                                y[t][i] = __builtin_fmaf(dv[k], ig_term<T>(A[t][i], B[t][i], mn[i], d, dmin), y[t][i]);
                         }
                     }
                 }
@@ -709,19 +765,243 @@ __global__ __launch_bounds__(256, TT == 1 ? 3 : 2) void igemm_kernel(IgArgs g) {
     if (row >= g.rows) return;
 #pragma unroll
     for (int t = 0; t < TT; ++t) {
-        const uint32_t tile = mt * TT + t;
+        const IgStore o = ig_store(g, mt * TT + t, row);
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const uint32_t tok = 8 * (i / 4) + 4 * kh + (i % 4);
-            if (g.map.tile_mat) {
-                const int32_t r = g.map.row[tile * kIgTok + tok];
-                if (r >= 0) g.y[(uint64_t)r * g.ldy + row] = y[t][i];
-            } else {
-                const uint32_t k = tile / g.map.tpg, j = tile % g.map.tpg * kIgTok + tok;
-                if (j < g.map.cpg) g.y[((uint64_t)k * g.map.cpg + j) * g.ldy + row] = y[t][i];
+        for (int i = 0; i < 16; ++i) ig_put(o, g.ldy, i, kh, y[t][i]);
+    }
+}
+
+// Few tiles: one (32 rows x 32 columns) tile per workgroup, its chunks dealt to
+// KS waves.  Nothing is staged: a wave reads its weights and activations
+// straight into the registers that the k-steps free, one chunk ahead (the
+// activations half a chunk), so the
+// waves run apart and only meet to add up.  Q2_K parks each chunk's terms in
+// LDS and every wave adds its share of the tile in block order.
+//
+// Bound: memory latency (a wave has two to four chunks), then the activations'
+// way from L2 (8 KB a chunk and tile; lanes of dead columns read column 0).
+// 14336x4096, 16 columns: Q4_K 13.9 us with the image's kernel (24.3 with staged
+// activations and K split in two, 23.8 in decode passes), Q2_K 12.8 (25.4, 32.3);
+// 4096x14336: Q2_K 15.5 (68, 123), whose staged kernel cannot split K.
+template <uint32_t T, int KS>
+__global__ __launch_bounds__(64 * KS) __attribute__((amdgpu_waves_per_eu(KS == 4 ? 3 : 4))) void igemm_few_kernel(IgArgs g) {
+    constexpr uint32_t kTile = ig_pieces(T) * 1024;
+    constexpr int kOwn = 16 / KS;  // accumulators of the tile that a wave adds up
+    using W = Ig<T>;
+    if (g.gate && *g.gate) return;
+    __shared__ float part[(T == kQ2_K ? 2 : 1) * KS][16][64];
+    __shared__ __align__(16) float das[KS][32];
+    const uint32_t lane = threadIdx.x & 63, kg = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t ln = lane & 31, kh = lane >> 5, n = ln & 15, nchunk = g.nchunk;
+    const uint32_t G = g.NT * g.MT, per = G / 8, rest = G % 8, xcd = blockIdx.x % 8;
+    const uint32_t id = xcd * per + (xcd < rest ? xcd : rest) + blockIdx.x / 8;
+    const uint32_t nt = id / g.MT, mt = id % g.MT;
+    uint32_t live;
+    const uint32_t mat = ig_matrix(g.map, mt, live);
+    if (mat == kIgNone) return;
+    const bool zero = mat == kIgZero;
+    uint32_t t16 = nt * 2 + (ln >> 4);
+    t16 = t16 < g.ntiles16 ? t16 : g.ntiles16 - 1;
+    const uint8_t* wt = g.w + (zero ? 0 : (uint64_t)mat * g.mat_bytes) + (uint64_t)t16 * nchunk * W::kChunk;
+    const uint32_t col = ln < live ? ln : 0;
+    const uint8_t* at = g.img + (uint64_t)mt * nchunk * kTile;
+
+    typename W::Raw r;
+    i32x4 act[4];
+    float da = 0.0f;
+    f16x8 bs = {};
+    auto load_act = [&](int s, uint32_t c) {
+        act[s % 4] = *(const i32x4*)(at + (uint64_t)c * kTile + s * 1024 + kh * 512 + col * 16);
+    };
+    auto load_scales = [&](uint32_t c) {
+        da = *(const float*)(at + (uint64_t)c * kTile + kIgD + col * 4);
+        if (ig_mins(T)) bs = *(const f16x8*)(at + (uint64_t)c * kTile + kIgBsum + kh * 512 + col * 16);
+    };
+    const uint32_t c0 = kg < nchunk ? kg : nchunk - 1;
+#pragma unroll
+    for (int s = 0; s < 4; ++s) load_act(s, c0);
+    load_scales(c0);
+    ig_load<T>(r, wt + (uint64_t)c0 * W::kChunk, n, kh);
+    int bad = 0;
+    for (uint32_t i = threadIdx.x; i < g.nflags; i += 64 * KS) bad |= (int)g.flags[i];
+    if (__syncthreads_or(bad)) return;
+
+    float y[16], own[kOwn];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) y[i] = 0.0f;
+#pragma unroll
+    for (int i = 0; i < kOwn; ++i) own[i] = 0.0f;
+    // one chunk; more: the loads of chunk c + KS follow the last use of what
+    // they replace.  Q2_K: y is the chunk's term, otherwise the running sum.
+    auto chunk = [&](auto more_, uint32_t c) {
+        constexpr bool more = decltype(more_)::value;
+        const uint8_t* wn = wt + (uint64_t)(c + KS) * W::kChunk;
+        const typename W::Pre pre = W::pre(r, kh);
+        const float d = W::d(r);
+        float dmin = 0.0f;
+        f16x8 mins = {};
+        if constexpr (ig_mins(T)) dmin = W::dmin(r), mins = W::mins(r, kh);
+        if (kh == 0) das[kg][ln] = da;
+        if (more) W::head(r, wn, n);
+        i32x16 A = {}, B = {};
+        ig_steps([&](auto s_) {
+            constexpr int S = decltype(s_)::value;
+            i32x4 wa, wb;
+            W::template ops<S>(r, pre, wa, wb);
+            A = ig_mfma(act[S % 4], wa, A);
+            if (W::kPlanes == 2) B = ig_mfma(act[S % 4], wb, B);
+            if (more) W::template refill<S>(r, wn, n, kh);
+            if (S < 4) load_act(S + 4, c);
+            else if (more) load_act(S - 4, c + KS);
+        });
+        f32x16 mn = {};
+        if constexpr (ig_mins(T)) mn = __builtin_amdgcn_mfma_f32_32x32x16_f16(bs, mins, (f32x16){}, 0, 0, 0);
+        if (more) load_scales(c + KS);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const float4 dq = *(const float4*)&das[kg][8 * q + 4 * kh];
+            const float dv[4] = {dq.x, dq.y, dq.z, dq.w};
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const int i = 4 * q + k;
+                if constexpr (T == kQ2_K) y[i] = ig_q2_term(A[i], mn[i], dv[k], d, dmin);
+                else y[i] = __builtin_fmaf(dv[k], ig_term<T>(A[i], B[i], mn[i], d, dmin), y[i]);
             }
         }
+    };
+    if constexpr (T == kQ2_K) {
+        for (uint32_t it = 0; it * KS < nchunk && !zero; ++it) {
+            const uint32_t c = it * KS + kg;
+            float(*p)[16][64] = part + (it & 1) * KS;
+            if (c < nchunk) {
+                if (c + KS < nchunk) chunk(std::true_type{}, c);
+                else chunk(std::false_type{}, c);
+#pragma unroll
+                for (int i = 0; i < 16; ++i) p[kg][i][lane] = y[i];
+            }
+            ig_lds_barrier();  // (two buffers: the next step's terms go to the other one)
+            const uint32_t m = nchunk - it * KS < KS ? nchunk - it * KS : KS;
+            for (uint32_t j = 0; j < m; ++j)
+#pragma unroll
+                for (int i = 0; i < kOwn; ++i) own[i] = own[i] + p[j][kg * kOwn + i][lane];
+        }
+    } else {
+        if (!zero && kg < nchunk) {
+            uint32_t c = kg;
+            for (; c + KS < nchunk; c += KS) chunk(std::true_type{}, c);
+            chunk(std::false_type{}, c);
+        }
+#pragma unroll
+        for (int i = 0; i < 16; ++i) part[kg][i][lane] = y[i];
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < KS; ++j)
+#pragma unroll
+            for (int i = 0; i < kOwn; ++i) own[i] += part[j][kg * kOwn + i][lane];
     }
+    const uint32_t row = nt * 32 + ln;
+    if (row >= g.rows) return;
+    const IgStore o = ig_store(g, mt, row);
+#pragma unroll
+    for (int k = 0; k < kOwn; ++k) ig_put(o, g.ldy, kg * kOwn + k, kh, own[k]);
+}
+
+// Few tiles of Q8_0: eight waves take one pair of blocks each per step, three
+// steps ahead (19 registers a step), park both blocks' terms in LDS, and every
+// wave adds two of the tile's sixteen accumulators over the step's sixteen
+// blocks in order.  One buffer and two barriers a step, so that two workgroups
+// fit a CU's LDS.  Bound: a step's LDS traffic (128 KB a workgroup) and f32 terms,
+// 1.2 to 1.4 us.  4096x4096, 16 columns: 16.8 us (46 staged, 27 in decode passes);
+// 4096x14336: 39 (138, 187).
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void igemm_few_q8_kernel(IgArgs g) {
+    constexpr int KS = 8, D = 3;
+    constexpr uint32_t kTile = ig_pieces(kQ8_0) * 1024;
+    if (g.gate && *g.gate) return;
+    __shared__ __align__(16) float2 part[2 * KS][8][64];  // [block][accumulator pair][lane]
+    __shared__ __align__(16) float das[KS][2][32];
+    const uint32_t lane = threadIdx.x & 63, kg = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t ln = lane & 31, kh = lane >> 5, n = ln & 15, npairs = g.npairs;
+    const uint32_t G = g.NT * g.MT, per = G / 8, rest = G % 8, xcd = blockIdx.x % 8;
+    const uint32_t id = xcd * per + (xcd < rest ? xcd : rest) + blockIdx.x / 8;
+    const uint32_t nt = id / g.MT, mt = id % g.MT;
+    uint32_t live;
+    const uint32_t mat = ig_matrix(g.map, mt, live);
+    if (mat == kIgNone) return;
+    const bool zero = mat == kIgZero;
+    uint32_t t16 = nt * 2 + (ln >> 4);
+    t16 = t16 < g.ntiles16 ? t16 : g.ntiles16 - 1;
+    const uint8_t* wt = g.w + (zero ? 0 : (uint64_t)mat * g.mat_bytes) + (uint64_t)t16 * npairs * kQ80Chunk;
+    const uint32_t col = ln < live ? ln : 0, steps = zero ? 0 : (npairs + KS - 1) / KS;
+    const uint8_t* at = g.img + (uint64_t)mt * g.nchunk * kTile;
+
+    struct Step {
+        i32x4 w[2], a[2];
+        uint32_t dw;
+        float da[2];
+    } buf[D];
+    auto load = [&](Step& q, uint32_t it) {
+        const uint32_t want = it * KS + kg, P = want < npairs ? want : npairs - 1;
+        const uint8_t* p = wt + (uint64_t)P * kQ80Chunk;
+        const uint8_t* x = at + (uint64_t)(P / 4) * kTile;
+#pragma unroll
+        for (uint32_t b = 0; b < 2; ++b) {
+            const uint32_t s = 2 * (P % 4) + b;
+            q.w[b] = *(const i32x4*)(p + (16 * (2 * b + kh) + n) * 16);
+            q.a[b] = *(const i32x4*)(x + s * 1024 + kh * 512 + col * 16);
+            q.da[b] = *(const float*)(x + kIgD + s * 128 + col * 4);
+        }
+        q.dw = *(const uint32_t*)(p + 1024 + n * 4);
+    };
+#pragma unroll
+    for (int d = 0; d < D; ++d) load(buf[d], d);
+    int bad = 0;
+    for (uint32_t i = threadIdx.x; i < g.nflags; i += 64 * KS) bad |= (int)g.flags[i];
+    if (__syncthreads_or(bad)) return;
+
+    float own[2] = {0.0f, 0.0f};
+    auto step = [&](Step& q, uint32_t it) {
+        if (it * KS + kg < npairs) {
+#pragma unroll
+            for (int b = 0; b < 2; ++b) {
+                if (kh == 0) das[kg][b][ln] = q.da[b];
+                const float dw = half_to_float(b ? q.dw >> 16 : q.dw);
+                const i32x16 I = ig_mfma(q.a[b], q.w[b], (i32x16){});
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    const float4 dq = *(const float4*)&das[kg][b][8 * k + 4 * kh];  // matvec.rs:124-128
+                    part[2 * kg + b][2 * k][lane] = make_float2((float)I[4 * k] * (dw * dq.x), (float)I[4 * k + 1] * (dw * dq.y));
+                    part[2 * kg + b][2 * k + 1][lane] =
+                        make_float2((float)I[4 * k + 2] * (dw * dq.z), (float)I[4 * k + 3] * (dw * dq.w));
+                }
+            }
+        }
+        load(q, it + D);
+        ig_lds_barrier();
+        const uint32_t left = npairs - it * KS, m = 2 * (left < KS ? left : KS);
+        if (m == 2 * KS) {
+#pragma unroll
+            for (int j = 0; j < 2 * KS; ++j) {
+                const float2 t = part[j][kg][lane];
+                own[0] = own[0] + t.x, own[1] = own[1] + t.y;
+            }
+        } else {
+            for (uint32_t j = 0; j < m; ++j) {
+                const float2 t = part[j][kg][lane];
+                own[0] = own[0] + t.x, own[1] = own[1] + t.y;
+            }
+        }
+        ig_lds_barrier();
+    };
+    for (uint32_t it = 0; it < steps; it += D) {
+#pragma unroll
+        for (int d = 0; d < D; ++d)
+            if (it + d < steps) step(buf[d], it + d);
+    }
+    const uint32_t row = nt * 32 + ln;
+    if (row >= g.rows) return;
+    const IgStore o = ig_store(g, mt, row);
+#pragma unroll
+    for (uint32_t k = 0; k < 2; ++k) ig_put(o, g.ldy, kg * 2 + k, kh, own[k]);
 }
 
 // ---------------------------------------------------------------------------
@@ -742,31 +1022,50 @@ static hipError_t ig_launch_one(IgArgs g, uint32_t tiles, hipStream_t s) {
     return hipGetLastError();
 }
 
-// Shape of the workgroups, by the number of (32 rows x 32 columns) tiles.
-// Up to 512 of them leave most SIMDs idle: four waves split K (1024x4096, 77
-// columns, Q4_K / Q5_K / Q6_K: 13.4 / 16.2 / 14.2 us against 26 / 36 / 29
-// without); up to 1100, two do (14336x4096, 64 columns: 21.9 / 31.5 / 29.9
-// against 28.7 / 39 / 31.8).  Beyond, a wave takes two column tiles, so that
-// the weights it unpacks serve both (14336x4096, 512 columns, Q3_K / Q5_K /
-// Q6_K: 87 / 116 / 109 us against 124 / 147 / 153), with K still split in two
-// up to 3000 tiles (4096x4096, 512 columns: Q3_K 36.1 against 41.5, Q6_K 38.8
-// against 42.1).  Q4_K unpacks in fewest steps and keeps one column tile up to
-// 4000 tiles (37 us against 45); Q8_0 and Q2_K cannot split K, and Q8_0, whose
-// work is the f32 terms, keeps one column tile throughout (124 us against 137).
-// pairs: two neighbouring column tiles may share a wave.
+template <uint32_t T, int KS>
+static hipError_t ig_launch_few(IgArgs g, uint32_t tiles, hipStream_t s) {
+    g.NT = (g.rows + 31) / 32;
+    g.MT = tiles;
+    const uint64_t grid = (uint64_t)g.NT * g.MT;
+    if (grid == 0 || grid > 0x7fffffffull) return hipErrorInvalidValue;
+    if constexpr (T == kQ8_0) hipLaunchKernelGGL(igemm_few_q8_kernel, dim3((unsigned)grid), dim3(512), 0, s, g);
+    else hipLaunchKernelGGL((igemm_few_kernel<T, KS>), dim3((unsigned)grid), dim3(64 * KS), 0, s, g);
+    return hipGetLastError();
+}
+
+// The kernel, by the number n of (32 rows x 32 columns) tiles; us of both sides
+// at 4096 columns unless said otherwise.  pairs: two neighbouring column tiles
+// may share a wave.
+//  - One tile per workgroup while that still gives few workgroups.  16 waves to
+//    160 tiles (4096x14336, 16 columns: Q4_K 16.3 against 18.7 with 8, Q2_K 15.5
+//    against 18.0), 8 to 512 (14336 rows, 16 columns: Q4_K 13.9 against 15.6 with
+//    4), then 4 until the kernel below, whose waves share activations, is
+//    faster: 1700 tiles of Q3_K and Q6_K (4096 rows, 384 columns = 1536: 35.2
+//    against 36.3 and 38.1 against 40.1; 512 columns = 2048: 43.6 against 38.1 and
+//    47.2 against 42.0), 2048 of Q2_K (32.5 against 34.7; 14336 rows, 192 columns
+//    = 2688: 38.0 against 38.6), 2700 of Q5_K (59.3 against 80; 256 columns = 3584:
+//    76.8 against 67.4), 3500 of Q4_K (43.0 against 45.8; 53.0 against 56.1), and
+//    4000 where column tiles cannot be paired.  Q8_0 to 1024 (4096 rows, 256
+//    columns: 40 against 48; 384 = 1536: 56 against 50).
+//  - Beyond, two column tiles a wave, so that the weights it unpacks serve both
+//    (14336 rows, 512 columns, Q3_K / Q5_K / Q6_K: 87 / 116 / 109 against 124 / 147 /
+//    153), with K split in two to 3000 tiles (4096 rows, 512 columns: Q3_K 36.1
+//    against 41.5, Q6_K 38.8 against 42.1).  Q2_K, whose unpacking is short, from
+//    4000 tiles on; Q8_0, whose work is the f32 terms, never (124 against 137).
 template <uint32_t T>
 static hipError_t ig_launch(const IgArgs& g, uint32_t tiles, bool pairs, hipStream_t s) {
     const uint64_t live = g.map.tile_mat ? tiles : (uint64_t)tiles / g.map.tpg * ((g.map.cpg + kIgTok - 1) / kIgTok);
     const uint64_t n = (uint64_t)((g.rows + 31) / 32) * live;
     if constexpr (T == kQ8_0) {
-        return ig_launch_one<T, 1, 1>(g, tiles, s);
+        return n <= 1024 ? ig_launch_few<T, 8>(g, tiles, s) : ig_launch_one<T, 1, 1>(g, tiles, s);
     } else {
-        if constexpr (T != kQ2_K) {
-            if (n <= 512) return ig_launch_one<T, 1, 4>(g, tiles, s);
-            if (n <= 1100) return ig_launch_one<T, 1, 2>(g, tiles, s);
-            if (T != kQ4_K && n <= 3000 && pairs) return ig_launch_one<T, 2, T == kQ4_K ? 1 : 2>(g, tiles, s);
-        }
-        if (!pairs || n <= (T == kQ2_K || T == kQ4_K ? 4000 : 0)) return ig_launch_one<T, 1, 1>(g, tiles, s);
+        constexpr uint64_t kFew = T == kQ2_K ? 2048 : (T == kQ4_K ? 3500 : (T == kQ5_K ? 2700 : 1700));
+        if (n <= 160 && g.nchunk >= 16) return ig_launch_few<T, 16>(g, tiles, s);
+        if (n <= 512) return ig_launch_few<T, 8>(g, tiles, s);
+        if (n <= (pairs ? kFew : 4000)) return ig_launch_few<T, 4>(g, tiles, s);
+        if (!pairs || (T == kQ2_K && n <= 4000)) return ig_launch_one<T, 1, 1>(g, tiles, s);
+        if constexpr (T == kQ3_K || T == kQ6_K)
+            if (n <= 3000) return ig_launch_one<T, 2, 2>(g, tiles, s);
         return ig_launch_one<T, 2, 1>(g, tiles, s);
     }
 }
@@ -842,6 +1141,7 @@ hipError_t launch_igemm(uint32_t t, const uint8_t* w, uint64_t rows, uint64_t co
     if (st.cpg == 0 || st.groups == 0 || tiles > (1u << 20)) return hipErrorInvalidValue;
     IgMap map{};
     map.cpg = (uint32_t)st.cpg, map.tpg = (uint32_t)tpg, map.wn2 = (uint32_t)st.wn2, map.r3 = (uint32_t)st.r3;
+    map.one = st.groups == 1;
     return ig_run(t, w, rows, cols, st.mat_bytes, x, packed, map, (uint32_t)tiles, tpg % 2 == 0,
                   ig_carve(scratch, t, tiles, cols), y, ldy, nullptr, err_word, s);
 }
@@ -901,7 +1201,14 @@ __global__ __launch_bounds__(1024) void igemm_route_kernel(IgRoute r, uint32_t t
     for (uint32_t t = tid; t < tiles; t += 1024) {
         uint32_t m = 0;
         while (m <= r.mats && first[m + 1] <= t) ++m;
-        tile_mat[t] = m > r.mats ? kIgNone : (m == r.mats ? kIgZero : m);
+        uint32_t v = kIgNone;
+        if (m == r.mats) {
+            v = kIgZero;
+        } else if (m < r.mats) {  // (a group's second tile may be empty: one column, of zeros)
+            const uint32_t at = (t - first[m]) * kIgTok, left = count[m] > at ? count[m] - at : 1;
+            v = m | (left < kIgTok ? left : kIgTok) << 16;
+        }
+        tile_mat[t] = v;
     }
     __syncthreads();
     for (uint32_t i = tid; i <= r.mats; i += 1024) count[i] = 0;
