@@ -489,10 +489,13 @@ hipError_t decode_launch(rlq_context* ctx, const rlq_weights* w, const float* x,
 // 8 columns), the 128-column Q4_K GEMM, or the int8 GEMM of every format.
 enum class Route { kDecode, kGemm, kIgemm };
 
-// The Q4_K GEMM's workgroups take 128 columns x 256 rows and one CU each: from
-// three quarters of the CUs on it is the faster one (14336x4096, 512 columns =
-// 224 workgroups: 73 us against 95), below that the int8 GEMM's smaller tiles
-// are (4096x4096, 512 columns = 64 workgroups: 36 us).
+// The Q4_K GEMM's workgroups take 128 columns x 256 rows and one CU each, so
+// its time is that of whole rounds of the CUs (73 us at 4096 values a row); the
+// int8 GEMM's follows the rows times the columns (in pairs of 32) and is the
+// shorter one below about 5.8 million a round: us at 4096 values, int8 against
+// Q4_K GEMM: 14336 rows, 256 / 384 / 400 / 512 / 640 columns 49 / 64 / 80 / 83 /
+// 102 against 69 / 73 / 75 / 77 / 134; 4096 rows, 1024 columns 53 against 72; 60000
+// rows of 1024 values, 64 / 96 columns 22.8 / 30.2 against 26.6 / 28.1.
 //
 // Up to 8 columns the decode kernels read the weights once, with no launch
 // before them.  The int8 GEMM's two launches are faster where those kernels
@@ -508,8 +511,12 @@ enum class Route { kDecode, kGemm, kIgemm };
 // Not with an argmax, which the decode kernels finish in the same launch, and
 // not for the output head's row counts, where they are near the memory rate.
 Route matmul_route(uint32_t dtype, uint64_t rows, uint64_t cols, uint64_t batch, bool argmax) {
-    if (batch > kDecodeMaxBatch)
-        return dtype == kQ4_K && (rows + 255) / 256 * ((batch + 127) / 128) >= 192 ? Route::kGemm : Route::kIgemm;
+    if (batch > kDecodeMaxBatch) {
+        if (dtype != kQ4_K) return Route::kIgemm;
+        const uint64_t cus = (uint64_t)device_cus(), groups = (rows + 255) / 256 * ((batch + 127) / 128);
+        const uint64_t rounds = (groups + cus - 1) / cus;
+        return rows * ((batch + 63) / 64 * 64) < rounds * 5800000 ? Route::kIgemm : Route::kGemm;
+    }
     if (batch < 2 || argmax || rows > 32768) return Route::kDecode;
     const bool igemm = dtype == kQ6_K   ? batch == 2 || cols >= 2048
                        : dtype == kQ2_K ? batch >= 5 && cols >= 2048

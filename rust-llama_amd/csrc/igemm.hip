@@ -223,7 +223,8 @@ __device__ __forceinline__ f16x2 ig_byte_half2(uint32_t w, uint32_t sel) {
 }
 
 // One format: Raw holds a lane's loaded bytes of one (16-row tile, chunk) pair:
-// head loads the scales, refill<S> the pieces that no k-step after S uses; Pre is
+// head loads the scales, refill<S> the pieces that no k-step after S uses (kLoads
+// of them in 16 bytes each, not next to each other); Pre is
 // what a chunk's k-steps share; ops<S> makes the weight operand of k-step S.
 // Lane (ln, kh) of a wave works on row ln % 16 = n of layout tile ln / 16 and k
 // half kh.
@@ -233,6 +234,7 @@ struct Ig;
 template <>
 struct Ig<kQ2_K> {
     static constexpr uint32_t kChunk = kQ2KChunk;
+    static constexpr int kLoads = 3;
     static constexpr int kPlanes = 1, kShift = 0;
     struct Raw {
         uint4 q[2], sc;
@@ -279,6 +281,7 @@ struct Ig<kQ2_K> {
 template <>
 struct Ig<kQ3_K> {
     static constexpr uint32_t kChunk = kQ3KChunk;
+    static constexpr int kLoads = 3;
     static constexpr int kPlanes = 1, kShift = 0;
     struct Raw {
         uint4 q[2], hm;
@@ -352,6 +355,7 @@ __device__ __forceinline__ f16x8 ig_head_mins(const uint4& h, uint32_t kh) {
 template <>
 struct Ig<kQ4_K> {
     static constexpr uint32_t kChunk = kQ4KChunk;
+    static constexpr int kLoads = 5;
     static constexpr int kPlanes = 2, kShift = 3;
     struct Raw {
         uint4 q[4], h;
@@ -386,6 +390,7 @@ struct Ig<kQ4_K> {
 template <>
 struct Ig<kQ5_K> {
     static constexpr uint32_t kChunk = kQ5KChunk;
+    static constexpr int kLoads = 6;
     static constexpr int kPlanes = 2, kShift = 8;
     struct Raw {
         uint4 q[4], qh, h;
@@ -424,6 +429,7 @@ struct Ig<kQ5_K> {
 template <>
 struct Ig<kQ6_K> {
     static constexpr uint32_t kChunk = kQ6KChunk;
+    static constexpr int kLoads = 7;
     static constexpr int kPlanes = 2, kShift = 8;
     struct Raw {
         uint4 ql[4], qh[2], sc;
@@ -482,9 +488,16 @@ __device__ __forceinline__ void ig_load(typename Ig<T>::Raw& r, const uint8_t* p
 }
 
 // Q8_0: a chunk of four layout pairs (eight blocks of 32)
-struct IgQ8Raw {
-    uint4 q[8];
-    uint32_t d[4];
+template <uint32_t T>
+struct IgRaw {
+    using Raw = typename Ig<T>::Raw;
+};
+template <>
+struct IgRaw<kQ8_0> {
+    struct Raw {
+        uint4 q[8];
+        uint32_t d[4];
+    };
 };
 
 // ---------------------------------------------------------------------------
@@ -514,8 +527,11 @@ __device__ __forceinline__ i32x16 ig_mfma(i32x4 a, i32x4 b, i32x16 c) {
 __device__ __forceinline__ void ig_g2l(const void* sbase, uint32_t voff, uint32_t lds) {
     asm volatile("global_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(sbase), "{m0}"(lds));
 }
+// Barrier after which a stage has landed for every wave: at most N of a wave's
+// loads, all younger than the stage's, are still in flight.
+template <int N>
 __device__ __forceinline__ void ig_barrier() {
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
 }
 
 // LDS writes of every wave are visible after it; loads to registers stay in flight.
@@ -580,16 +596,21 @@ __device__ __forceinline__ void ig_put(const IgStore& o, uint64_t ldy, uint32_t 
 // A workgroup of four waves: RW = 4 / KS waves side by side along the rows (32
 // each) times KS along K; every wave takes TT column tiles of 32.  Wave group
 // kg takes chunks kg, kg + KS, ...; its activations are one LDS stage per
-// step, filled one step ahead, its weights go straight to registers, also one
-// step ahead.
+// step, filled one step ahead, its weights go straight to the registers that
+// the k-steps free, so that three waves fit a SIMD (the barrier before a stage
+// leaves those younger loads in flight).  With a second set of weight registers
+// and two waves: Q4_K 4096x14336, 1000 columns 193 us against 176, Q5_K
+// 14336x4096, 512 columns 122 against 111, Q2_K 80 against 77, Q6_K the same.
 //
 // Bound: many columns, the VALU (unpacking the weights, about 11 operations
 // per four Q5_K / Q6_K values and wave, and three to five per output and block)
-// beside the MFMAs: Q6_K 4096x14336, 1000 columns, 193 us = 610 TOP/s (8.24 ms
-// in passes of 8 columns); Q3_K 14336x4096, 512 columns, 87 us.  A step takes at
+// beside the MFMAs, which do not overlap: Q6_K 4096x14336, 1000 columns, 193 us =
+// 610 TOP/s (8.24 ms in passes of 8 columns) at 62 % VALU and 26 % MFMA busy.
+// (Four column tiles a wave, one wave per SIMD, unpack half as often but hide
+// nothing: 220 us against 222, Q5_K 220 against 210.)  A step takes at
 // least the memory latency, about 1.4 us: few tiles have a kernel of their own.
 template <uint32_t T, int TT, int KS>
-__global__ __launch_bounds__(256, TT == 1 ? 3 : 2) void igemm_kernel(IgArgs g) {
+__global__ __launch_bounds__(256, 3) void igemm_kernel(IgArgs g) {
     constexpr int RW = 4 / KS;
     constexpr uint32_t kPieces = ig_pieces(T), kTile = kPieces * 1024, kStage = KS * TT * kTile;
     if (g.gate && *g.gate) return;
@@ -628,8 +649,8 @@ __global__ __launch_bounds__(256, TT == 1 ? 3 : 2) void igemm_kernel(IgArgs g) {
         }
     };
 
-    using F = std::conditional_t<T == kQ8_0, IgQ8Raw, typename std::conditional_t<T == kQ8_0, Ig<kQ6_K>, Ig<T>>::Raw>;
-    F cur, nxt;
+    using F = typename IgRaw<T>::Raw;
+    F cur, nxt;  // nxt: Q8_0 only
     auto load = [&](F& r, uint32_t it) {
         const uint32_t c = chunk_of(it);
         if constexpr (T == kQ8_0) {
@@ -663,83 +684,104 @@ __global__ __launch_bounds__(256, TT == 1 ? 3 : 2) void igemm_kernel(IgArgs g) {
 #pragma unroll
         for (int i = 0; i < 16; ++i) y[t][i] = 0.0f;
 
-    for (uint32_t it = 0; it < (mat == kIgZero ? 0 : steps); ++it) {
-        ig_barrier();  // stage `it` has landed for every wave; the other one is free
-        if (it + 1 < steps) {
-            issue(it + 1);
-            load(nxt, it + 1);
-        }
-        const uint32_t c = it * KS + kg;
-        if (KS == 1 || c < nchunk) {
-            const uint8_t* st = smem + (it & 1) * kStage + kg * (TT * kTile);
+    const uint32_t run = mat == kIgZero ? 0 : steps;
+    if constexpr (T == kQ8_0) {
+        for (uint32_t it = 0; it < run; ++it) {
+            ig_barrier<0>();  // stage `it` has landed for every wave; the other one is free
+            if (it + 1 < steps) {
+                issue(it + 1);
+                load(nxt, it + 1);
+            }
+            const uint8_t* st = smem + (it & 1) * kStage;
             const uint8_t* ab = st + kh * 512 + ln * 16;
-            if constexpr (T == kQ8_0) {
 #pragma unroll
-                for (int s = 0; s < 8; ++s) {
-                    if (4 * c + s / 2 >= g.npairs) break;
-                    const i32x4 b = __builtin_bit_cast(i32x4, cur.q[s]);
-                    const float dw = half_to_float((s & 1) ? cur.d[s / 2] >> 16 : cur.d[s / 2]);
-#pragma unroll
-                    for (int t = 0; t < TT; ++t) {
-                        const i32x4 a = *(const i32x4*)(ab + t * kTile + s * 1024);
-                        const i32x16 I = ig_mfma(a, b, (i32x16){});
-#pragma unroll
-                        for (int q = 0; q < 4; ++q) {
-                            const float4 da = *(const float4*)(st + t * kTile + kIgD + s * 128 + (8 * q + 4 * kh) * 4);
-                            const float dv[4] = {da.x, da.y, da.z, da.w};
-#pragma unroll
-                            for (int k = 0; k < 4; ++k) {
-                                const float term = (float)I[4 * q + k] * (dw * dv[k]);  // matvec.rs:124-128
-                                y[t][4 * q + k] = y[t][4 * q + k] + term;
-                            }
-                        }
-                    }
-                }
-            } else {
-                using W = Ig<T>;
-                const typename W::Pre pre = W::pre(cur, kh);
-                i32x16 A[TT], B[TT];
-#pragma unroll
-                for (int t = 0; t < TT; ++t) A[t] = (i32x16){}, B[t] = (i32x16){};
-                ig_steps([&](auto s_) {
-                    constexpr int S = decltype(s_)::value;
-                    i32x4 wa, wb;
-                    W::template ops<S>(cur, pre, wa, wb);
-#pragma unroll
-                    for (int t = 0; t < TT; ++t) {
-                        const i32x4 a = *(const i32x4*)(ab + t * kTile + S * 1024);
-                        A[t] = ig_mfma(a, wa, A[t]);
-                        if (W::kPlanes == 2) B[t] = ig_mfma(a, wb, B[t]);
-                    }
-                });
-                const float d = W::d(cur);
-                float dmin = 0.0f;
-                f16x8 mins = {};
-                if constexpr (ig_mins(T)) dmin = W::dmin(cur), mins = W::mins(cur, kh);
+            for (int s = 0; s < 8; ++s) {
+                if (4 * it + s / 2 >= g.npairs) break;
+                const i32x4 b = __builtin_bit_cast(i32x4, cur.q[s]);
+                const float dw = half_to_float((s & 1) ? cur.d[s / 2] >> 16 : cur.d[s / 2]);
 #pragma unroll
                 for (int t = 0; t < TT; ++t) {
-                    f32x16 mn = {};
-                    if constexpr (ig_mins(T)) {
-                        const f16x8 bs = *(const f16x8*)(st + t * kTile + kIgBsum + kh * 512 + ln * 16);
-                        mn = __builtin_amdgcn_mfma_f32_32x32x16_f16(bs, mins, (f32x16){}, 0, 0, 0);
-                    }
+                    const i32x4 a = *(const i32x4*)(ab + t * kTile + s * 1024);
+                    const i32x16 I = ig_mfma(a, b, (i32x16){});
 #pragma unroll
                     for (int q = 0; q < 4; ++q) {
-                        const float4 da = *(const float4*)(st + t * kTile + kIgD + (8 * q + 4 * kh) * 4);
+                        const float4 da = *(const float4*)(st + t * kTile + kIgD + s * 128 + (8 * q + 4 * kh) * 4);
                         const float dv[4] = {da.x, da.y, da.z, da.w};
 #pragma unroll
                         for (int k = 0; k < 4; ++k) {
-                            const int i = 4 * q + k;
-                            if constexpr (T == kQ2_K)
-                                y[t][i] = y[t][i] + ig_q2_term(A[t][i], mn[i], dv[k], d, dmin);
-                            else
-                                y[t][i] = __builtin_fmaf(dv[k], ig_term<T>(A[t][i], B[t][i], mn[i], d, dmin), y[t][i]);
+                            const float term = (float)I[4 * q + k] * (dw * dv[k]);  // matvec.rs:124-128
+                            y[t][4 * q + k] = y[t][4 * q + k] + term;
                         }
                     }
                 }
             }
+            cur = nxt;
         }
-        cur = nxt;
+    } else {
+        using W = Ig<T>;
+        // one step; more: the next step's stage is issued first, its weights
+        // follow the last use of the registers they take
+        auto step = [&](auto more_, uint32_t it) {
+            constexpr bool more = decltype(more_)::value;
+            const uint8_t* wn = w + ((uint64_t)t16 * nchunk + chunk_of(it + 1)) * W::kChunk;
+            if (more) {
+                issue(it + 1);
+                asm volatile("" ::: "memory");  // no load of the next weights before the stage's
+            }
+            const uint8_t* st = smem + (it & 1) * kStage + kg * (TT * kTile);
+            const uint8_t* ab = st + kh * 512 + ln * 16;
+            const typename W::Pre pre = W::pre(cur, kh);
+            const float d = W::d(cur);
+            float dmin = 0.0f;
+            f16x8 mins = {};
+            if constexpr (ig_mins(T)) dmin = W::dmin(cur), mins = W::mins(cur, kh);
+            if (more) W::head(cur, wn, n);
+            i32x16 A[TT], B[TT];
+#pragma unroll
+            for (int t = 0; t < TT; ++t) A[t] = (i32x16){}, B[t] = (i32x16){};
+            ig_steps([&](auto s_) {
+                constexpr int S = decltype(s_)::value;
+                i32x4 wa, wb;
+                W::template ops<S>(cur, pre, wa, wb);
+#pragma unroll
+                for (int t = 0; t < TT; ++t) {
+                    const i32x4 a = *(const i32x4*)(ab + t * kTile + S * 1024);
+                    A[t] = ig_mfma(a, wa, A[t]);
+                    if (W::kPlanes == 2) B[t] = ig_mfma(a, wb, B[t]);
+                }
+                if (more) W::template refill<S>(cur, wn, n, kh);
+            });
+#pragma unroll
+            for (int t = 0; t < TT; ++t) {
+                f32x16 mn = {};
+                if constexpr (ig_mins(T)) {
+                    const f16x8 bs = *(const f16x8*)(st + t * kTile + kIgBsum + kh * 512 + ln * 16);
+                    mn = __builtin_amdgcn_mfma_f32_32x32x16_f16(bs, mins, (f32x16){}, 0, 0, 0);
+                }
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const float4 da = *(const float4*)(st + t * kTile + kIgD + (8 * q + 4 * kh) * 4);
+                    const float dv[4] = {da.x, da.y, da.z, da.w};
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        const int i = 4 * q + k;
+                        if constexpr (T == kQ2_K)
+                            y[t][i] = y[t][i] + ig_q2_term(A[t][i], mn[i], dv[k], d, dmin);
+                        else
+                            y[t][i] = __builtin_fmaf(dv[k], ig_term<T>(A[t][i], B[t][i], mn[i], d, dmin), y[t][i]);
+                    }
+                }
+            }
+        };
+        for (uint32_t it = 0; it + 1 < run; ++it) {
+            if (it == 0) ig_barrier<0>();
+            else ig_barrier<W::kLoads>();
+            step(std::true_type{}, it);
+        }
+        if (run) {
+            ig_barrier<0>();
+            if (KS == 1 || (run - 1) * KS + kg < nchunk) step(std::false_type{}, run - 1);
+        }
     }
 
     if (mat == kIgZero) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // its first stage must land before LDS is reused
