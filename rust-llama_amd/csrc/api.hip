@@ -499,17 +499,45 @@ enum class Route { kDecode, kGemm, kIgemm };
 //
 // Up to 8 columns the decode kernels read the weights once, with no launch
 // before them.  The int8 GEMM's two launches are faster where those kernels
-// take several passes or lose their K split (us, decode against GEMM):
-//  - Q6_K two columns (two passes: 4096x14336 30.5 / 22.7, 1024x1024 10.2 / 7.9), and
-//    three or more of 2048 or more values (4096x4096 17.4 / 12.0, 14336x4096 20.8 /
-//    18.5; 1024x1024 7.3 / 7.9);
-//  - Q2_K and Q3_K from five columns (a second group of columns) of 2048 or more
-//    values (4096x4096 17.4 / 9.1 and 17.7 / 10.4; 1024x1024 7.2 / 7.4 and 7.5 / 7.8),
-//    Q3_K below the balanced deal's 6144 rows (14336x4096 14.1 / 15.8);
-//  - Q8_0 whose parked terms no longer fit LDS (4096x14336: three columns 29.6 /
-//    40, five 80 / 40; 4096x4096, eight columns 13.5 / 16.6).
-// Not with an argmax, which the decode kernels finish in the same launch, and
-// not for the output head's row counts, where they are near the memory rate.
+// take several passes, a second group of columns, or lose their K split (us,
+// decode against GEMM; rows x values a row, columns):
+//  - Q6_K to 16384 rows: two columns to 4096 rows (two passes; 1000x512 9.6 / 7.8)
+//    or from 4096 values (6000x4096 17.4 / 12.9, 16384x4096 19.0 / 18.4; 9000x2048
+//    10.4 / 11.4), more from 4096 values (16384x4096, 3: 19.2 / 18.4) or from 2048 in
+//    five columns or to 6144 rows (6000x2048, 3: 10.6 / 8.9; 12288x2048, 3: 11.8 /
+//    12.7, 5: 13.1 / 12.7); 22000x8192, 3: 37.5 / 42.6;
+//  - Q2_K and Q3_K: from five columns of 2048 values outside the balanced deal
+//    (10240 to 16384 rows; 2500x2048 10.8 / 7.9 and 10.9 / 8.5; 2500x1024 7.4 / 7.4 and
+//    7.5 / 7.7), Q3_K above it from 4096 (30000x2048 15.1 / 15.9, x4096 24.8 / 24.0);
+//    inside it Q2_K from 4096 (12288x4096, 5: 12.1 / 11.7), Q3_K eight columns from
+//    8192 (24.6 / 23.3; 5: 20.3 / 23.3); Q2_K three from 8192 above 4096 rows outside
+//    it (6000x8192 17.2 / 13.0; 2500x8192 11.2 / 11.4; 12288x8192 13.7 / 16.8);
+//  - Q8_0 whose parked terms no longer fit LDS (1000x14336, 3: 25.7 / 37.9, 5: 78 /
+//    39; 30000x8192, 8: 72 / 75, x14336, 5: 166 / 131), and of more tiles than CUs to
+//    16384 rows from 8192 values (9000x8192, 3: 41.9 / 37.1; 22000: 51 / 59) or eight
+//    columns from 4096 (6000x4096 26.9 / 17.2, 5: 12.8 / 17.0).
+// Not with an argmax, which the decode kernels finish in the same launch.
+bool few_columns_igemm(uint32_t dtype, uint64_t rows, uint64_t cols, uint64_t batch) {
+    const bool deal = rows >= 10240 && rows <= 16384;
+    const uint64_t blocks = batch * (cols / 32);
+    switch (dtype) {
+        case kQ6_K:
+            if (rows > 16384) return false;
+            if (batch == 2) return rows <= 4096 || cols >= 4096;
+            return cols >= 4096 || (cols >= 2048 && (batch >= 5 || rows <= 6144));
+        case kQ2_K:
+            if (batch < 5) return batch >= 3 && cols >= 8192 && rows > 4096 && !deal;
+            return cols >= (deal ? 4096 : 2048);
+        case kQ3_K:
+            if (deal) return batch == 8 && cols >= 8192;
+            return batch >= 5 && cols >= (rows > 16384 ? 4096 : 2048);
+        case kQ8_0:
+            if (blocks > (rows <= 24576 ? 1600 : 2100)) return true;
+            return rows > 4096 && rows <= 16384 && ((batch >= 3 && cols >= 8192) || (batch == 8 && cols >= 4096));
+        default: return false;
+    }
+}
+
 Route matmul_route(uint32_t dtype, uint64_t rows, uint64_t cols, uint64_t batch, bool argmax) {
     if (batch > kDecodeMaxBatch) {
         if (dtype != kQ4_K) return Route::kIgemm;
@@ -517,12 +545,7 @@ Route matmul_route(uint32_t dtype, uint64_t rows, uint64_t cols, uint64_t batch,
         const uint64_t rounds = (groups + cus - 1) / cus;
         return rows * ((batch + 63) / 64 * 64) < rounds * 5800000 ? Route::kIgemm : Route::kGemm;
     }
-    if (batch < 2 || argmax || rows > 32768) return Route::kDecode;
-    const bool igemm = dtype == kQ6_K   ? batch == 2 || cols >= 2048
-                       : dtype == kQ2_K ? batch >= 5 && cols >= 2048
-                       : dtype == kQ3_K ? batch >= 5 && cols >= 2048 && rows < 6144
-                       : dtype == kQ8_0 ? batch * (cols / 32) > 1600
-                                        : false;
+    const bool igemm = batch >= 2 && !argmax && rows <= 32768 && few_columns_igemm(dtype, rows, cols, batch);
     return igemm ? Route::kIgemm : Route::kDecode;
 }
 

@@ -34,13 +34,15 @@ def cases():
         for batch in (9, 17, 32):
             yield t, 95, 2304, batch
     # two to eight columns on the GEMM
-    yield DT.Q6_K, 100, 512, 2
-    for batch in (3, 8):
-        yield DT.Q6_K, 100, 2048, batch
+    for batch in (2, 3, 8):
+        yield DT.Q6_K, 100, 4096, batch
+    yield DT.Q6_K, 30, 512, 2
     for t in (DT.Q2_K, DT.Q3_K):
         yield t, 100, 2304, 5
         yield t, 17, 2048, 8
+    yield DT.Q2_K, 4100, 8192, 3
     yield DT.Q8_0, 40, 32 * 331, 5
+    yield DT.Q8_0, 4100, 4096, 8
 
 
 @pytest.mark.parametrize("t,rows,cols,batch", list(cases()), ids=lambda v: v.name if isinstance(v, DT) else str(v))
