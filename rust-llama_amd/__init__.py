@@ -318,13 +318,27 @@ def _dev_ptr(t, dtype):
         raise TypeError("expected a torch tensor on the GPU")
     if t.dtype != dtype or not t.is_contiguous():
         raise TypeError(f"expected a contiguous {dtype} tensor")
-    return ctypes.c_void_p(t.data_ptr())
+    return t.data_ptr()  # (the signatures' void pointers take an int)
+
+
+# torch's current stream as a handle.  torch.cuda.current_stream() makes a Stream
+# object for it, 2.9 us of a call whose kernels may take 4; torch's own code
+# generators read the handle as below.
+_raw_stream = getattr(getattr(torch, "_C", None), "_cuda_getCurrentRawStream", None)
+_raw_device = getattr(getattr(torch, "_C", None), "_cuda_getDevice", None)
 
 
 def _stream_ptr(stream):
     if stream is None:
-        return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
-    return ctypes.c_void_p(stream if isinstance(stream, int) else stream.cuda_stream)
+        if _raw_stream and _raw_device:
+            return _raw_stream(_raw_device())
+        return torch.cuda.current_stream().cuda_stream
+    return stream if isinstance(stream, int) else stream.cuda_stream
+
+
+def _columns(x, cols):
+    """x as [batch, cols]; as it is when it has that shape (a reshape costs 1 us)."""
+    return x if x.ndim == 2 and x.shape[1] == cols else x.reshape(-1, cols)
 
 
 class Context:
@@ -348,7 +362,7 @@ class Context:
 
     def matmul(self, w, x, y=None, stream=None):
         """MUL_MAT / Matrix::multiply: x [batch, cols] f32 -> y [batch, rows] f32."""
-        x2 = x.reshape(-1, w.cols)
+        x2 = _columns(x, w.cols)
         if y is None:
             y = torch.empty((x2.shape[0], w.rows), dtype=torch.float32, device=x.device)
         err = _Err()
@@ -369,7 +383,7 @@ class Context:
 
     def matmul_argmax(self, w, x, y=None, argmax=None, stream=None):
         """matmul followed by the greedy sampler's index per column."""
-        x2 = x.reshape(-1, w.cols)
+        x2 = _columns(x, w.cols)
         batch = x2.shape[0]
         if y is None:
             y = torch.empty((batch, w.rows), dtype=torch.float32, device=x.device)
@@ -388,7 +402,7 @@ class Context:
         arguments launches the same call again with only the C call's own
         cost (for serving loops; it raises like matmul).  The tensors stay
         referenced by the function."""
-        x2 = x.reshape(-1, w.cols)
+        x2 = _columns(x, w.cols)
         batch = x2.shape[0]
         if y.numel() != batch * w.rows:
             raise ValueError("y must hold batch * rows f32 values")
@@ -418,7 +432,7 @@ class Context:
         """rlq_matmul_noalloc: matmul (argmax None) or matmul_argmax into the
         caller's y [batch, rows] (and argmax [batch] int32), with the
         library's static device scratch instead of any allocation."""
-        x2 = x.reshape(-1, w.cols)
+        x2 = _columns(x, w.cols)
         err = _Err()
         _check(_lib.rlq_matmul_noalloc(self._h, w._h, _dev_ptr(x2, torch.float32), x2.shape[0],
                                        _dev_ptr(y, torch.float32),
@@ -476,7 +490,7 @@ class Context:
         """Exact per-(row, block) integer sums of w against column 0 of x
         ([batch, cols] or [cols], batch <= 8), from the kernel that matmul
         uses for that batch size."""
-        x2 = x.reshape(-1, w.cols)
+        x2 = _columns(x, w.cols)
         nb = w.cols // (32 if w.dtype == DType.Q8_0 else 256)
         isum = torch.empty((w.rows, nb), dtype=torch.int32, device=x.device)
         imin = torch.empty((w.rows, nb), dtype=torch.int32, device=x.device)
@@ -493,7 +507,7 @@ class Context:
         flags=SUMS_SILU_PAIR the decode step's gate/up kernel runs over w (Q4_K
         / Q5_K rows whose 16-row tiles alternate gate and up) and y holds
         silu(gate) * up, rows / 2 values; otherwise y is [batch, rows]."""
-        x2 = x.reshape(-1, w.cols)
+        x2 = _columns(x, w.cols)
         nb = w.cols // (32 if w.dtype == DType.Q8_0 else 256)
         isum = torch.empty((w.rows, nb), dtype=torch.int32, device=x.device)
         imin = torch.empty((w.rows, nb), dtype=torch.int32, device=x.device)
