@@ -273,9 +273,26 @@ template <bool MAD>
 __device__ __forceinline__ float fit_error(float difference) {
     return MAD ? fabsf(difference) : difference * difference;
 }
+// The levels of one grid: round((x - minimum) * inverse) clamped to 0..nmax, kept
+// as f32 (the reference's i32 levels only enter f32 expressions).  `nearest`
+// fails for a value past +-4194303; x -> inverse * (x - minimum) is monotonic, each
+// operation rounding monotonically, so the grid is checked at the smallest and
+// the largest x only (affine_in_range).
+__device__ __forceinline__ float affine_level(float x, float minimum, float inverse, float nmax) {
+    return __builtin_amdgcn_fmed3f(__builtin_rintf(inverse * (x - minimum)), 0.0f, nmax);
+}
+__device__ __forceinline__ bool affine_in_range(float lo, float hi, float minimum, float inverse) {
+    const float a = inverse * (lo - minimum), b = inverse * (hi - minimum);
+    return fabsf(a) <= 4194303.0f && fabsf(b) <= 4194303.0f;  // (false for a NaN)
+}
+
+// Bound: the VALU, sixteen operations per value and grid of 16 to 21.  4096x4096
+// Q4_K / Q5_K / Q2_K 166 / 134 / 148 us; with i32 levels, a range check per value
+// and the best grid's levels copied 223 / 180 / 164.  The best grid is remembered
+// instead, and its levels are formed by the caller that needs them.
 template <int N, bool MAD>
-__device__ bool make_affine2(const float (&x)[N], int32_t nmax, const float (&weights)[N], int32_t (&levels)[N],
-                             float rmin, float rdelta, int steps, float& scale_out, float& min_out) {
+__device__ bool make_affine2(const float (&x)[N], int32_t nmax, const float (&weights)[N], float rmin, float rdelta,
+                             int steps, float& scale_out, float& min_out, float& grid_min, float& grid_inverse) {
     float minimum = x[0], maximum = x[0];
     float sum_w = weights[0];
     float sum_x = sum_w * x[0];
@@ -287,43 +304,38 @@ __device__ bool make_affine2(const float (&x)[N], int32_t nmax, const float (&we
         sum_x += weights[i] * x[i];
     }
     if (!finite(sum_w) || !finite(sum_x)) return false;
+    const float lowest = minimum, top = (float)nmax;
     if (minimum > 0.0f) minimum = 0.0f;
+    grid_min = minimum;
+    grid_inverse = 0.0f;  // every level 0
     if (maximum == minimum) {
-#pragma unroll
-        for (int i = 0; i < N; ++i) levels[i] = 0;
         scale_out = 0.0f;
         min_out = -minimum;
         return true;
     }
-    float inverse = (float)nmax / (maximum - minimum);
+    float inverse = top / (maximum - minimum);
     float scale = 1.0f / inverse;
     float best_error = 0.0f;
-    bool ok = true;
+    if (!affine_in_range(lowest, maximum, minimum, inverse)) return false;
+    grid_inverse = inverse;
 #pragma unroll
     for (int i = 0; i < N; ++i) {
-        int32_t l = 0;
-        ok &= nearest(inverse * (x[i] - minimum), l);
-        levels[i] = clampi(l, 0, nmax);
-        const float difference = scale * (float)levels[i] + minimum - x[i];
+        const float difference = scale * affine_level(x[i], minimum, inverse, top) + minimum - x[i];
         best_error += weights[i] * fit_error<MAD>(difference);
     }
-    if (!ok) return false;
     for (int step = 0; step <= steps; ++step) {
-        inverse = (rmin + rdelta * (float)step + (float)nmax) / (maximum - minimum);
+        inverse = (rmin + rdelta * (float)step + top) / (maximum - minimum);
+        if (!affine_in_range(lowest, maximum, minimum, inverse)) return false;
         float sum_l = 0.0f, sum_l2 = 0.0f, sum_xl = 0.0f;
-        int32_t candidate[N];
+        float candidate[N];
 #pragma unroll
         for (int i = 0; i < N; ++i) {
-            int32_t l = 0;
-            ok &= nearest(inverse * (x[i] - minimum), l);
-            l = clampi(l, 0, nmax);
+            const float l = affine_level(x[i], minimum, inverse, top), wl = weights[i] * l;
             candidate[i] = l;
-            const float w = weights[i];
-            sum_l += w * (float)l;
-            sum_l2 += w * (float)l * (float)l;
-            sum_xl += w * (float)l * x[i];
+            sum_l += wl;
+            sum_l2 += wl * l;
+            sum_xl += wl * x[i];
         }
-        if (!ok) return false;
         const float determinant = sum_w * sum_l2 - sum_l * sum_l;
         if (determinant > 0.0f) {
             float candidate_scale = (sum_w * sum_xl - sum_x * sum_l) / determinant;
@@ -335,12 +347,11 @@ __device__ bool make_affine2(const float (&x)[N], int32_t nmax, const float (&we
             float error = 0.0f;
 #pragma unroll
             for (int i = 0; i < N; ++i) {
-                const float difference = candidate_scale * (float)candidate[i] + candidate_minimum - x[i];
+                const float difference = candidate_scale * candidate[i] + candidate_minimum - x[i];
                 error += weights[i] * fit_error<MAD>(difference);
             }
             if (error < best_error) {
-#pragma unroll
-                for (int i = 0; i < N; ++i) levels[i] = candidate[i];
+                grid_min = minimum, grid_inverse = inverse;
                 best_error = error;
                 scale = candidate_scale;
                 minimum = candidate_minimum;
@@ -351,6 +362,13 @@ __device__ bool make_affine2(const float (&x)[N], int32_t nmax, const float (&we
     scale_out = scale;
     min_out = -minimum;
     return true;
+}
+// The levels of make_affine2's best grid.
+template <int N>
+__device__ __forceinline__ void affine_levels(const float (&x)[N], int32_t nmax, float grid_min, float grid_inverse,
+                                              int32_t (&levels)[N]) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) levels[i] = (int32_t)affine_level(x[i], grid_min, grid_inverse, (float)nmax);
 }
 
 // Q4_K / Q5_K (encode_k.rs:430-507): 8 lanes per super-block (one 32-value
@@ -382,8 +400,10 @@ __global__ __launch_bounds__(64) void encode_q45k_kernel(const float* __restrict
 #pragma unroll
     for (int i = 0; i < 32; ++i) weights[i] = average + fabsf(xs[i]);
     int32_t levels[32];
-    float scale = 0.0f, minimum = 0.0f;
-    if (ok) ok &= make_affine2<32, false>(xs, kNmax, weights, levels, FIVE ? -0.5f : -1.0f, 0.1f, FIVE ? 15 : 20, scale, minimum);
+    float scale = 0.0f, minimum = 0.0f, grid_min = 0.0f, grid_inverse = 0.0f;
+    if (ok)
+        ok &= make_affine2<32, false>(xs, kNmax, weights, FIVE ? -0.5f : -1.0f, 0.1f, FIVE ? 15 : 20, scale, minimum,
+                                      grid_min, grid_inverse);
 
     // maximum_scale / maximum_minimum: strict `>` from +0.0 (encode_k.rs:454-459)
     float ms = scale > 0.0f ? scale : 0.0f, mm = minimum > 0.0f ? minimum : 0.0f;
@@ -438,6 +458,8 @@ __global__ __launch_bounds__(64) void encode_q45k_kernel(const float* __restrict
             ok &= nearest((xs[i] + minimum2) / scale2, l);
             levels[i] = clampi(l, 0, kNmax);
         }
+    } else {
+        affine_levels(xs, kNmax, grid_min, grid_inverse, levels);
     }
 #pragma unroll
     for (int i = 0; i < 32; ++i) lv[gb][sub * 32 + i] = (uint8_t)levels[i];
@@ -478,8 +500,15 @@ __global__ __launch_bounds__(64) void encode_q45k_kernel(const float* __restrict
     }
 }
 
-// make_qx with rmse = 1 and no importance weights, encode_k.rs:70-137.
-__device__ bool make_qx_rmse1(const float (&x)[16], int32_t nmax, int32_t (&levels)[16], float& scale_out) {
+// make_qx with rmse = 1 and no importance weights, encode_k.rs:70-137.  The grid
+// of the result is remembered (flat: all levels 0); qx_level gives its levels.
+// |inverse * x| is largest at the largest |x|, so `nearest`'s range is checked
+// there; a NaN shows in the sums.  Q6_K 4096x4096 94 us (122 with i32 levels, a
+// check per value and the best levels copied).
+__device__ __forceinline__ float qx_level(float x, float inverse, float nmax) {
+    return __builtin_amdgcn_fmed3f(__builtin_rintf(inverse * x), -nmax, nmax - 1.0f);
+}
+__device__ bool make_qx_rmse1(const float (&x)[16], int32_t nmax, float& scale_out, float& grid_inverse, bool& flat) {
     float maximum = 0.0f, magnitude = 0.0f;
 #pragma unroll
     for (int i = 0; i < 16; ++i)
@@ -487,48 +516,39 @@ __device__ bool make_qx_rmse1(const float (&x)[16], int32_t nmax, int32_t (&leve
             magnitude = fabsf(x[i]);
             maximum = x[i];
         }
-    if (magnitude < 1e-15f) {
-#pragma unroll
-        for (int i = 0; i < 16; ++i) levels[i] = 0;
+    flat = magnitude < 1e-15f;
+    grid_inverse = 0.0f;
+    if (flat) {
         scale_out = 0.0f;
         return true;
     }
-    bool ok = true;
-    float inverse = (float)(-nmax) / maximum;
+    const float top = (float)nmax;
+    float inverse = -top / maximum;
     float sum_lx = 0.0f, sum_l2 = 0.0f;
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-        int32_t l = 0;
-        ok &= nearest(inverse * x[i], l);
-        l = clampi(l, -nmax, nmax - 1);
-        levels[i] = l + nmax;
-        const float w = x[i] * x[i];
-        sum_lx += w * x[i] * (float)l;
-        sum_l2 += w * (float)l * (float)l;
+        const float l = qx_level(x[i], inverse, top), w = x[i] * x[i];
+        sum_lx += w * x[i] * l;
+        sum_l2 += w * l * l;
     }
-    if (!ok || !finite(sum_lx) || !finite(sum_l2)) return false;
+    if (!(fabsf(inverse * maximum) <= 4194303.0f) || !finite(sum_lx) || !finite(sum_l2)) return false;
+    grid_inverse = inverse;
     float scale = sum_l2 != 0.0f ? sum_lx / sum_l2 : 0.0f;
     float best = scale * sum_lx;
     for (int step = -9; step <= 9; ++step) {
         if (step == 0) continue;
-        inverse = -((float)nmax + 0.1f * (float)step) / maximum;
+        inverse = -(top + 0.1f * (float)step) / maximum;
         sum_lx = 0.0f;
         sum_l2 = 0.0f;
-        int32_t cand[16];
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
-            int32_t l = 0;
-            ok &= nearest(inverse * x[i], l);
-            l = clampi(l, -nmax, nmax - 1);
-            cand[i] = nmax + l;
-            const float w = x[i] * x[i];
-            sum_lx += w * x[i] * (float)l;
-            sum_l2 += w * (float)l * (float)l;
+            const float l = qx_level(x[i], inverse, top), w = x[i] * x[i];
+            sum_lx += w * x[i] * l;
+            sum_l2 += w * l * l;
         }
-        if (!ok || !finite(sum_lx) || !finite(sum_l2)) return false;
+        if (!(fabsf(inverse * maximum) <= 4194303.0f) || !finite(sum_lx) || !finite(sum_l2)) return false;
         if (sum_l2 > 0.0f && sum_lx * sum_lx > best * sum_l2) {
-#pragma unroll
-            for (int i = 0; i < 16; ++i) levels[i] = cand[i];
+            grid_inverse = inverse;
             scale = sum_lx / sum_l2;
             best = scale * sum_lx;
         }
@@ -553,7 +573,11 @@ __global__ __launch_bounds__(64) void encode_q6k_kernel(const float* __restrict_
     }
     int32_t levels[16];
     float scale = 0.0f;
-    bool ok = make_qx_rmse1(xs, 32, levels, scale);
+    float grid_inverse;
+    bool flat;
+    bool ok = make_qx_rmse1(xs, 32, scale, grid_inverse, flat);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) levels[i] = flat ? 0 : (int32_t)qx_level(xs[i], grid_inverse, 32.0f) + 32;
 
     // first sub-block of largest |scale| (strict `>` from 0, encode_k.rs:525-528)
     uint64_t key = fabsf(scale) > 0.0f ? (((uint64_t)__float_as_uint(fabsf(scale)) << 32) | (15u - sub)) : 0;
@@ -636,8 +660,8 @@ __global__ __launch_bounds__(64) void encode_q2k_kernel(const float* __restrict_
 #pragma unroll
     for (int i = 0; i < 16; ++i) weights[i] = fabsf(xs[i]);
     int32_t levels[16];
-    float scale = 0.0f, minimum = 0.0f;
-    bool ok = make_affine2<16, true>(xs, 3, weights, levels, -0.5f, 0.1f, 15, scale, minimum);
+    float scale = 0.0f, minimum = 0.0f, grid_min = 0.0f, grid_inverse = 0.0f;
+    bool ok = make_affine2<16, true>(xs, 3, weights, -0.5f, 0.1f, 15, scale, minimum, grid_min, grid_inverse);
 
     // maximum_scale / maximum_minimum: strict `>` from +0.0 (encode_k.rs:313-318)
     float ms = scale > 0.0f ? scale : 0.0f, mm = minimum > 0.0f ? minimum : 0.0f;
@@ -671,6 +695,8 @@ __global__ __launch_bounds__(64) void encode_q2k_kernel(const float* __restrict_
             ok &= nearest((xs[i] + minimum2) / scale2, l);
             levels[i] = clampi(l, 0, 3);
         }
+    } else {
+        affine_levels(xs, 3, grid_min, grid_inverse, levels);
     }
 #pragma unroll
     for (int i = 0; i < 16; ++i) lv[gb][sub * 16 + i] = (uint8_t)levels[i];
