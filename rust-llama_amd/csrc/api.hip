@@ -716,11 +716,7 @@ static int32_t gemm_launch(rlq_context* ctx, const rlq_weights* w, Route r, cons
     else
         HIP_TRY(launch_igemm(w->dtype, w->dev, w->rows, w->cols, x, false, IgStack{1, batch, 1, 1, 0}, y, w->rows, scratch,
                              ctx->err_words, s));
-    if (argmax) {
-        HIP_TRY(launch_fill_u64(keys, batch, 0ull, s));
-        HIP_TRY(launch_argmax_rows(y, batch, w->rows, keys, s));
-        HIP_TRY(launch_argmax_finish(keys, batch, y, w->rows, argmax, s));
-    }
+    if (argmax) HIP_TRY(launch_argmax(y, batch, w->rows, keys, argmax, s));
     return ok(err);
 }
 
@@ -817,10 +813,10 @@ int32_t rlq_matmul_noalloc(rlq_context* ctx, const rlq_weights* w, const float* 
     DeviceGuard g(ctx->device);
     const hipStream_t s = pick(ctx, stream);
     // the scratch keeps the last call's contents: what must start at 0 is cleared
-    if (argmax) HIP_TRY(launch_fill_u64((unsigned long long*)ctx->scratch, 1, 0ull, s));  // the arrival counter
     if (route != Route::kDecode)
         return gemm_launch(ctx, w, route, x, batch, y, ctx->scratch + state_bytes + keys_bytes,
                            (unsigned long long*)(ctx->scratch + state_bytes), argmax, s, err);
+    if (argmax) HIP_TRY(launch_fill_u64((unsigned long long*)ctx->scratch, 1, 0ull, s));  // the arrival counter
     const MvArgmax am = argmax_state(ctx->scratch, argmax);
     HIP_TRY(launch_matvec(w->dtype, w->dev, w->rows, w->cols, x, nullptr, batch, y, w->rows, argmax ? &am : nullptr,
                           ctx->err_words, nullptr, nullptr, s));

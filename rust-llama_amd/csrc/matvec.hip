@@ -3498,6 +3498,50 @@ __global__ __launch_bounds__(256) void argmax_rows_kernel(const float* __restric
     if ((threadIdx.x & 63) == 0 && best) atomicMax(keys + b, best);
 }
 
+// The whole greedy argmax of stored rows of up to kArgmaxOneGroup values, one
+// workgroup per column.  Bound: one workgroup's read of a row.  In place of the
+// fill, fold and finish of the keys' path, whose workgroups meet in one atomic
+// per column (Q4_K with the product: 11268x768, 19 columns 36 -> 15 us; 32000x2048,
+// 32 columns 69 -> 23; 128256x4096, 16 columns 104 -> 87; 200000x512, 10 columns 52
+// against 53, 262144x256 48 against 58).
+__global__ __launch_bounds__(1024) void argmax_columns_kernel(const float* __restrict__ y, uint32_t rows,
+                                                              uint32_t* __restrict__ out) {
+    __shared__ unsigned long long best_s;
+    if (threadIdx.x == 0) best_s = 0ull;
+    __syncthreads();
+    const float* c = y + (uint64_t)blockIdx.x * rows;
+    unsigned long long best = 0;
+    for (uint32_t r0 = threadIdx.x; r0 < rows; r0 += 8 * 1024) {
+        float v[8];
+#pragma unroll
+        for (uint32_t k = 0; k < 8; ++k) v[k] = r0 + k * 1024 < rows ? c[r0 + k * 1024] : 0.0f;
+#pragma unroll
+        for (uint32_t k = 0; k < 8; ++k) {
+            const unsigned long long key = r0 + k * 1024 < rows ? argmax_key(v[k], r0 + k * 1024) : 0ull;
+            best = key > best ? key : best;
+        }
+    }
+#pragma unroll
+    for (int m = 1; m < 64; m <<= 1) {
+        const unsigned long long o = __shfl_xor(best, m, 64);
+        best = o > best ? o : best;
+    }
+    if ((threadIdx.x & 63) == 0 && best) atomicMax(&best_s, best);
+    __syncthreads();
+    if (threadIdx.x == 0) out[blockIdx.x] = best_s == 0 ? 0u : (uint32_t)(0xffffffffull - (best_s & 0xffffffffull));
+}
+
+hipError_t launch_argmax(const float* y, uint64_t batch, uint64_t rows, unsigned long long* keys, uint32_t* out,
+                         hipStream_t s) {
+    if (rows <= kArgmaxOneGroup) {
+        hipLaunchKernelGGL(argmax_columns_kernel, dim3((unsigned)batch), dim3(1024), 0, s, y, (uint32_t)rows, out);
+        return hipGetLastError();
+    }
+    hipError_t e = launch_fill_u64(keys, batch, 0ull, s);
+    if (e == hipSuccess) e = launch_argmax_rows(y, batch, rows, keys, s);
+    return e == hipSuccess ? launch_argmax_finish(keys, batch, y, rows, out, s) : e;
+}
+
 hipError_t launch_argmax_rows(const float* y, uint64_t batch, uint64_t rows, unsigned long long* keys, hipStream_t s) {
     const uint64_t per = (rows + 255) / 256;
     hipLaunchKernelGGL(argmax_rows_kernel, dim3((unsigned)(per < 64 ? per : 64), (unsigned)batch), dim3(256), 0, s, y,

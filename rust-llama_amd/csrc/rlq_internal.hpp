@@ -240,6 +240,11 @@ struct LlamaModel {
                     unsigned long long* err_word, hipStream_t s);
 };
 
+// The greedy argmax of the stored rows y[b*rows ..], through `keys` (batch) for
+// long rows.
+constexpr uint64_t kArgmaxOneGroup = 160000;
+hipError_t launch_argmax(const float* y, uint64_t batch, uint64_t rows, unsigned long long* keys, uint32_t* out,
+                         hipStream_t s);
 // Argmax keys of the stored rows y[b*rows ..] (keys zeroed beforehand).
 hipError_t launch_argmax_rows(const float* y, uint64_t batch, uint64_t rows, unsigned long long* keys, hipStream_t s);
 // Decode argmax keys into u32 indices; reset: then set the keys back to 0.

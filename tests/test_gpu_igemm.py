@@ -84,6 +84,29 @@ def test_many_columns(t, rows, cols, batch):
         ctx.close()
 
 
+@pytest.mark.parametrize("rows", [1, 63, 1025, 8192, 8200, 160000, 160016])
+def test_argmax_of_many_columns(rows):
+    """The first of equal maxima: every row occurs twice, and a zero column ties
+    everywhere.  The lengths sit at the argmax kernel's strides and its limit."""
+    say("argmax", rows)
+    w = _weights(DT.Q4_K, (rows + 1) // 2, 256, rows).reshape(-1, 144)
+    w = np.concatenate([w, w])[:rows].reshape(-1)
+    x = np.random.default_rng(rows).standard_normal((10, 256)).astype(np.float32)
+    x[4] = 0.0
+    ctx = rlq.Context(0)
+    try:
+        W = rlq.Weights(ctx, DT.Q4_K, w, rows, 256)
+        y, best = ctx.matmul_argmax(W, torch.from_numpy(x).cuda())
+        z, same = torch.empty_like(y), torch.empty_like(best)
+        ctx.matmul_noalloc(W, torch.from_numpy(x).cuda(), z, same)
+        ctx.sync()
+        assert np.array_equal(best.cpu().numpy(), y.cpu().numpy().argmax(axis=1))
+        assert torch.equal(best, same) and torch.equal(y, z)
+        W.close()
+    finally:
+        ctx.close()
+
+
 # ---- several matrices -------------------------------------------------------------
 
 def check(t, y, want):
