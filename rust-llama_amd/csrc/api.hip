@@ -744,17 +744,24 @@ static int32_t matmul_impl(rlq_context* ctx, const rlq_weights* w, const float* 
     // scratch may be replaced by a later, larger call: what needs no scratch
     // (every type but Q4_K) is recorded as decode passes.
     if (route == Route::kIgemm && w->dtype != kQ4_K && capturing(s)) route = Route::kDecode;
+    if (route != Route::kDecode) {
+        const hipError_t e = ensure(ctx, ctx->planes, route_bytes(route, w->dtype, batch, w->cols));
+        if (e == hipErrorOutOfMemory && w->dtype != kQ4_K) {  // decode passes need no image
+            (void)hipGetLastError();
+            route = Route::kDecode;
+        } else {
+            HIP_TRY(e);
+        }
+    }
     if (argmax) {
         bool grown = false;
         HIP_TRY(ensure(ctx, ctx->keys,
                        kArgmaxStateBytes + (route != Route::kDecode ? batch * sizeof(unsigned long long) : 0), &grown));
         if (grown) HIP_TRY(launch_fill_u64((unsigned long long*)ctx->keys.p, 1, 0ull, s));  // the arrival counter
     }
-    if (route != Route::kDecode) {
-        HIP_TRY(ensure(ctx, ctx->planes, route_bytes(route, w->dtype, batch, w->cols)));
+    if (route != Route::kDecode)
         return gemm_launch(ctx, w, route, x, batch, y, ctx->planes.p,
                            (unsigned long long*)((uint8_t*)ctx->keys.p + kArgmaxStateBytes), argmax, s, err);
-    }
     // decode: the argmax is finished inside each launch
     const MvArgmax am = argmax_state(ctx->keys.p, argmax);
     HIP_TRY(decode_launch(ctx, w, x, batch, y, argmax ? &am : nullptr, nullptr, nullptr, MvExtra{}, s));

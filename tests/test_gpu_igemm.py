@@ -84,6 +84,32 @@ def test_many_columns(t, rows, cols, batch):
         ctx.close()
 
 
+def test_flags_of_very_many_columns():
+    """Past 8192 flags one launch folds them: slices of the result equal the
+    slices' own products bit for bit, and the last column's error still
+    suppresses every output."""
+    say("igemm, 262176 columns")
+    rows, cols, batch = 17, 256, 262176
+    ctx = rlq.Context(0)
+    try:
+        W = rlq.Weights(ctx, DT.Q2_K, _weights(DT.Q2_K, rows, cols, 5), rows, cols)
+        x = torch.randn((batch, cols), generator=torch.Generator(device="cuda").manual_seed(6), device="cuda")
+        y = ctx.matmul(W, x)
+        for i in (0, 131072, batch - 40):
+            assert torch.equal(y[i:i + 40], ctx.matmul(W, x[i:i + 40]))
+        ctx.sync()
+        x[-1, -1] = float("nan")
+        y.fill_(7.0)
+        ctx.matmul(W, x, y)
+        with pytest.raises(rlq.QuantError) as e:
+            ctx.sync()
+        assert (e.value.name, e.value.index, e.value.b) == ("NonFiniteInput", 255, batch - 1)
+        assert bool((y == 7.0).all())
+        W.close()
+    finally:
+        ctx.close()
+
+
 @pytest.mark.parametrize("rows", [1, 63, 1025, 8192, 8200, 160000, 160016])
 def test_argmax_of_many_columns(rows):
     """The first of equal maxima: every row occurs twice, and a zero column ties
