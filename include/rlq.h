@@ -194,7 +194,7 @@ void rlq_weights_stack(const rlq_weights *w, uint64_t *n2, uint64_t *n3);
  * the weights; more (and, of some types and shapes, two to eight) run a GEMM
  * over an image of the quantized columns in the context's scratch (while
  * `stream` is being captured, types other than Q4_K run passes of 8 columns,
- * which need none).  A call takes at most 8388606 columns (the error keys carry
+ * which need none, Q5_K its planes).  A call takes at most 8388606 columns (the error keys carry
  * the column): more return RLQ_UNIMPLEMENTED (a = batch, b = the limit), as
  * do rlq_matmul_argmax, rlq_matmul_noalloc and rlq_quantize_device. */
 int32_t rlq_matmul(rlq_context *ctx, const rlq_weights *w, const float *x, uint64_t batch, float *y,

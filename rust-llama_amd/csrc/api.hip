@@ -741,8 +741,8 @@ static int32_t matmul_impl(rlq_context* ctx, const rlq_weights* w, const float* 
     const hipStream_t s = pick(ctx, stream);
     Route route = matmul_route(w->dtype, w->rows, w->cols, batch, argmax != nullptr);
     // A graph keeps the addresses it was captured with, and the context's
-    // scratch may be replaced by a later, larger call: what needs no scratch
-    // (every type but Q4_K) is recorded as decode passes.
+    // scratch may be replaced by a later, larger call: types other than Q4_K are
+    // recorded as decode passes, which need none (Q5_K: its columns' planes).
     if (route == Route::kIgemm && w->dtype != kQ4_K && capturing(s)) route = Route::kDecode;
     if (route != Route::kDecode) {
         const hipError_t e = ensure(ctx, ctx->planes, route_bytes(route, w->dtype, batch, w->cols));
