@@ -192,11 +192,15 @@ void rlq_weights_stack(const rlq_weights *w, uint64_t *n2, uint64_t *n3);
  * y[b*rows + r] = dot_packed(weights row r, activation b).  x and y are
  * device pointers (x 16-byte aligned).  Up to 8 columns share one pass over
  * the weights; more (and, of some types and shapes, two to eight) run a GEMM
- * over an image of the quantized columns in the context's scratch (while
+ * over an image of the quantized columns in the context's scratch.  While
  * `stream` is being captured, types other than Q4_K run passes of 8 columns,
- * which need none, Q5_K its planes).  A call takes at most 8388606 columns (the error keys carry
- * the column): more return RLQ_UNIMPLEMENTED (a = batch, b = the limit), as
- * do rlq_matmul_argmax, rlq_matmul_noalloc and rlq_quantize_device. */
+ * which need no image (Q5_K its planes).  What a captured call needs of the
+ * scratch must be there: the same call made once before the capture sees to
+ * it.  Later calls may grow the scratch; a graph's own part of it stays until
+ * the context is destroyed.  A call takes at most 8388606 columns (the error
+ * keys carry the column): more return RLQ_UNIMPLEMENTED (a = batch, b = the
+ * limit), as do rlq_matmul_argmax, rlq_matmul_noalloc and
+ * rlq_quantize_device. */
 int32_t rlq_matmul(rlq_context *ctx, const rlq_weights *w, const float *x, uint64_t batch, float *y,
                    void *stream, rlq_error *err);
 

@@ -88,6 +88,11 @@ constexpr uint64_t kDecodeMaxBatch = 8;
 struct DevBuf {
     void* p = nullptr;
     size_t n = 0;
+    bool recorded = false;  // a stream capture has recorded p
+};
+struct Retired {  // a replaced buffer that a captured graph may still use
+    void* p;
+    Retired* next;
 };
 
 }  // namespace
@@ -102,6 +107,7 @@ struct rlq_context {
     // set to 0 when the buffer is made, and left at 0 by every launch), then
     // the prefill path's per-column keys
     DevBuf planes, keys, stage_in, stage_w, stage_out, gate;
+    Retired* retired = nullptr;
 };
 
 struct rlq_weights {
@@ -116,25 +122,44 @@ struct rlq_weights {
 
 namespace {
 
-// Grow-only scratch.  Growing waits for the whole device first (callers may
-// pass their own streams), so no kernel still reads the old buffer when it is
-// freed.  *grown (may be null) tells whether the buffer was replaced: its
-// contents are then undefined, even when the allocator hands back the old
-// address.
-hipError_t ensure(rlq_context* ctx, DevBuf& b, size_t need, bool* grown = nullptr) {
-    (void)ctx;
+// Whether the stream records a graph (or HIP will not say).
+bool capturing(hipStream_t s) {
+    if (!s) return false;  // the null stream cannot be captured
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &st) != hipSuccess) {
+        (void)hipGetLastError();
+        return true;
+    }
+    return st != hipStreamCaptureStatusNone;
+}
+
+// Grow-only scratch for work on stream s.  Growing waits for the whole device
+// first (callers may pass their own streams), so no kernel still reads the old
+// buffer when it is freed.  A graph keeps the addresses it was captured with and
+// may be replayed at any time: a buffer that a capture has recorded is kept
+// until the context ends.  *grown (may be null) tells whether the buffer was
+// replaced: its contents are then undefined, even when the allocator hands back
+// the old address.
+hipError_t ensure(rlq_context* ctx, DevBuf& b, size_t need, hipStream_t s, bool* grown = nullptr) {
     if (grown) *grown = false;
-    if (b.n >= need) return hipSuccess;
+    if (b.n >= need) {
+        b.recorded = b.recorded || capturing(s);
+        return hipSuccess;
+    }
     if (grown) *grown = true;
     hipError_t e = hipDeviceSynchronize();
     if (e != hipSuccess) return e;
-    if (b.p) (void)hipFree(b.p);
-    b.p = nullptr;
-    b.n = 0;
+    if (b.p && b.recorded) {  // (without memory for the note it is never freed)
+        if (Retired* r = new (std::nothrow) Retired{b.p, ctx->retired}) ctx->retired = r;
+    } else if (b.p) {
+        (void)hipFree(b.p);
+    }
+    b = DevBuf{};
     size_t n = need < 4096 ? 4096 : need;
     e = hipMalloc(&b.p, n);
     if (e != hipSuccess) return e;
     b.n = n;
+    b.recorded = capturing(s);
     return hipSuccess;
 }
 
@@ -367,6 +392,11 @@ void rlq_context_destroy(rlq_context* ctx) {
     if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
     for (DevBuf* b : {&ctx->planes, &ctx->keys, &ctx->stage_in, &ctx->stage_w, &ctx->stage_out, &ctx->gate})
         if (b->p) (void)hipFree(b->p);
+    while (Retired* r = ctx->retired) {
+        ctx->retired = r->next;
+        (void)hipFree(r->p);
+        delete r;
+    }
     if (ctx->err_words) (void)hipFree(ctx->err_words);
     if (ctx->host_err) (void)hipHostFree(ctx->host_err);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
@@ -447,8 +477,8 @@ int32_t mm_stage(rlq_context* ctx, const rlq_weights* w, uint32_t at, uint32_t x
                  uint64_t columns, const int32_t* ids, uint64_t pairs, float* y, hipStream_t s, ActPlanes* planes,
                  uint32_t** gate, rlq_error* err) {
     const uint64_t K = w->cols, nb = K / block_size(at);
-    HIP_TRY(ensure(ctx, ctx->planes, act_planes_bytes(at, K, columns)));
-    HIP_TRY(ensure(ctx, ctx->gate, sizeof(uint32_t)));
+    HIP_TRY(ensure(ctx, ctx->planes, act_planes_bytes(at, K, columns), s));
+    HIP_TRY(ensure(ctx, ctx->gate, sizeof(uint32_t), s));
     *planes = act_planes_carve(ctx->planes.p, at, K, columns);
     *gate = (uint32_t*)ctx->gate.p;
     if (x_dtype == 0) {
@@ -473,7 +503,7 @@ constexpr uint64_t kPlanesMinBatch = 7;
 hipError_t decode_launch(rlq_context* ctx, const rlq_weights* w, const float* x, uint64_t batch, float* y,
                          const MvArgmax* am, int32_t* isum, int32_t* imin, const MvExtra& ex, hipStream_t s) {
     if ((w->dtype == kQ4_K || w->dtype == kQ5_K) && batch >= kPlanesMinBatch && ex.epilogue == 0) {
-        hipError_t e = ensure(ctx, ctx->planes, act_planes_bytes(kQ8_K, w->cols, batch));
+        hipError_t e = ensure(ctx, ctx->planes, act_planes_bytes(kQ8_K, w->cols, batch), s);
         if (e != hipSuccess) return e;
         const ActPlanes pl = act_planes_carve(ctx->planes.p, kQ8_K, w->cols, batch);
         e = launch_quantize_q8k(x, w->cols, batch, &pl, nullptr, ctx->err_words, s);
@@ -607,7 +637,7 @@ int32_t rlq_mul_mat(rlq_context* ctx, const rlq_weights* w, uint32_t x_dtype, co
     // 103).  Single columns keep the decode kernels, whose sums are in the
     // reference's order.
     if (mm_igemm_takes(w->dtype, x_dtype, x) && ncols > 1) {
-        HIP_TRY(ensure(ctx, ctx->planes, igemm_bytes(w->dtype, st.groups, st.cpg, w->cols)));
+        HIP_TRY(ensure(ctx, ctx->planes, igemm_bytes(w->dtype, st.groups, st.cpg, w->cols), s));
         HIP_TRY(launch_igemm(w->dtype, w->dev, w->rows, w->cols, x, x_dtype != 0, st, y, w->rows, ctx->planes.p,
                              ctx->err_words, s));
         return ok(err);
@@ -681,7 +711,7 @@ int32_t rlq_mul_mat_id(rlq_context* ctx, const rlq_weights* w, uint32_t x_dtype,
     const uint64_t again = (pairs - (pairs < w->n2 ? pairs : w->n2)) * w->mat_bytes;
     if (again >= (80ull << 20) && w->n2 <= kIgMaxMats && pairs <= 0x7fffffull && mm_igemm_takes(w->dtype, x_dtype, x)) {
         const IgRoute r{ids, (uint32_t)pairs, (uint32_t)w->n2, (uint32_t)columns, (uint32_t)slots, (uint32_t)ncols};
-        HIP_TRY(ensure(ctx, ctx->planes, igemm_ids_bytes(w->dtype, w->cols, r)));
+        HIP_TRY(ensure(ctx, ctx->planes, igemm_ids_bytes(w->dtype, w->cols, r), s));
         HIP_TRY(launch_igemm_ids(w->dtype, w->dev, w->rows, w->cols, w->mat_bytes, x, x_dtype != 0, r, y, w->rows,
                                  ctx->planes.p, ctx->err_words, s));
         return ok(err);
@@ -720,17 +750,6 @@ static int32_t gemm_launch(rlq_context* ctx, const rlq_weights* w, Route r, cons
     return ok(err);
 }
 
-// Whether the stream records a graph (or HIP will not say).
-static bool capturing(hipStream_t s) {
-    if (!s) return false;  // the null stream cannot be captured
-    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(s, &st) != hipSuccess) {
-        (void)hipGetLastError();
-        return true;
-    }
-    return st != hipStreamCaptureStatusNone;
-}
-
 static int32_t matmul_impl(rlq_context* ctx, const rlq_weights* w, const float* x, uint64_t batch, float* y,
                            uint32_t* argmax, void* stream, rlq_error* err) {
     if (!ctx || !w || !x || !y) return fail(err, RLQ_INVALID_ARGUMENT);
@@ -745,7 +764,7 @@ static int32_t matmul_impl(rlq_context* ctx, const rlq_weights* w, const float* 
     // recorded as decode passes, which need none (Q5_K: its columns' planes).
     if (route == Route::kIgemm && w->dtype != kQ4_K && capturing(s)) route = Route::kDecode;
     if (route != Route::kDecode) {
-        const hipError_t e = ensure(ctx, ctx->planes, route_bytes(route, w->dtype, batch, w->cols));
+        const hipError_t e = ensure(ctx, ctx->planes, route_bytes(route, w->dtype, batch, w->cols), s);
         if (e == hipErrorOutOfMemory && w->dtype != kQ4_K) {  // decode passes need no image
             (void)hipGetLastError();
             route = Route::kDecode;
@@ -756,7 +775,7 @@ static int32_t matmul_impl(rlq_context* ctx, const rlq_weights* w, const float* 
     if (argmax) {
         bool grown = false;
         HIP_TRY(ensure(ctx, ctx->keys,
-                       kArgmaxStateBytes + (route != Route::kDecode ? batch * sizeof(unsigned long long) : 0), &grown));
+                       kArgmaxStateBytes + (route != Route::kDecode ? batch * sizeof(unsigned long long) : 0), s, &grown));
         if (grown) HIP_TRY(launch_fill_u64((unsigned long long*)ctx->keys.p, 1, 0ull, s));  // the arrival counter
     }
     if (route != Route::kDecode)
@@ -1272,11 +1291,11 @@ int32_t rlq_block_sums_ex(rlq_context* ctx, const rlq_weights* w, const float* x
     DeviceGuard g(ctx->device);
     const hipStream_t s = pick(ctx, stream);
     if (!y) {
-        HIP_TRY(ensure(ctx, ctx->stage_out, batch * w->rows * sizeof(float)));
+        HIP_TRY(ensure(ctx, ctx->stage_out, batch * w->rows * sizeof(float), s));
         y = (float*)ctx->stage_out.p;
     }
     if (w->dtype == kQ4_K && batch > kDecodeMaxBatch) {
-        HIP_TRY(ensure(ctx, ctx->planes, gemm_planes_bytes(batch, w->cols)));
+        HIP_TRY(ensure(ctx, ctx->planes, gemm_planes_bytes(batch, w->cols), s));
         HIP_TRY(launch_gemm_q4k(w->dev, w->rows, w->cols, x, batch, y, w->rows, ctx->planes.p, ctx->err_words, isum,
                                 imin, s));
     } else {
@@ -1312,8 +1331,8 @@ int32_t rlq_quantize_into(uint32_t dtype, const float* values, uint64_t n, uint8
     if (rc) return rc;
     DeviceGuard g(ctx->device);
     const hipStream_t s = ctx->stream;
-    HIP_TRY(ensure(ctx, ctx->stage_in, n * sizeof(float)));
-    HIP_TRY(ensure(ctx, ctx->stage_out, out_len));
+    HIP_TRY(ensure(ctx, ctx->stage_in, n * sizeof(float), s));
+    HIP_TRY(ensure(ctx, ctx->stage_out, out_len, s));
     float* xd = (float*)ctx->stage_in.p;
     uint8_t* od = (uint8_t*)ctx->stage_out.p;
     unsigned long long* ew = ctx->err_words + 1;
@@ -1348,8 +1367,8 @@ int32_t rlq_dequantize_into(uint32_t dtype, const uint8_t* bytes, uint64_t len, 
     if (rc) return rc;
     DeviceGuard g(ctx->device);
     const hipStream_t s = ctx->stream;
-    HIP_TRY(ensure(ctx, ctx->stage_w, len));
-    HIP_TRY(ensure(ctx, ctx->stage_out, n * sizeof(float)));
+    HIP_TRY(ensure(ctx, ctx->stage_w, len, s));
+    HIP_TRY(ensure(ctx, ctx->stage_out, n * sizeof(float), s));
     HIP_TRY(hipMemcpyAsync(ctx->stage_w.p, bytes, len, hipMemcpyHostToDevice, s));
     HIP_TRY(launch_dequantize(dtype, (const uint8_t*)ctx->stage_w.p, n, (float*)ctx->stage_out.p, s));
     HIP_TRY(hipMemcpyAsync(out, ctx->stage_out.p, n * sizeof(float), hipMemcpyDeviceToHost, s));
@@ -1384,9 +1403,9 @@ int32_t rlq_dot_packed(uint32_t wtype, const uint8_t* weights, uint64_t weights_
     uint8_t* wd = nullptr;
     hipError_t e = upload_weights(wtype, weights, weights_len, 1, elements, false, &wd, s);
     if (e != hipSuccess) return hip_fail(err, e);
-    e = ensure(ctx, ctx->stage_in, activation_len);
-    if (e == hipSuccess) e = ensure(ctx, ctx->planes, act_planes_bytes(at, elements, 1));
-    if (e == hipSuccess) e = ensure(ctx, ctx->stage_out, sizeof(float));
+    e = ensure(ctx, ctx->stage_in, activation_len, s);
+    if (e == hipSuccess) e = ensure(ctx, ctx->planes, act_planes_bytes(at, elements, 1), s);
+    if (e == hipSuccess) e = ensure(ctx, ctx->stage_out, sizeof(float), s);
     ActPlanes planes{};
     if (e == hipSuccess) {
         planes = act_planes_carve(ctx->planes.p, at, elements, 1);
@@ -1426,8 +1445,8 @@ int32_t rlq_matvec(uint32_t wtype, const uint8_t* weights, uint64_t weights_len,
     uint8_t* wd = nullptr;
     hipError_t e = upload_weights(wtype, weights, weights_len, rows, cols, false, &wd, s);
     if (e != hipSuccess) return e == hipErrorOutOfMemory ? fail(err, RLQ_ALLOCATION_FAILED, wtype) : hip_fail(err, e);
-    e = ensure(ctx, ctx->stage_in, cols * sizeof(float));
-    if (e == hipSuccess) e = ensure(ctx, ctx->stage_out, rows * sizeof(float));
+    e = ensure(ctx, ctx->stage_in, cols * sizeof(float), s);
+    if (e == hipSuccess) e = ensure(ctx, ctx->stage_out, rows * sizeof(float), s);
     if (e == hipSuccess) e = hipMemcpyAsync(ctx->stage_in.p, input, cols * sizeof(float), hipMemcpyHostToDevice, s);
     if (e == hipSuccess)
         e = launch_matvec(wtype, wd, rows, cols, (const float*)ctx->stage_in.p, nullptr, 1, (float*)ctx->stage_out.p,
