@@ -103,10 +103,10 @@ struct rlq_context {
     hipStream_t stream = nullptr;
     unsigned long long* err_words = nullptr;  // [0] device API (sticky), [1] host API (per call)
     unsigned long long* host_err = nullptr;   // pinned readback
-    // keys: the decode launches' argmax state (kArgmaxStateBytes; its counter
-    // set to 0 when the buffer is made, and left at 0 by every launch), then
-    // the prefill path's per-column keys
-    DevBuf planes, keys, stage_in, stage_w, stage_out, gate;
+    // keys: the decode launches' argmax state (kArgmaxStateBytes, so never
+    // replaced; its counter set to 0 when the buffer is made, and left at 0 by
+    // every launch); column_keys: one per column, the argmax of long rows after a GEMM
+    DevBuf planes, keys, column_keys, stage_in, stage_w, stage_out, gate;
     Retired* retired = nullptr;
 };
 
@@ -390,7 +390,7 @@ void rlq_context_destroy(rlq_context* ctx) {
     if (!ctx) return;
     DeviceGuard g(ctx->device);
     if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
-    for (DevBuf* b : {&ctx->planes, &ctx->keys, &ctx->stage_in, &ctx->stage_w, &ctx->stage_out, &ctx->gate})
+    for (DevBuf* b : {&ctx->planes, &ctx->keys, &ctx->column_keys, &ctx->stage_in, &ctx->stage_w, &ctx->stage_out, &ctx->gate})
         if (b->p) (void)hipFree(b->p);
     while (Retired* r = ctx->retired) {
         ctx->retired = r->next;
@@ -737,7 +737,8 @@ static size_t route_bytes(Route r, uint32_t dtype, uint64_t batch, uint64_t cols
 }
 
 // The GEMM of a route other than kDecode over `scratch` (route_bytes), then the
-// argmax over the stored rows (keys: one u64 per column, or null).
+// argmax over the stored rows (keys: one u64 per column, for more than
+// kArgmaxOneGroup rows).
 static int32_t gemm_launch(rlq_context* ctx, const rlq_weights* w, Route r, const float* x, uint64_t batch, float* y,
                            void* scratch, unsigned long long* keys, uint32_t* argmax, hipStream_t s, rlq_error* err) {
     if (r == Route::kGemm)
@@ -759,9 +760,8 @@ static int32_t matmul_impl(rlq_context* ctx, const rlq_weights* w, const float* 
     DeviceGuard g(ctx->device);
     const hipStream_t s = pick(ctx, stream);
     Route route = matmul_route(w->dtype, w->rows, w->cols, batch, argmax != nullptr);
-    // A graph keeps the addresses it was captured with, and the context's
-    // scratch may be replaced by a later, larger call: types other than Q4_K are
-    // recorded as decode passes, which need none (Q5_K: its columns' planes).
+    // A capture cannot allocate: types other than Q4_K are recorded as decode
+    // passes, which need no image (Q5_K: its columns' planes).
     if (route == Route::kIgemm && w->dtype != kQ4_K && capturing(s)) route = Route::kDecode;
     if (route != Route::kDecode) {
         const hipError_t e = ensure(ctx, ctx->planes, route_bytes(route, w->dtype, batch, w->cols), s);
@@ -772,15 +772,16 @@ static int32_t matmul_impl(rlq_context* ctx, const rlq_weights* w, const float* 
             HIP_TRY(e);
         }
     }
-    if (argmax) {
+    if (argmax) {  // (for a GEMM too: a capture of the same call runs decode passes)
         bool grown = false;
-        HIP_TRY(ensure(ctx, ctx->keys,
-                       kArgmaxStateBytes + (route != Route::kDecode ? batch * sizeof(unsigned long long) : 0), s, &grown));
+        HIP_TRY(ensure(ctx, ctx->keys, kArgmaxStateBytes, s, &grown));
         if (grown) HIP_TRY(launch_fill_u64((unsigned long long*)ctx->keys.p, 1, 0ull, s));  // the arrival counter
+        if (route != Route::kDecode && w->rows > kArgmaxOneGroup)
+            HIP_TRY(ensure(ctx, ctx->column_keys, batch * sizeof(unsigned long long), s));
     }
     if (route != Route::kDecode)
-        return gemm_launch(ctx, w, route, x, batch, y, ctx->planes.p,
-                           (unsigned long long*)((uint8_t*)ctx->keys.p + kArgmaxStateBytes), argmax, s, err);
+        return gemm_launch(ctx, w, route, x, batch, y, ctx->planes.p, (unsigned long long*)ctx->column_keys.p, argmax, s,
+                           err);
     // decode: the argmax is finished inside each launch
     const MvArgmax am = argmax_state(ctx->keys.p, argmax);
     HIP_TRY(decode_launch(ctx, w, x, batch, y, argmax ? &am : nullptr, nullptr, nullptr, MvExtra{}, s));

@@ -110,3 +110,44 @@ def test_many_columns_need_no_scratch(t):
         W.close()
     finally:
         ctx.close()
+
+
+@pytest.mark.parametrize("t,rows,eager", [(DT.Q6_K, 3000, (16, 4000, 100000)), (DT.Q4_K, 160016, (10, 300, 700))],
+                         ids=["Q6_K", "Q4_K"])
+def test_recorded_argmax_outlives_larger_calls(t, rows, eager):
+    """Captured output heads of one column and of nine, replayed between argmax
+    calls of ever more columns (past 160000 rows Q4_K's use one key a column)."""
+    say("captured argmax", t.name, rows)
+    cols = 256
+    ctx = rlq.Context(0)
+    try:
+        W = rlq.Weights(ctx, t, _weights(t, rows, cols, 4), rows, cols)
+        xs = [normal(5, 1, cols), normal(6, 9, cols)]
+        ys = [torch.zeros((len(x), rows), device="cuda") for x in xs]
+        bests = [torch.zeros(len(x), dtype=torch.int32, device="cuda") for x in xs]
+
+        def heads():
+            for x, y, best in zip(xs, ys, bests):
+                ctx.matmul_argmax(W, x, y, best)
+
+        heads()
+        graph = capture(heads)
+        for k, columns in enumerate(eager):
+            for x in xs:
+                x.mul_(-1.5)
+            want = [ctx.matmul_argmax(W, x) for x in xs]
+            ctx.matmul_argmax(W, normal(7 + k, columns, cols))
+            ctx.sync()
+            fill = [torch.full((n,), 1e30, device="cuda") for n in (1 << 10, 1 << 12, 1 << 16)]
+            for best in bests:
+                best.fill_(-1)
+            graph.replay()
+            ctx.sync()
+            for y, best, (z, index) in zip(ys, bests, want):
+                assert torch.equal(best, y.argmax(dim=1).to(torch.int32)), k
+                assert torch.equal(index, z.argmax(dim=1).to(torch.int32)), k
+                assert all(rel_l2(a, b) <= 2 * REL_L2 for a, b in zip(y.cpu().numpy(), z.cpu().numpy())), k
+            assert all(bool((f == 1e30).all()) for f in fill), k
+        W.close()
+    finally:
+        ctx.close()
