@@ -625,8 +625,11 @@ int32_t rlq_mul_mat(rlq_context* ctx, const rlq_weights* w, uint32_t x_dtype, co
     }
     // the columns of one matrix are contiguous over the r2 slices it serves
     const IgStack st{n3 * w->n2, n2 / w->n2 * ncols, w->n2, n3 / w->n3, w->mat_bytes};
-    const bool plain = columns <= kDecodeMaxBatch && st.groups == 1 && x_dtype == 0 && ncols > 1;
-    // two to eight f32 columns of one matrix: the launch of rlq_matmul
+    // two to eight f32 columns of one matrix: the launch of rlq_matmul, where a
+    // single one takes them all (each launch holds back only its own columns
+    // when one of them is bad, and a refused call writes nothing)
+    const bool plain = columns <= kDecodeMaxBatch && st.groups == 1 && x_dtype == 0 && ncols > 1 &&
+                       matvec_pass_columns(w->dtype, w->rows, w->cols, columns, columns) == columns;
     if (plain && matmul_route(w->dtype, w->rows, w->cols, columns, false) == Route::kDecode) {
         HIP_TRY(decode_launch(ctx, w, (const float*)x, columns, y, nullptr, nullptr, nullptr, MvExtra{}, s));
         return ok(err);

@@ -126,6 +126,9 @@ constexpr uint32_t mv_chk(uint32_t scale, uint32_t in, uint32_t quant, uint32_t 
 // zeroes the outputs of pairs with id -1, writes *gate.
 hipError_t launch_mm_prepare(const int32_t* ids, uint64_t pairs, uint32_t experts, const uint8_t* bad, uint64_t nbad,
                              float* y, uint64_t rows, uint32_t* gate, unsigned long long* err_word, hipStream_t s);
+// Columns of the next launch of launch_matvec_ex when `left` of `batch` remain:
+// up to 8, fewer where their LDS image would not fit.
+uint32_t matvec_pass_columns(uint32_t wtype, uint64_t rows, uint64_t cols, uint64_t batch, uint64_t left);
 hipError_t launch_matvec_ex(uint32_t wtype, const uint8_t* w, uint64_t rows, uint64_t cols, const float* x,
                             const ActPlanes* pre, uint64_t batch, float* y, uint64_t ldy, const MvArgmax* am,
                             unsigned long long* err_word, int32_t* dbg_isum, int32_t* dbg_imin, const MvExtra& ex,
