@@ -741,16 +741,18 @@ static size_t route_bytes(Route r, uint32_t dtype, uint64_t batch, uint64_t cols
 
 // The GEMM of a route other than kDecode over `scratch` (route_bytes), then the
 // argmax over the stored rows (keys: one u64 per column, for more than
-// kArgmaxOneGroup rows).
+// kArgmaxOneGroup rows; am_state: kArgmaxStateBytes).
 static int32_t gemm_launch(rlq_context* ctx, const rlq_weights* w, Route r, const float* x, uint64_t batch, float* y,
-                           void* scratch, unsigned long long* keys, uint32_t* argmax, hipStream_t s, rlq_error* err) {
+                           void* scratch, unsigned long long* keys, void* am_state, uint32_t* argmax, hipStream_t s,
+                           rlq_error* err) {
+    uint32_t* refused = argmax ? argmax_refused(am_state) : nullptr;
     if (r == Route::kGemm)
-        HIP_TRY(launch_gemm_q4k(w->dev, w->rows, w->cols, x, batch, y, w->rows, scratch, ctx->err_words, nullptr, nullptr,
-                                s));
+        HIP_TRY(launch_gemm_q4k(w->dev, w->rows, w->cols, x, batch, y, w->rows, scratch, ctx->err_words, nullptr, nullptr, s,
+                                refused));
     else
         HIP_TRY(launch_igemm(w->dtype, w->dev, w->rows, w->cols, x, false, IgStack{1, batch, 1, 1, 0}, y, w->rows, scratch,
-                             ctx->err_words, s));
-    if (argmax) HIP_TRY(launch_argmax(y, batch, w->rows, keys, argmax, s));
+                             ctx->err_words, s, refused));
+    if (argmax) HIP_TRY(launch_argmax(y, batch, w->rows, keys, argmax, refused, s));
     return ok(err);
 }
 
@@ -783,8 +785,8 @@ static int32_t matmul_impl(rlq_context* ctx, const rlq_weights* w, const float* 
             HIP_TRY(ensure(ctx, ctx->column_keys, batch * sizeof(unsigned long long), s));
     }
     if (route != Route::kDecode)
-        return gemm_launch(ctx, w, route, x, batch, y, ctx->planes.p, (unsigned long long*)ctx->column_keys.p, argmax, s,
-                           err);
+        return gemm_launch(ctx, w, route, x, batch, y, ctx->planes.p, (unsigned long long*)ctx->column_keys.p, ctx->keys.p,
+                           argmax, s, err);
     // decode: the argmax is finished inside each launch
     const MvArgmax am = argmax_state(ctx->keys.p, argmax);
     HIP_TRY(decode_launch(ctx, w, x, batch, y, argmax ? &am : nullptr, nullptr, nullptr, MvExtra{}, s));
@@ -845,7 +847,7 @@ int32_t rlq_matmul_noalloc(rlq_context* ctx, const rlq_weights* w, const float* 
     // the scratch keeps the last call's contents: what must start at 0 is cleared
     if (route != Route::kDecode)
         return gemm_launch(ctx, w, route, x, batch, y, ctx->scratch + state_bytes + keys_bytes,
-                           (unsigned long long*)(ctx->scratch + state_bytes), argmax, s, err);
+                           (unsigned long long*)(ctx->scratch + state_bytes), ctx->scratch, argmax, s, err);
     if (argmax) HIP_TRY(launch_fill_u64((unsigned long long*)ctx->scratch, 1, 0ull, s));  // the arrival counter
     const MvArgmax am = argmax_state(ctx->scratch, argmax);
     HIP_TRY(launch_matvec(w->dtype, w->dev, w->rows, w->cols, x, nullptr, batch, y, w->rows, argmax ? &am : nullptr,

@@ -182,6 +182,7 @@ struct GemmArgs {
     uint64_t ldy;
     int32_t* dbg_isum;  // exact integers of token 0, or null
     int32_t* dbg_imin;
+    uint32_t* refused;  // set to whether a data error suppressed every output, or null
 };
 
 __device__ __forceinline__ f32x16 mfma16(f16x8 a, f16x8 b, f32x16 c) {
@@ -539,7 +540,9 @@ __global__ __launch_bounds__(kGemmThreads, 8 / kGemmWaves) void q4k_gemm_kernel(
 #pragma unroll
         for (int k = 0; k < 8; ++k) bad |= (int)(f[k] & 0x01010101u);
     }
-    if (__syncthreads_or(bad)) {
+    bad = __syncthreads_or(bad);
+    if (g.refused && blockIdx.x == 0 && threadIdx.x == 0) *g.refused = (uint32_t)(bad != 0);
+    if (bad) {
         // the LDS-DMA loads must land before the workgroup's LDS is released
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         return;
@@ -575,7 +578,7 @@ size_t gemm_planes_bytes(uint64_t M, uint64_t K) {
 
 hipError_t launch_gemm_q4k(const uint8_t* w, uint64_t rows, uint64_t cols, const float* x, uint64_t M, float* y,
                            uint64_t ldy, void* scratch, unsigned long long* err_word, int32_t* dbg_isum,
-                           int32_t* dbg_imin, hipStream_t s) {
+                           int32_t* dbg_imin, hipStream_t s, uint32_t* refused) {
     if (rows == 0 || cols == 0 || cols % 256 || M == 0 || rows > 0xffffffffull || cols > (1u << 30) ||
         M > (1u << 24))
         return hipErrorInvalidValue;
@@ -600,6 +603,7 @@ hipError_t launch_gemm_q4k(const uint8_t* w, uint64_t rows, uint64_t cols, const
     g.ldy = ldy;
     g.dbg_isum = dbg_isum;
     g.dbg_imin = dbg_imin;
+    g.refused = refused;
     static LdsLimit lds_plain, lds_dbg;
     e = dbg_isum ? lds_dbg.raise((const void*)q4k_gemm_kernel<true>, kGemmLds)
                  : lds_plain.raise((const void*)q4k_gemm_kernel<false>, kGemmLds);

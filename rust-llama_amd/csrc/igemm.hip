@@ -528,7 +528,15 @@ struct IgArgs {
     const uint32_t* gate;  // nonzero: the call was refused (igemm_route_kernel)
     IgMap map;
     uint64_t mat_bytes;  // between the stack's matrices
+    uint32_t* refused;   // set to whether a data error suppressed every output, or null
 };
+// A data error in any column (`bad`: one that this thread saw): the call writes
+// nothing.
+__device__ __forceinline__ bool ig_refused(const IgArgs& g, int bad) {
+    bad = __syncthreads_or(bad);
+    if (g.refused && blockIdx.x == 0 && threadIdx.x == 0) *g.refused = (uint32_t)(bad != 0);
+    return bad != 0;
+}
 
 __device__ __forceinline__ i32x16 ig_mfma(i32x4 a, i32x4 b, i32x16 c) {
     return __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b, c, 0, 0, 0);
@@ -683,10 +691,9 @@ __global__ __launch_bounds__(256, 3) void igemm_kernel(IgArgs g) {
 
     issue(0);
     load(cur, 0);
-    // a data error in any column: this call writes nothing
     int bad = 0;
     for (uint32_t i = threadIdx.x; i < g.nflags; i += 256) bad |= (int)g.flags[i];
-    if (__syncthreads_or(bad)) {
+    if (ig_refused(g, bad)) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the stage must land before its LDS is released
         return;
     }
@@ -879,7 +886,7 @@ __global__ __launch_bounds__(64 * KS) __attribute__((amdgpu_waves_per_eu(KS == 4
     ig_load<T>(r, wt + (uint64_t)c0 * W::kChunk, n, kh);
     int bad = 0;
     for (uint32_t i = threadIdx.x; i < g.nflags; i += 64 * KS) bad |= (int)g.flags[i];
-    if (__syncthreads_or(bad)) return;
+    if (ig_refused(g, bad)) return;
 
     float y[16], own[kOwn];
 #pragma unroll
@@ -1011,7 +1018,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void i
     for (int d = 0; d < D; ++d) load(buf[d], d);
     int bad = 0;
     for (uint32_t i = threadIdx.x; i < g.nflags; i += 64 * KS) bad |= (int)g.flags[i];
-    if (__syncthreads_or(bad)) return;
+    if (ig_refused(g, bad)) return;
 
     float own[2] = {0.0f, 0.0f};
     auto step = [&](Step& q, uint32_t it) {
@@ -1143,7 +1150,7 @@ static hipError_t ig_act(const void* x, bool packed, const IgMap& map, uint32_t 
 // The image of the columns, then the product.
 static hipError_t ig_run(uint32_t t, const uint8_t* w, uint64_t rows, uint64_t cols, uint64_t mat_bytes, const void* x,
                          bool packed, const IgMap& map, uint32_t tiles, bool pairs, const IgImage& im, float* y, uint64_t ldy,
-                         const uint32_t* gate, unsigned long long* err, hipStream_t s) {
+                         const uint32_t* gate, unsigned long long* err, hipStream_t s, uint32_t* refused = nullptr) {
     if (rows == 0 || cols == 0 || cols % (t == kQ8_0 ? 32 : 256) || tiles == 0 || rows > 0x7fffffffull ||
         cols > (1u << 30) || tiles > (1u << 20) || (uint64_t)tiles * im.nchunk > 0x7fffffffull)
         return hipErrorInvalidValue;
@@ -1164,6 +1171,7 @@ static hipError_t ig_run(uint32_t t, const uint8_t* w, uint64_t rows, uint64_t c
     g.gate = gate;
     g.map = map;
     g.mat_bytes = mat_bytes;
+    g.refused = refused;
     hipError_t e;
 #define RLQ_IG(TYPE)                                                                        \
     case TYPE:                                                                              \
@@ -1198,14 +1206,14 @@ size_t igemm_bytes(uint32_t t, uint64_t groups, uint64_t cpg, uint64_t cols) {
 
 hipError_t launch_igemm(uint32_t t, const uint8_t* w, uint64_t rows, uint64_t cols, const void* x, bool packed,
                         const IgStack& st, float* y, uint64_t ldy, void* scratch, unsigned long long* err_word,
-                        hipStream_t s) {
+                        hipStream_t s, uint32_t* refused) {
     const uint64_t tpg = ig_group_tiles(st.cpg), tiles = tpg * st.groups;
     if (st.cpg == 0 || st.groups == 0 || tiles > (1u << 20)) return hipErrorInvalidValue;
     IgMap map{};
     map.cpg = (uint32_t)st.cpg, map.tpg = (uint32_t)tpg, map.wn2 = (uint32_t)st.wn2, map.r3 = (uint32_t)st.r3;
     map.one = st.groups == 1;
     return ig_run(t, w, rows, cols, st.mat_bytes, x, packed, map, (uint32_t)tiles, tpg % 2 == 0,
-                  ig_carve(scratch, t, tiles, cols), y, ldy, nullptr, err_word, s);
+                  ig_carve(scratch, t, tiles, cols), y, ldy, nullptr, err_word, s, refused);
 }
 
 // ---------------------------------------------------------------------------

@@ -3472,13 +3472,12 @@ hipError_t launch_mm_prepare(const int32_t* ids, uint64_t pairs, uint32_t expert
     return hipGetLastError();
 }
 
-__global__ void argmax_finish_kernel(unsigned long long* keys, uint64_t batch, const float* y, uint64_t ldy,
-                                     uint32_t* out, bool reset) {
+__global__ void argmax_finish_kernel(const unsigned long long* keys, uint64_t batch, const float* y, uint64_t ldy,
+                                     uint32_t* out, const uint32_t* refused) {
     const uint64_t b = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= batch) return;
+    if (b >= batch || *refused) return;
     const float y0 = y[b * ldy];
     const unsigned long long k = keys[b];
-    if (reset) keys[b] = 0ull;
     // A NaN first logit is never replaced by the reference's strict `>` scan.
     out[b] = (y0 != y0 || k == 0) ? 0u : (uint32_t)(0xffffffffull - (k & 0xffffffffull));
 }
@@ -3508,8 +3507,9 @@ __global__ __launch_bounds__(256) void argmax_rows_kernel(const float* __restric
 // 32 columns 69 -> 23; 128256x4096, 16 columns 104 -> 87; 200000x512, 10 columns 52
 // against 53, 262144x256 48 against 58).
 __global__ __launch_bounds__(1024) void argmax_columns_kernel(const float* __restrict__ y, uint32_t rows,
-                                                              uint32_t* __restrict__ out) {
+                                                              uint32_t* __restrict__ out, const uint32_t* refused) {
     __shared__ unsigned long long best_s;
+    if (*refused) return;
     if (threadIdx.x == 0) best_s = 0ull;
     __syncthreads();
     const float* c = y + (uint64_t)blockIdx.x * rows;
@@ -3535,27 +3535,18 @@ __global__ __launch_bounds__(1024) void argmax_columns_kernel(const float* __res
 }
 
 hipError_t launch_argmax(const float* y, uint64_t batch, uint64_t rows, unsigned long long* keys, uint32_t* out,
-                         hipStream_t s) {
+                         const uint32_t* refused, hipStream_t s) {
     if (rows <= kArgmaxOneGroup) {
-        hipLaunchKernelGGL(argmax_columns_kernel, dim3((unsigned)batch), dim3(1024), 0, s, y, (uint32_t)rows, out);
+        hipLaunchKernelGGL(argmax_columns_kernel, dim3((unsigned)batch), dim3(1024), 0, s, y, (uint32_t)rows, out, refused);
         return hipGetLastError();
     }
     hipError_t e = launch_fill_u64(keys, batch, 0ull, s);
-    if (e == hipSuccess) e = launch_argmax_rows(y, batch, rows, keys, s);
-    return e == hipSuccess ? launch_argmax_finish(keys, batch, y, rows, out, s) : e;
-}
-
-hipError_t launch_argmax_rows(const float* y, uint64_t batch, uint64_t rows, unsigned long long* keys, hipStream_t s) {
-    const uint64_t per = (rows + 255) / 256;
-    hipLaunchKernelGGL(argmax_rows_kernel, dim3((unsigned)(per < 64 ? per : 64), (unsigned)batch), dim3(256), 0, s, y,
-                       rows, keys);
-    return hipGetLastError();
-}
-
-hipError_t launch_argmax_finish(unsigned long long* keys, uint64_t batch, const float* y, uint64_t ldy, uint32_t* out,
-                                hipStream_t s, bool reset) {
-    hipLaunchKernelGGL(argmax_finish_kernel, dim3((unsigned)((batch + 63) / 64)), dim3(64), 0, s, keys, batch, y, ldy,
-                       out, reset);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(argmax_rows_kernel, dim3(64, (unsigned)batch), dim3(256), 0, s, y, rows, keys);
+    e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(argmax_finish_kernel, dim3((unsigned)((batch + 63) / 64)), dim3(64), 0, s, keys, batch, y, rows, out,
+                       refused);
     return hipGetLastError();
 }
 

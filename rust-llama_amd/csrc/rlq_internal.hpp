@@ -71,6 +71,9 @@ constexpr size_t kArgmaxStateBytes = 256 + size_t(kArgmaxMaxGrid) * 8 * 8;
 inline MvArgmax argmax_state(void* base, uint32_t* out) {
     return MvArgmax{(unsigned long long*)((uint8_t*)base + 256), (unsigned int*)base, out};
 }
+// A word of the same state that a GEMM sets to whether a data error made it
+// write nothing, for the argmax after it.
+inline uint32_t* argmax_refused(void* base) { return (uint32_t*)((uint8_t*)base + 128); }
 
 // y[b*ldy + r] = dot(row r, activation column b) for every b < batch, in
 // launches of up to 8 columns.  The activations are quantized in the kernel
@@ -142,7 +145,7 @@ hipError_t launch_matvec_ex(uint32_t wtype, const uint8_t* w, uint64_t rows, uin
 size_t gemm_planes_bytes(uint64_t M, uint64_t K);
 hipError_t launch_gemm_q4k(const uint8_t* w, uint64_t rows, uint64_t cols, const float* x, uint64_t M, float* y,
                            uint64_t ldy, void* scratch, unsigned long long* err_word, int32_t* dbg_isum,
-                           int32_t* dbg_imin, hipStream_t s);
+                           int32_t* dbg_imin, hipStream_t s, uint32_t* refused = nullptr);
 
 // ---- igemm.hip ----
 // The int8 GEMM of every weight format.  The columns, `groups` of cpg
@@ -150,14 +153,15 @@ hipError_t launch_gemm_q4k(const uint8_t* w, uint64_t rows, uint64_t cols, const
 // rows of activation blocks taken as given; group k takes matrix
 // k / wn2 / r3 * wn2 + k % wn2 of a stack, mat_bytes apart, and
 // y[c*ldy + r] = dot(row r of its matrix, column c).  `scratch`: igemm_bytes.  A
-// data error in any column goes to `err_word` and suppresses every output.
+// data error in any column goes to `err_word` and suppresses every output;
+// `refused` (may be null) is set to whether there was one.
 struct IgStack {
     uint64_t groups, cpg, wn2, r3, mat_bytes;
 };
 size_t igemm_bytes(uint32_t t, uint64_t groups, uint64_t cpg, uint64_t cols);
 hipError_t launch_igemm(uint32_t t, const uint8_t* w, uint64_t rows, uint64_t cols, const void* x, bool packed,
                         const IgStack& st, float* y, uint64_t ldy, void* scratch, unsigned long long* err_word,
-                        hipStream_t s);
+                        hipStream_t s, uint32_t* refused = nullptr);
 // MUL_MAT_ID: product i takes matrix ids[i] of `mats` (-1: its row is 0) and
 // column i / slots * ncols + i % slots % ncols, and writes y + i * ldy.  An id
 // out of range is reported and suppresses every output, as a data error in
@@ -244,16 +248,10 @@ struct LlamaModel {
 };
 
 // The greedy argmax of the stored rows y[b*rows ..], through `keys` (batch) for
-// long rows.
+// long rows; nothing is written where `refused` holds a nonzero word.
 constexpr uint64_t kArgmaxOneGroup = 160000;
 hipError_t launch_argmax(const float* y, uint64_t batch, uint64_t rows, unsigned long long* keys, uint32_t* out,
-                         hipStream_t s);
-// Argmax keys of the stored rows y[b*rows ..] (keys zeroed beforehand).
-hipError_t launch_argmax_rows(const float* y, uint64_t batch, uint64_t rows, unsigned long long* keys, hipStream_t s);
-// Decode argmax keys into u32 indices; reset: then set the keys back to 0.
-hipError_t launch_argmax_finish(unsigned long long* keys, uint64_t batch, const float* y, uint64_t ldy, uint32_t* out,
-                                hipStream_t s, bool reset = false);
-
+                         const uint32_t* refused, hipStream_t s);
 // ---- per-device launch state (any number of host threads) ----
 constexpr int kMaxDevices = 256;
 

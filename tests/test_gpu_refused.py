@@ -37,3 +37,33 @@ def test_mul_mat_of_long_rows(t, cols, ncols):
         W.close()
     finally:
         ctx.close()
+
+
+@pytest.mark.parametrize("t,rows,cols,batch", [
+    (DT.Q6_K, 300, 512, 12), (DT.Q8_0, 300, 96, 40), (DT.Q4_K, 300, 512, 12),  # int8 GEMM
+    (DT.Q2_K, 64, 256, 262200),  # its folded flags
+    (DT.Q3_K, 160016, 256, 9),  # keys of long rows
+    (DT.Q4_K, 60000, 256, 96), (DT.Q4_K, 170000, 256, 130),  # f16 GEMM
+], ids=lambda v: v.name if isinstance(v, DT) else str(v))
+@pytest.mark.parametrize("noalloc", [False, True])
+def test_argmax_of_many_columns(t, rows, cols, batch, noalloc):
+    say("refused argmax", t.name, rows, cols, batch, "noalloc" if noalloc else "")
+    ctx = rlq.Context(0)
+    try:
+        W = rlq.Weights(ctx, t, _weights(t, rows, cols, 5), rows, cols)
+        x = torch.randn((batch, cols), generator=torch.Generator(device="cuda").manual_seed(6), device="cuda")
+        y = torch.full((batch, rows), 7.0, device="cuda")
+        best = torch.full((batch,), -5, dtype=torch.int32, device="cuda")
+        call = (lambda: ctx.matmul_noalloc(W, x, y, best)) if noalloc else (lambda: ctx.matmul_argmax(W, x, y, best))
+        x[-1, -1] = float("inf")
+        call()
+        refused(ctx, cols - 1, batch - 1)
+        if not (noalloc and batch > 200000):  # (past the static scratch: passes of 8 columns)
+            assert bool((y == 7.0).all()) and bool((best == -5).all())
+        x[-1, -1] = 0.0
+        call()
+        ctx.sync()
+        assert torch.equal(y.gather(1, best.long().view(-1, 1))[:, 0], y.amax(dim=1))
+        W.close()
+    finally:
+        ctx.close()
