@@ -163,6 +163,16 @@ hipError_t ensure(rlq_context* ctx, DevBuf& b, size_t need, hipStream_t s, bool*
     return hipSuccess;
 }
 
+// The int8 GEMM's image, which the decode kernels do without: *fits false where
+// there is no memory for it.
+hipError_t ensure_image(rlq_context* ctx, size_t need, hipStream_t s, bool* fits) {
+    const hipError_t e = ensure(ctx, ctx->planes, need, s);
+    *fits = e == hipSuccess;
+    if (e != hipErrorOutOfMemory) return e;
+    (void)hipGetLastError();
+    return hipSuccess;
+}
+
 struct DeviceGuard {
     int prev = -1;
     explicit DeviceGuard(int dev) {
@@ -640,10 +650,13 @@ int32_t rlq_mul_mat(rlq_context* ctx, const rlq_weights* w, uint32_t x_dtype, co
     // 103).  Single columns keep the decode kernels, whose sums are in the
     // reference's order.
     if (mm_igemm_takes(w->dtype, x_dtype, x) && ncols > 1) {
-        HIP_TRY(ensure(ctx, ctx->planes, igemm_bytes(w->dtype, st.groups, st.cpg, w->cols), s));
-        HIP_TRY(launch_igemm(w->dtype, w->dev, w->rows, w->cols, x, x_dtype != 0, st, y, w->rows, ctx->planes.p,
-                             ctx->err_words, s));
-        return ok(err);
+        bool fits;
+        HIP_TRY(ensure_image(ctx, igemm_bytes(w->dtype, st.groups, st.cpg, w->cols), s, &fits));
+        if (fits) {
+            HIP_TRY(launch_igemm(w->dtype, w->dev, w->rows, w->cols, x, x_dtype != 0, st, y, w->rows, ctx->planes.p,
+                                 ctx->err_words, s));
+            return ok(err);
+        }
     }
     ActPlanes planes;
     uint32_t* gate;
@@ -714,10 +727,13 @@ int32_t rlq_mul_mat_id(rlq_context* ctx, const rlq_weights* w, uint32_t x_dtype,
     const uint64_t again = (pairs - (pairs < w->n2 ? pairs : w->n2)) * w->mat_bytes;
     if (again >= (80ull << 20) && w->n2 <= kIgMaxMats && pairs <= 0x7fffffull && mm_igemm_takes(w->dtype, x_dtype, x)) {
         const IgRoute r{ids, (uint32_t)pairs, (uint32_t)w->n2, (uint32_t)columns, (uint32_t)slots, (uint32_t)ncols};
-        HIP_TRY(ensure(ctx, ctx->planes, igemm_ids_bytes(w->dtype, w->cols, r), s));
-        HIP_TRY(launch_igemm_ids(w->dtype, w->dev, w->rows, w->cols, w->mat_bytes, x, x_dtype != 0, r, y, w->rows,
-                                 ctx->planes.p, ctx->err_words, s));
-        return ok(err);
+        bool fits;
+        HIP_TRY(ensure_image(ctx, igemm_ids_bytes(w->dtype, w->cols, r), s, &fits));
+        if (fits) {
+            HIP_TRY(launch_igemm_ids(w->dtype, w->dev, w->rows, w->cols, w->mat_bytes, x, x_dtype != 0, r, y, w->rows,
+                                     ctx->planes.p, ctx->err_words, s));
+            return ok(err);
+        }
     }
     ActPlanes planes;
     uint32_t* gate;
@@ -769,13 +785,11 @@ static int32_t matmul_impl(rlq_context* ctx, const rlq_weights* w, const float* 
     // passes, which need no image (Q5_K: its columns' planes).
     if (route == Route::kIgemm && w->dtype != kQ4_K && capturing(s)) route = Route::kDecode;
     if (route != Route::kDecode) {
-        const hipError_t e = ensure(ctx, ctx->planes, route_bytes(route, w->dtype, batch, w->cols), s);
-        if (e == hipErrorOutOfMemory && w->dtype != kQ4_K) {  // decode passes need no image
-            (void)hipGetLastError();
-            route = Route::kDecode;
-        } else {
-            HIP_TRY(e);
-        }
+        const size_t need = route_bytes(route, w->dtype, batch, w->cols);
+        bool fits = true;
+        if (w->dtype == kQ4_K) HIP_TRY(ensure(ctx, ctx->planes, need, s));
+        else HIP_TRY(ensure_image(ctx, need, s, &fits));
+        if (!fits) route = Route::kDecode;
     }
     if (argmax) {  // (for a GEMM too: a capture of the same call runs decode passes)
         bool grown = false;
