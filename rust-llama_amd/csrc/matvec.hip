@@ -3536,18 +3536,26 @@ __global__ __launch_bounds__(1024) void argmax_columns_kernel(const float* __res
 
 hipError_t launch_argmax(const float* y, uint64_t batch, uint64_t rows, unsigned long long* keys, uint32_t* out,
                          const uint32_t* refused, hipStream_t s) {
-    if (rows <= kArgmaxOneGroup) {
-        hipLaunchKernelGGL(argmax_columns_kernel, dim3((unsigned)batch), dim3(1024), 0, s, y, (uint32_t)rows, out, refused);
-        return hipGetLastError();
+    // a launch takes at most 65535 grid rows and fewer than 2^32 threads (past
+    // those HIP runs a part of the grid and reports nothing)
+    constexpr uint64_t kMaxColumns = 65535;
+    for (uint64_t b = 0; b < batch; b += kMaxColumns) {
+        const uint64_t n = batch - b < kMaxColumns ? batch - b : kMaxColumns;
+        const float* yb = y + b * rows;
+        if (rows <= kArgmaxOneGroup) {
+            hipLaunchKernelGGL(argmax_columns_kernel, dim3((unsigned)n), dim3(1024), 0, s, yb, (uint32_t)rows, out + b,
+                               refused);
+        } else {
+            const hipError_t e = launch_fill_u64(keys + b, n, 0ull, s);
+            if (e != hipSuccess) return e;
+            hipLaunchKernelGGL(argmax_rows_kernel, dim3(64, (unsigned)n), dim3(256), 0, s, yb, rows, keys + b);
+            hipLaunchKernelGGL(argmax_finish_kernel, dim3((unsigned)((n + 63) / 64)), dim3(64), 0, s, keys + b, n, yb, rows,
+                               out + b, refused);
+        }
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
     }
-    hipError_t e = launch_fill_u64(keys, batch, 0ull, s);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(argmax_rows_kernel, dim3(64, (unsigned)batch), dim3(256), 0, s, y, rows, keys);
-    e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(argmax_finish_kernel, dim3((unsigned)((batch + 63) / 64)), dim3(64), 0, s, keys, batch, y, rows, out,
-                       refused);
-    return hipGetLastError();
+    return hipSuccess;
 }
 
 }  // namespace rlq

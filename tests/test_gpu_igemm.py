@@ -213,3 +213,21 @@ def test_mul_mat_broadcast_many_columns(t, ncols, packed):
         W.close()
     finally:
         ctx.close()
+
+
+@pytest.mark.parametrize("rows,batch", [(16, 4194305), (160016, 65537)])
+def test_argmax_of_very_many_columns(rows, batch):
+    """More columns than one launch of the argmax kernels takes."""
+    say("argmax", rows, "columns", batch)
+    ctx = rlq.Context(0)
+    try:
+        W = rlq.Weights(ctx, DT.Q8_0, _weights(DT.Q8_0, rows, 32, 5), rows, 32)
+        x = torch.randn((batch, 32), generator=torch.Generator(device="cuda").manual_seed(6), device="cuda")
+        best = torch.full((batch,), -1, dtype=torch.int32, device="cuda")
+        y, _ = ctx.matmul_argmax(W, x, argmax=best)
+        ctx.sync()
+        assert bool(((best >= 0) & (best < rows)).all())
+        assert torch.equal(y.gather(1, best.long().view(-1, 1))[:, 0], y.amax(dim=1))
+        W.close()
+    finally:
+        ctx.close()

@@ -63,6 +63,7 @@ def test_argmax_of_many_columns(t, rows, cols, batch, noalloc):
         x[-1, -1] = 0.0
         call()
         ctx.sync()
+        assert bool(((best >= 0) & (best < rows)).all())
         assert torch.equal(y.gather(1, best.long().view(-1, 1))[:, 0], y.amax(dim=1))
         W.close()
     finally:
