@@ -580,7 +580,7 @@ bool few_columns_igemm(uint32_t dtype, uint64_t rows, uint64_t cols, uint64_t ba
 
 Route matmul_route(uint32_t dtype, uint64_t rows, uint64_t cols, uint64_t batch, bool argmax) {
     if (batch > kDecodeMaxBatch) {
-        if (dtype != kQ4_K) return Route::kIgemm;
+        if (dtype != kQ4_K) return igemm_takes(rows, 1, batch, cols) ? Route::kIgemm : Route::kDecode;
         const uint64_t cus = (uint64_t)device_cus(), groups = (rows + 255) / 256 * ((batch + 127) / 128);
         const uint64_t rounds = (groups + cus - 1) / cus;
         return rows * ((batch + 63) / 64 * 64) < rounds * 5800000 ? Route::kIgemm : Route::kGemm;
@@ -649,7 +649,7 @@ int32_t rlq_mul_mat(rlq_context* ctx, const rlq_weights* w, uint32_t x_dtype, co
     // slices of 4 columns: 25 us against 66; one matrix, 100 columns: 25 against
     // 103).  Single columns keep the decode kernels, whose sums are in the
     // reference's order.
-    if (mm_igemm_takes(w->dtype, x_dtype, x) && ncols > 1) {
+    if (mm_igemm_takes(w->dtype, x_dtype, x) && ncols > 1 && igemm_takes(w->rows, st.groups, st.cpg, w->cols)) {
         bool fits;
         HIP_TRY(ensure_image(ctx, igemm_bytes(w->dtype, st.groups, st.cpg, w->cols), s, &fits));
         if (fits) {
@@ -725,8 +725,9 @@ int32_t rlq_mul_mat_id(rlq_context* ctx, const rlq_weights* w, uint32_t x_dtype,
     // 8 pairs 50 us against 55, 16 pairs 95 against 71, 90 pairs 526 against 72;
     // of 4096x2048: 16 pairs 20 against 26, 32 pairs 32 against 26).
     const uint64_t again = (pairs - (pairs < w->n2 ? pairs : w->n2)) * w->mat_bytes;
-    if (again >= (80ull << 20) && w->n2 <= kIgMaxMats && pairs <= 0x7fffffull && mm_igemm_takes(w->dtype, x_dtype, x)) {
-        const IgRoute r{ids, (uint32_t)pairs, (uint32_t)w->n2, (uint32_t)columns, (uint32_t)slots, (uint32_t)ncols};
+    const IgRoute r{ids, (uint32_t)pairs, (uint32_t)w->n2, (uint32_t)columns, (uint32_t)slots, (uint32_t)ncols};
+    if (again >= (80ull << 20) && pairs <= 0x7fffffull && mm_igemm_takes(w->dtype, x_dtype, x) &&
+        igemm_ids_takes(w->rows, w->cols, r)) {
         bool fits;
         HIP_TRY(ensure_image(ctx, igemm_ids_bytes(w->dtype, w->cols, r), s, &fits));
         if (fits) {

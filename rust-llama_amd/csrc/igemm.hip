@@ -1075,7 +1075,7 @@ static hipError_t ig_launch_one(IgArgs g, uint32_t tiles, hipStream_t s) {
     g.NT = (g.rows + 32 * RW - 1) / (32 * RW);
     g.MT = tiles / TT;
     const uint64_t grid = (uint64_t)g.NT * g.MT;
-    if (grid == 0 || grid > 0x7fffffffull) return hipErrorInvalidValue;
+    if (grid == 0 || grid * 256 > 0xffffffffull) return hipErrorInvalidValue;
     static LdsLimit lim;
     constexpr uint32_t lds = ig_lds<T, TT, KS>();
     const hipError_t e = lim.raise((const void*)igemm_kernel<T, TT, KS>, lds);
@@ -1089,7 +1089,7 @@ static hipError_t ig_launch_few(IgArgs g, uint32_t tiles, hipStream_t s) {
     g.NT = (g.rows + 31) / 32;
     g.MT = tiles;
     const uint64_t grid = (uint64_t)g.NT * g.MT;
-    if (grid == 0 || grid > 0x7fffffffull) return hipErrorInvalidValue;
+    if (grid == 0 || grid * 64 * KS > 0xffffffffull) return hipErrorInvalidValue;
     if constexpr (T == kQ8_0) hipLaunchKernelGGL(igemm_few_q8_kernel, dim3((unsigned)grid), dim3(512), 0, s, g);
     else hipLaunchKernelGGL((igemm_few_kernel<T, KS>), dim3((unsigned)grid), dim3(64 * KS), 0, s, g);
     return hipGetLastError();
@@ -1147,12 +1147,20 @@ static hipError_t ig_act(const void* x, bool packed, const IgMap& map, uint32_t 
     return hipGetLastError();
 }
 
+// Whether the launches stay below 2^32 threads (HIP runs a part of a larger grid
+// and reports nothing): 512 for each record of the image, 256 for each tile of
+// 128 rows x 32 columns (or of 64 x 64) of the product.  igemm_few_kernel's
+// grids are bounded by the tiles that it is chosen for.
+static bool ig_takes(uint64_t rows, uint64_t cols, uint64_t tiles) {
+    return rows <= 0x7fffffffull && cols <= (1u << 30) && tiles <= (1u << 20) &&
+           tiles * ig_chunks(cols) * 512 <= 0xffffffffull && (rows + 127) / 128 * tiles * 256 <= 0xffffffffull;
+}
+
 // The image of the columns, then the product.
 static hipError_t ig_run(uint32_t t, const uint8_t* w, uint64_t rows, uint64_t cols, uint64_t mat_bytes, const void* x,
                          bool packed, const IgMap& map, uint32_t tiles, bool pairs, const IgImage& im, float* y, uint64_t ldy,
                          const uint32_t* gate, unsigned long long* err, hipStream_t s, uint32_t* refused = nullptr) {
-    if (rows == 0 || cols == 0 || cols % (t == kQ8_0 ? 32 : 256) || tiles == 0 || rows > 0x7fffffffull ||
-        cols > (1u << 30) || tiles > (1u << 20) || (uint64_t)tiles * im.nchunk > 0x7fffffffull)
+    if (rows == 0 || cols == 0 || cols % (t == kQ8_0 ? 32 : 256) || tiles == 0 || !ig_takes(rows, cols, tiles))
         return hipErrorInvalidValue;
     IgArgs g{};
     g.w = w;
@@ -1200,6 +1208,10 @@ static uint64_t ig_group_tiles(uint64_t cpg) {
     return t > 2 ? (t + 1) & ~1ull : t;
 }
 
+bool igemm_takes(uint64_t rows, uint64_t groups, uint64_t cpg, uint64_t cols) {
+    return ig_takes(rows, cols, groups * ig_group_tiles(cpg));
+}
+
 size_t igemm_bytes(uint32_t t, uint64_t groups, uint64_t cpg, uint64_t cols) {
     return igemm_image_bytes(t, groups * ig_group_tiles(cpg), cols);
 }
@@ -1208,7 +1220,7 @@ hipError_t launch_igemm(uint32_t t, const uint8_t* w, uint64_t rows, uint64_t co
                         const IgStack& st, float* y, uint64_t ldy, void* scratch, unsigned long long* err_word,
                         hipStream_t s, uint32_t* refused) {
     const uint64_t tpg = ig_group_tiles(st.cpg), tiles = tpg * st.groups;
-    if (st.cpg == 0 || st.groups == 0 || tiles > (1u << 20)) return hipErrorInvalidValue;
+    if (st.cpg == 0 || st.groups == 0 || !ig_takes(rows, cols, tiles)) return hipErrorInvalidValue;
     IgMap map{};
     map.cpg = (uint32_t)st.cpg, map.tpg = (uint32_t)tpg, map.wn2 = (uint32_t)st.wn2, map.r3 = (uint32_t)st.r3;
     map.one = st.groups == 1;
@@ -1302,6 +1314,11 @@ static uint64_t ig_route_tiles(const IgRoute& r) {
     return (n / (u * kIgTok) + (r.products < r.mats ? r.products : r.mats) + 1) * u;
 }
 
+bool igemm_ids_takes(uint64_t rows, uint64_t cols, const IgRoute& r) {
+    return r.products > 0 && r.mats > 0 && r.mats <= kIgMaxMats && r.columns <= kIgMaxColumns &&
+           ig_takes(rows, cols, ig_route_tiles(r));
+}
+
 size_t igemm_ids_bytes(uint32_t t, uint64_t cols, const IgRoute& r) {
     const uint64_t tiles = ig_route_tiles(r);
     return igemm_image_bytes(t, tiles, cols) + 4 + tiles * (4 + kIgTok * 8);
@@ -1310,9 +1327,8 @@ size_t igemm_ids_bytes(uint32_t t, uint64_t cols, const IgRoute& r) {
 hipError_t launch_igemm_ids(uint32_t t, const uint8_t* w, uint64_t rows, uint64_t cols, uint64_t mat_bytes, const void* x,
                             bool packed, const IgRoute& r, float* y, uint64_t ldy, void* scratch,
                             unsigned long long* err_word, hipStream_t s) {
+    if (!igemm_ids_takes(rows, cols, r)) return hipErrorInvalidValue;
     const uint64_t tiles = ig_route_tiles(r);
-    if (r.products == 0 || r.mats == 0 || r.mats > kIgMaxMats || r.columns > kIgMaxColumns || tiles > (1u << 20))
-        return hipErrorInvalidValue;
     const IgImage im = ig_carve(scratch, t, tiles, cols);
     uint32_t* gate = im.flags + tiles * im.nchunk + 1;
     uint32_t* tile_mat = gate + 1;

@@ -158,6 +158,8 @@ hipError_t launch_gemm_q4k(const uint8_t* w, uint64_t rows, uint64_t cols, const
 struct IgStack {
     uint64_t groups, cpg, wn2, r3, mat_bytes;
 };
+// Whether the launches of such a call stay within a grid's limits.
+bool igemm_takes(uint64_t rows, uint64_t groups, uint64_t cpg, uint64_t cols);
 size_t igemm_bytes(uint32_t t, uint64_t groups, uint64_t cpg, uint64_t cols);
 hipError_t launch_igemm(uint32_t t, const uint8_t* w, uint64_t rows, uint64_t cols, const void* x, bool packed,
                         const IgStack& st, float* y, uint64_t ldy, void* scratch, unsigned long long* err_word,
@@ -171,6 +173,7 @@ struct IgRoute {
     uint32_t products, mats, columns, slots, ncols;
 };
 constexpr uint32_t kIgMaxMats = 1024, kIgMaxColumns = 65536;
+bool igemm_ids_takes(uint64_t rows, uint64_t cols, const IgRoute& r);
 size_t igemm_ids_bytes(uint32_t t, uint64_t cols, const IgRoute& r);
 hipError_t launch_igemm_ids(uint32_t t, const uint8_t* w, uint64_t rows, uint64_t cols, uint64_t mat_bytes, const void* x,
                             bool packed, const IgRoute& r, float* y, uint64_t ldy, void* scratch,
