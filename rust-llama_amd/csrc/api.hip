@@ -597,6 +597,52 @@ bool mm_igemm_takes(uint32_t dtype, uint32_t x_dtype, const void* x) {
     return x_dtype == 0 || (!(dtype == kQ2_K || dtype == kQ4_K || dtype == kQ5_K) && ((uintptr_t)x & 3) == 0);
 }
 
+// Whether the stack's products run on the int8 GEMM; otherwise one decode launch
+// per slice, after the quantizer and the gate.  The GEMM has two launches
+// whatever the slices, and reads a matrix once for all the slices it serves
+// (Q4_K 4096x4096, 4 matrices of 2 slices of 4 columns: 25 us against 66; one
+// matrix, 100 columns: 25 against 103).  Single columns keep the decode
+// kernels, whose sums are in the reference's order.
+//
+// A slice of two to eight columns with a matrix to itself is read once by
+// either.  The launches saved then weigh against the decode kernels' faster
+// reads of large matrices (us, decode / GEMM; matrices times rows x values,
+// columns): the line is a matrix's size by type, higher where more launches
+// are saved if the GEMM still runs its few-tile kernels there.
+//  - Q2_K: the GEMM (4 times 28672x8192, 2: 88.8 / 88.6; 32000x4096, 4: 70 / 46);
+//  - any type: the GEMM where the columns take more than half of a CU's LDS (Q5_K,
+//    2 times 4096x14336, 6: 31.7 / 26.1, 4: 28.0 / 26.3, 2: 26.4 / 26.2);
+//  - Q3_K: 2 times 14336x8192 (48 MB), 2: 35.6 / 38.0, 4 times: 67 / 60; 65536x4096
+//    110 / 138; from five columns on the GEMM (2 times 65536x4096, 6: 76 / 70);
+//  - Q4_K: to four columns, 4 times 28672x8192 (126 MB) 107 / 121, 2 times 40000x8192
+//    67 / 88; 4 times 14336x8192 61 / 53;
+//  - Q5_K: 2 times 14336x4096 (38 MB), 4: 25.2 / 26.7, 4 times: 47 / 40; 2 times
+//    14336x8192 38 / 44;
+//  - Q6_K: 4 times 32000x4096 (102 MB), 2: 90 / 100; 14336x8192 runs the GEMM alone;
+//  - Q8_0: 2 times 32000x4096 (133 MB), 2: 57.7 / 53.4, 4 times 107 / 111; 28672x8192
+//    (238 MB) 178 / 204.
+// One slice of packed columns saves one launch only: Q8_0 1024x4096 13.1 / 15.0,
+// 28672x8192 49 / 65; Q3_K 14336x4096 (24 MB), 2: 14.5 / 13.3, 4096x14336 17.0 / 18.5 and
+// with 4: 21.6 / 18.8, 14336x8192 19.9 / 21.9; Q6_K 32000x4096 25.6 / 27.7.
+bool mul_mat_igemm(const rlq_weights* w, uint32_t x_dtype, const void* x, uint64_t ncols, const IgStack& st) {
+    if (ncols == 1 || !mm_igemm_takes(w->dtype, x_dtype, x) || !igemm_takes(w->rows, st.groups, st.cpg, w->cols))
+        return false;
+    if (st.cpg > ncols || ncols > kDecodeMaxBatch || ncols * w->cols > 65536 ||
+        matvec_pass_columns(w->dtype, w->rows, w->cols, ncols, ncols) < ncols ||
+        few_columns_igemm(w->dtype, w->rows, w->cols, ncols))
+        return true;
+    uint64_t most = 0;  // MB
+    switch (w->dtype) {
+        case kQ2_K: return true;
+        case kQ3_K: most = ncols > 4 ? ~0ull >> 20 : st.groups == 1 ? 30 : (st.groups == 2 ? 44 : 60); break;
+        case kQ4_K: most = ncols > 4 ? ~0ull >> 20 : 120; break;
+        case kQ5_K: most = st.groups == 2 ? 36 : 48; break;
+        case kQ6_K: most = 100; break;
+        default: most = st.groups == 1 ? 0 : 140; break;
+    }
+    return w->mat_bytes <= most << 20;
+}
+
 // Common argument checks: (x_dtype, x alignment, column count).
 int32_t mm_check_rhs(const rlq_weights* w, uint32_t at, uint32_t x_dtype, const void* x, const float* y,
                      uint64_t columns, rlq_error* err) {
@@ -644,12 +690,7 @@ int32_t rlq_mul_mat(rlq_context* ctx, const rlq_weights* w, uint32_t x_dtype, co
         HIP_TRY(decode_launch(ctx, w, (const float*)x, columns, y, nullptr, nullptr, nullptr, MvExtra{}, s));
         return ok(err);
     }
-    // The GEMM's two launches against one decode launch per slice after the
-    // quantizer and the gate: always fewer (Q4_K 4096x4096, 4 matrices of 2
-    // slices of 4 columns: 25 us against 66; one matrix, 100 columns: 25 against
-    // 103).  Single columns keep the decode kernels, whose sums are in the
-    // reference's order.
-    if (mm_igemm_takes(w->dtype, x_dtype, x) && ncols > 1 && igemm_takes(w->rows, st.groups, st.cpg, w->cols)) {
+    if (mul_mat_igemm(w, x_dtype, x, ncols, st)) {
         bool fits;
         HIP_TRY(ensure_image(ctx, igemm_bytes(w->dtype, st.groups, st.cpg, w->cols), s, &fits));
         if (fits) {

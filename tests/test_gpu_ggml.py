@@ -332,3 +332,32 @@ def test_errors_refuse_the_whole_call(ctx):
         ctx.sync()
     assert (e.value.name, e.value.index, e.value.b) == ("NonFiniteInput", 9, 7)
     assert bool((ym == 7.0).all())
+
+
+@pytest.mark.parametrize("t,rows,cols,mats,ncols,packed", [
+    (DT.Q2_K, 9000, 4096, 2, 2, False), (DT.Q3_K, 26000, 4096, 2, 2, False), (DT.Q3_K, 26500, 4096, 2, 2, True),
+    (DT.Q3_K, 17800, 4096, 1, 2, True), (DT.Q3_K, 17900, 4096, 1, 2, True), (DT.Q4_K, 54000, 4096, 2, 4, False),
+    (DT.Q4_K, 55000, 4096, 2, 4, False), (DT.Q5_K, 13300, 4096, 2, 3, False), (DT.Q5_K, 13500, 4096, 2, 8, False),
+    (DT.Q5_K, 5000, 14336, 2, 5, False),
+    (DT.Q5_K, 13500, 4096, 3, 3, False), (DT.Q6_K, 31000, 4096, 1, 3, True), (DT.Q6_K, 32000, 4096, 2, 2, True),
+    (DT.Q8_0, 33600, 4096, 2, 4, False), (DT.Q8_0, 34000, 4096, 2, 4, True), (DT.Q8_0, 600, 512, 1, 5, True)],
+    ids=lambda v: DT(v).name if isinstance(v, DT) else str(v))
+def test_mul_mat_routes_of_few_columns(ctx, t, rows, cols, mats, ncols, packed):
+    """Slices of few columns with a matrix each, about the sizes where the GEMM
+    and the decode kernels take turns: against the products of the matrices one
+    by one, a column at a time (bitwise the oracle's in test_gpu_sweep)."""
+    say("mul_mat routes", t, rows, cols, mats, ncols, packed)
+    gen = torch.Generator(device="cuda").manual_seed(rows)
+    w = ctx.quantize(t, torch.randn((mats * rows, cols), generator=gen, device="cuda") * 0.02).reshape(-1)
+    x = torch.randn((1, mats, ncols, cols), generator=gen, device="cuda")
+    at = O.matvec_activation_dtype(int(t))
+    xs = ctx.quantize(DT(at), x.reshape(-1, cols)).reshape(1, mats, ncols, -1) if packed else x
+    y = ctx.mul_mat(rlq.Weights(ctx, t, w, rows, cols, mats), xs, DT(at) if packed else DT.F32)
+    ctx.sync()
+    for i, part in enumerate(w.reshape(mats, -1)):
+        W = rlq.Weights(ctx, t, part.contiguous(), rows, cols)
+        for c in range(ncols):
+            want = ctx.matmul(W, x[0, i, c:c + 1])[0]
+            error = (y[0, i, c] - want).norm() / want.norm()
+            assert float(error) <= (0.0 if t in EXACT else 2e-5), (i, c)
+        W.close()
