@@ -105,7 +105,8 @@ struct rlq_context {
     unsigned long long* host_err = nullptr;   // pinned readback
     // keys: the decode launches' argmax state (kArgmaxStateBytes, so never
     // replaced; its counter set to 0 when the buffer is made, and left at 0 by
-    // every launch); column_keys: one per column, the argmax of long rows after a GEMM
+    // every launch); column_keys: one per column, of an argmax after a GEMM that
+    // uses them (argmax_one_group)
     DevBuf planes, keys, column_keys, stage_in, stage_w, stage_out, gate;
     Retired* retired = nullptr;
 };
@@ -798,8 +799,8 @@ static size_t route_bytes(Route r, uint32_t dtype, uint64_t batch, uint64_t cols
 }
 
 // The GEMM of a route other than kDecode over `scratch` (route_bytes), then the
-// argmax over the stored rows (keys: one u64 per column, for more than
-// kArgmaxOneGroup rows; am_state: kArgmaxStateBytes).
+// argmax over the stored rows (keys: one u64 per column, or null where
+// argmax_one_group; am_state: kArgmaxStateBytes).
 static int32_t gemm_launch(rlq_context* ctx, const rlq_weights* w, Route r, const float* x, uint64_t batch, float* y,
                            void* scratch, unsigned long long* keys, void* am_state, uint32_t* argmax, hipStream_t s,
                            rlq_error* err) {
@@ -837,7 +838,7 @@ static int32_t matmul_impl(rlq_context* ctx, const rlq_weights* w, const float* 
         bool grown = false;
         HIP_TRY(ensure(ctx, ctx->keys, kArgmaxStateBytes, s, &grown));
         if (grown) HIP_TRY(launch_fill_u64((unsigned long long*)ctx->keys.p, 1, 0ull, s));  // the arrival counter
-        if (route != Route::kDecode && w->rows > kArgmaxOneGroup)
+        if (route != Route::kDecode && !argmax_one_group(w->rows, batch))
             HIP_TRY(ensure(ctx, ctx->column_keys, batch * sizeof(unsigned long long), s));
     }
     if (route != Route::kDecode)

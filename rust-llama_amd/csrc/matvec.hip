@@ -3482,39 +3482,15 @@ __global__ void argmax_finish_kernel(const unsigned long long* keys, uint64_t ba
     out[b] = (y0 != y0 || k == 0) ? 0u : (uint32_t)(0xffffffffull - (k & 0xffffffffull));
 }
 
-// Greedy argmax keys of stored rows (the GEMM path): keys[b] = max over r of
-// argmax_key(y[b*rows + r], r); keys must start at 0.
-__global__ __launch_bounds__(256) void argmax_rows_kernel(const float* __restrict__ y, uint64_t rows,
-                                                          unsigned long long* keys) {
-    const uint64_t b = blockIdx.y;
-    unsigned long long best = 0;
-    for (uint64_t r = (uint64_t)blockIdx.x * 256 + threadIdx.x; r < rows; r += (uint64_t)gridDim.x * 256) {
-        const unsigned long long k = argmax_key(y[b * rows + r], r);
-        best = k > best ? k : best;
-    }
-#pragma unroll
-    for (int m = 1; m < 64; m <<= 1) {
-        const unsigned long long o = __shfl_xor(best, m, 64);
-        best = o > best ? o : best;
-    }
-    if ((threadIdx.x & 63) == 0 && best) atomicMax(keys + b, best);
-}
-
-// The whole greedy argmax of stored rows of up to kArgmaxOneGroup values, one
-// workgroup per column.  Bound: one workgroup's read of a row.  In place of the
-// fill, fold and finish of the keys' path, whose workgroups meet in one atomic
-// per column (Q4_K with the product: 11268x768, 19 columns 36 -> 15 us; 32000x2048,
-// 32 columns 69 -> 23; 128256x4096, 16 columns 104 -> 87; 200000x512, 10 columns 52
-// against 53, 262144x256 48 against 58).
-__global__ __launch_bounds__(1024) void argmax_columns_kernel(const float* __restrict__ y, uint32_t rows,
-                                                              uint32_t* __restrict__ out, const uint32_t* refused) {
+// The largest argmax_key of rows first .. rows - 1, every `stride`-th run of 8 *
+// 1024 of them, of a column; in thread 0 of the 1024.
+__device__ __forceinline__ unsigned long long argmax_group(const float* __restrict__ c, uint64_t first, uint64_t stride,
+                                                           uint64_t rows) {
     __shared__ unsigned long long best_s;
-    if (*refused) return;
     if (threadIdx.x == 0) best_s = 0ull;
     __syncthreads();
-    const float* c = y + (uint64_t)blockIdx.x * rows;
     unsigned long long best = 0;
-    for (uint32_t r0 = threadIdx.x; r0 < rows; r0 += 8 * 1024) {
+    for (uint64_t r0 = first + threadIdx.x; r0 < rows; r0 += stride) {
         float v[8];
 #pragma unroll
         for (uint32_t k = 0; k < 8; ++k) v[k] = r0 + k * 1024 < rows ? c[r0 + k * 1024] : 0.0f;
@@ -3531,7 +3507,26 @@ __global__ __launch_bounds__(1024) void argmax_columns_kernel(const float* __res
     }
     if ((threadIdx.x & 63) == 0 && best) atomicMax(&best_s, best);
     __syncthreads();
-    if (threadIdx.x == 0) out[blockIdx.x] = best_s == 0 ? 0u : (uint32_t)(0xffffffffull - (best_s & 0xffffffffull));
+    return best_s;
+}
+
+// The whole greedy argmax of a column by one workgroup (argmax_one_group).  Bound:
+// the latency of its loads, 32 KB in flight.  Q4_K 11268x768, 19 columns with the
+// product 15 us (36 through keys).
+__global__ __launch_bounds__(1024) void argmax_columns_kernel(const float* __restrict__ y, uint32_t rows,
+                                                              uint32_t* __restrict__ out, const uint32_t* refused) {
+    if (*refused) return;
+    const unsigned long long best = argmax_group(y + (uint64_t)blockIdx.x * rows, 0, 8 * 1024, rows);
+    if (threadIdx.x == 0) out[blockIdx.x] = best == 0 ? 0u : (uint32_t)(0xffffffffull - (best & 0xffffffffull));
+}
+
+// The workgroups of a column (gridDim.x) each fold their runs and meet in one
+// atomic a workgroup (keys must start at 0).  With one atomic a wave of 256 and
+// one load at a time: Q6_K 300000x512, 16 columns 77 us with the product, now 47.
+__global__ __launch_bounds__(1024) void argmax_rows_kernel(const float* __restrict__ y, uint64_t rows,
+                                                           unsigned long long* keys) {
+    const unsigned long long best = argmax_group(y + blockIdx.y * rows, blockIdx.x * 8192ull, gridDim.x * 8192ull, rows);
+    if (threadIdx.x == 0 && best) atomicMax(keys + blockIdx.y, best);
 }
 
 hipError_t launch_argmax(const float* y, uint64_t batch, uint64_t rows, unsigned long long* keys, uint32_t* out,
@@ -3542,13 +3537,15 @@ hipError_t launch_argmax(const float* y, uint64_t batch, uint64_t rows, unsigned
     for (uint64_t b = 0; b < batch; b += kMaxColumns) {
         const uint64_t n = batch - b < kMaxColumns ? batch - b : kMaxColumns;
         const float* yb = y + b * rows;
-        if (rows <= kArgmaxOneGroup) {
+        if (argmax_one_group(rows, batch)) {
             hipLaunchKernelGGL(argmax_columns_kernel, dim3((unsigned)n), dim3(1024), 0, s, yb, (uint32_t)rows, out + b,
                                refused);
         } else {
             const hipError_t e = launch_fill_u64(keys + b, n, 0ull, s);
             if (e != hipSuccess) return e;
-            hipLaunchKernelGGL(argmax_rows_kernel, dim3(64, (unsigned)n), dim3(256), 0, s, yb, rows, keys + b);
+            const uint64_t runs = (rows + 8191) / 8192;
+            hipLaunchKernelGGL(argmax_rows_kernel, dim3((unsigned)(runs < 64 ? runs : 64), (unsigned)n), dim3(1024), 0, s, yb,
+                               rows, keys + b);
             hipLaunchKernelGGL(argmax_finish_kernel, dim3((unsigned)((n + 63) / 64)), dim3(64), 0, s, keys + b, n, yb, rows,
                                out + b, refused);
         }

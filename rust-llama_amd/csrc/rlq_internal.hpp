@@ -250,9 +250,14 @@ struct LlamaModel {
                     unsigned long long* err_word, hipStream_t s);
 };
 
-// The greedy argmax of the stored rows y[b*rows ..], through `keys` (batch) for
-// long rows; nothing is written where `refused` holds a nonzero word.
-constexpr uint64_t kArgmaxOneGroup = 160000;
+// The greedy argmax of the stored rows y[b*rows ..], one workgroup a column or
+// through `keys` (batch); nothing is written where `refused` holds a nonzero word.
+// One workgroup reads a row at about 20 GB/s, the keys take two launches more:
+// to 28000 rows the one (Q6_K with the product, 256 values a row, 16 columns: 24000
+// rows 15.3 us against 15.9, 32000 rows 17.5 against 16.7, 128256 rows 37 against
+// 22), and to 160000 where the columns alone fill the CUs (500 columns: 32000 rows
+// 43 against 49, 159000 rows 192 against 202).
+inline bool argmax_one_group(uint64_t rows, uint64_t batch) { return rows <= (batch > 256 ? 160000 : 28000); }
 hipError_t launch_argmax(const float* y, uint64_t batch, uint64_t rows, unsigned long long* keys, uint32_t* out,
                          const uint32_t* refused, hipStream_t s);
 // ---- per-device launch state (any number of host threads) ----

@@ -215,6 +215,28 @@ def test_mul_mat_broadcast_many_columns(t, ncols, packed):
         ctx.close()
 
 
+@pytest.mark.parametrize("rows,batch", [(28000, 10), (28001, 10), (28001, 256), (28001, 257), (160000, 257),
+                                        (160001, 257)])
+def test_argmax_at_its_lines(rows, batch):
+    """One workgroup a column, or keys, on both sides of the lines between them;
+    a zero column ties in every row."""
+    say("argmax lines", rows, batch)
+    ctx = rlq.Context(0)
+    try:
+        W = rlq.Weights(ctx, DT.Q8_0, _weights(DT.Q8_0, rows, 32, 5), rows, 32)
+        x = torch.randn((batch, 32), generator=torch.Generator(device="cuda").manual_seed(6), device="cuda")
+        x[1] = 0.0
+        y, best = ctx.matmul_argmax(W, x)
+        z, same = torch.empty_like(y), torch.empty_like(best)
+        ctx.matmul_noalloc(W, x, z, same)
+        ctx.sync()
+        assert np.array_equal(best.cpu().numpy(), y.cpu().numpy().argmax(axis=1)) and int(best[1]) == 0
+        assert torch.equal(best, same) and torch.equal(y, z)
+        W.close()
+    finally:
+        ctx.close()
+
+
 @pytest.mark.parametrize("rows,batch", [(16, 4194305), (160016, 65537)])
 def test_argmax_of_very_many_columns(rows, batch):
     """More columns than one launch of the argmax kernels takes."""
