@@ -11,7 +11,8 @@ several, odd and even, so that stages, the K split and the refilled registers
 are used again: by tiles of 32 rows x 32 columns (in brackets)
   up to 160, 16 or more chunks: 16 waves a tile; up to 512: 8; then 4 waves;
   [2304], [4617] columns in pairs: one column tile a wave (Q2_K, Q8_0), two with
-  the K split (Q3_K, Q6_K) and without;  [4126] column tiles that cannot pair.
+  the K split (Q3_K, Q6_K) and without;  [4126] two column tiles;  [4097] one,
+  which cannot pair.
 """
 import numpy as np
 import pytest
@@ -81,6 +82,7 @@ def shapes(t):
         yield 16390, nb, 275
     yield 66000, 3, 40
     yield 66000, 4, 64
+    yield 131100, 3, 20
 
 
 @pytest.mark.parametrize("t", TYPES, ids=lambda t: DT(t).name)
