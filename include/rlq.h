@@ -216,22 +216,30 @@ int32_t rlq_matmul(rlq_context *ctx, const rlq_weights *w, const float *x, uint6
 int32_t rlq_multiply(rlq_context *ctx, const rlq_weights *w, const float *x, float *y, void *stream, rlq_error *err);
 
 /* rlq_matmul followed by the greedy sampler's choice per column
- * (crates/llama-behavior/src/sampling.rs:607-613: the first strict maximum),
- * fused into the matvec epilogue: argmax[b] = index of the largest y[b*rows+r]. */
+ * (crates/llama-behavior/src/sampling.rs:607-613: the first strict maximum):
+ * argmax[b] = index of the largest y[b*rows+r] that this call writes, fused into
+ * the matvec epilogue up to 8 columns.  There the products are always those of
+ * the decode kernels, while rlq_matmul of two to eight columns may run the GEMM:
+ * then the two calls' y of Q3_K and Q6_K weights agree to the f32 order of
+ * their sums, not bit for bit (Q8_0 and Q2_K have one order in every kernel). */
 int32_t rlq_matmul_argmax(rlq_context *ctx, const rlq_weights *w, const float *x, uint64_t batch, float *y,
                           uint32_t *argmax, void *stream, rlq_error *err);
 
 /* No counterpart in the reference: for callers that cannot allocate device
  * memory (code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc).  rlq_matmul (argmax null) or rlq_matmul_argmax (argmax
- * non-null) on the same kernels, with the same results, that allocates and
- * frees nothing: the argmax keys and the GEMMs' activation images live in a static 32 MiB device array that each GPU holds until the
- * process ends.  A call with Q4_K weights whose workspace exceeds it returns
- * RLQ_SCRATCH_LIMIT (a = bytes needed, b = 33554432); for 4096 columns that is
- * a batch of about 3,700.  With other weights such a call runs passes of 8
- * columns.  Every call on one GPU, from
- * any context, shares that GPU's array: calls that overlap on one GPU (other
- * streams, other threads) race and must be ordered by the caller. */
+ * non-null) that allocates and frees nothing: the argmax keys and the GEMMs'
+ * activation images live in a static 32 MiB device array that each GPU holds
+ * until the process ends.  While the workspace fits it, the kernels are those of
+ * the allocating call and so are the results.  Where it does not, a call with
+ * Q4_K weights returns RLQ_SCRATCH_LIMIT (a = bytes needed, b = 33554432; for
+ * 4096 columns from a batch of about 3,700 on); with other weights it runs passes
+ * of 8 columns, as rlq_matmul does while its stream is being captured or when
+ * its image finds no memory: the f32 sums of Q3_K, Q5_K and Q6_K are then in another
+ * order, and a data error holds back the outputs of its own pass only.  Every
+ * call on one GPU, from any context, shares that GPU's array: calls that overlap
+ * on one GPU (other streams, other threads) race and must be ordered by the
+ * caller. */
 int32_t rlq_matmul_noalloc(rlq_context *ctx, const rlq_weights *w, const float *x, uint64_t batch, float *y,
                            uint32_t *argmax, void *stream, rlq_error *err);
 

@@ -488,8 +488,9 @@ class Context:
 
     def block_sums(self, w, x, stream=None):
         """Exact per-(row, block) integer sums of w against column 0 of x
-        ([batch, cols] or [cols], batch <= 8), from the kernel that matmul
-        uses for that batch size."""
+        ([batch, cols] or [cols], batch <= 8), from the decode kernel of that
+        batch size (matmul runs it too, or for some shapes of two and more
+        columns the int8 GEMM); more columns of Q4_K: from its f16 GEMM."""
         x2 = _columns(x, w.cols)
         nb = w.cols // (32 if w.dtype == DType.Q8_0 else 256)
         isum = torch.empty((w.rows, nb), dtype=torch.int32, device=x.device)

@@ -245,9 +245,9 @@ rlq_context* g_default = nullptr;
 
 // ---- static scratch of rlq_matmul_noalloc ----------------------------------
 // Device memory that rlq_matmul_noalloc uses instead of allocating: with an
-// argmax, the decode launches' argmax state (kArgmaxStateBytes) and, on the
-// prefill path, 8 bytes of keys per column (padded to 256); then the prefill
-// GEMM's activation image (gemm_planes_bytes).  Each device holds its own
+// argmax, the decode launches' argmax state (kArgmaxStateBytes) and, for a GEMM,
+// 8 bytes of keys per column (padded to 256); then the GEMM's activation image
+// (route_bytes).  Each device holds its own
 // copy for the life of the process.  Host code never passes the array's name
 // to a kernel (on the host it is only a handle): every use goes through the
 // device address hipGetSymbolAddress returns, taken once per device at
@@ -558,6 +558,11 @@ enum class Route { kDecode, kGemm, kIgemm };
 //    16384 rows from 8192 values (9000x8192, 3: 41.9 / 37.1; 22000: 51 / 59) or eight
 //    columns from 4096 (6000x4096 26.9 / 17.2, 5: 12.8 / 17.0).
 // Not with an argmax, which the decode kernels finish in the same launch.
+// rlq_matmul applies the rule to 32768 rows, which is as far as it was swept, not
+// where the sides meet: above, the decode kernels stay, also where the GEMM is the
+// faster one (Q2_K 34000x4096, 5: 29.3 / 20.8, 128256x4096, 5: 67.9 / 38.3; Q3_K
+// 34000x14336, 8: 155 / 71, 128256x4096, 5: 67.3 / 69.1; Q8_0 34000x14336, 5: 238 /
+// 159; Q2_K 34000x8192, 3: 30.1 / 33.1).
 bool few_columns_igemm(uint32_t dtype, uint64_t rows, uint64_t cols, uint64_t batch) {
     const bool deal = rows >= 10240 && rows <= 16384;
     const uint64_t blocks = batch * (cols / 32);

@@ -624,9 +624,10 @@ __device__ __forceinline__ void ig_put(const IgStore& o, uint64_t ldy, uint32_t 
 // 14336x4096, 512 columns 122 against 111, Q2_K 80 against 77, Q6_K the same.
 //
 // Bound: many columns, the VALU (unpacking the weights, about 11 operations
-// per four Q5_K / Q6_K values and wave, and three to five per output and block)
-// beside the MFMAs, which do not overlap: Q6_K 4096x14336, 1000 columns, 193 us =
-// 610 TOP/s (8.24 ms in passes of 8 columns) at 62 % VALU and 26 % MFMA busy.
+// per four Q5_K / Q6_K values and wave, and three to five per output and block):
+// Q6_K 4096x14336, 1000 columns, 201 us = 584 TOP/s (8.24 ms in passes of 8
+// columns) with the VALU issuing during 68 % of the cycles, the MFMAs busy during
+// 29 %, both during 17 %.
 // (Four column tiles a wave, one wave per SIMD, unpack half as often but hide
 // nothing: 220 us against 222, Q5_K 220 against 210.)  A step takes at
 // least the memory latency, about 1.4 us: few tiles have a kernel of their own.

@@ -287,8 +287,8 @@ __device__ __forceinline__ bool affine_in_range(float lo, float hi, float minimu
 }
 
 // Bound: the VALU, sixteen operations per value and grid of 16 to 21.  4096x4096
-// Q4_K / Q5_K / Q2_K 166 / 134 / 148 us; with i32 levels, a range check per value
-// and the best grid's levels copied 223 / 180 / 164.  The best grid is remembered
+// Q4_K / Q5_K / Q2_K 155 / 134 / 148 us; with i32 levels, a range check per value
+// and the best grid's levels copied 217 / 180 / 164.  The best grid is remembered
 // instead, and its levels are formed by the caller that needs them.
 template <int N, bool MAD>
 __device__ bool make_affine2(const float (&x)[N], int32_t nmax, const float (&weights)[N], float rmin, float rdelta,

@@ -116,7 +116,7 @@ def test_many_columns_need_no_scratch(t):
                          ids=["Q6_K", "Q4_K"])
 def test_recorded_argmax_outlives_larger_calls(t, rows, eager):
     """Captured output heads of one column and of nine, replayed between argmax
-    calls of ever more columns (past 160000 rows Q4_K's use one key a column)."""
+    calls of ever more columns (Q4_K's of 160016 rows use one key a column)."""
     say("captured argmax", t.name, rows)
     cols = 256
     ctx = rlq.Context(0)

@@ -4,7 +4,8 @@ against the oracle: bitwise for Q8_0 and Q2_K (one f32 order), relative L2 <=
 block terms; the bar of test_gpu_sweep).  The sizes sit at the edges of its
 tiles (16-row layout tiles, 32-row wave tiles, 32-column tiles), at one block a
 row, at K splits with fewer blocks than waves, at partial 256-value chunks and
-odd block counts of Q8_0, and on every workgroup shape of its dispatch.
+odd block counts of Q8_0, and on both sides of its dispatch's tile counts (every
+kernel with several chunks: test_gpu_igemm_exact).
 """
 import numpy as np
 import pytest
@@ -113,7 +114,8 @@ def test_flags_of_very_many_columns():
 @pytest.mark.parametrize("rows", [1, 63, 1025, 8192, 8200, 160000, 160016])
 def test_argmax_of_many_columns(rows):
     """The first of equal maxima: every row occurs twice, and a zero column ties
-    everywhere.  The lengths sit at the argmax kernel's strides and its limit."""
+    everywhere.  The lengths sit at the argmax kernels' strides (their lines:
+    test_argmax_at_its_lines)."""
     say("argmax", rows)
     w = _weights(DT.Q4_K, (rows + 1) // 2, 256, rows).reshape(-1, 144)
     w = np.concatenate([w, w])[:rows].reshape(-1)

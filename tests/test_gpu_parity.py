@@ -743,12 +743,15 @@ def test_fused_quantizer_on_golden_q8k_inputs(ctx, t, batch):
             assert np.all(np.abs(got[in_range].astype(np.float64) - want[in_range]) <= tol), i
 
 
-# ------------------------------------------------------------ prefill GEMM (Q4_K, batch > 8)
+# ------------------------------------------------------------ Q4_K, batch > 8
+# block_sums runs the f16 GEMM at every batch above 8; matmul sends it the calls
+# that fill its tiles (here the prefill shape; others in test_gpu_f16_gemm) and
+# the smaller ones to the int8 GEMM.
 
 @pytest.mark.parametrize("rows,cols,batch", [(300, 4096, 16), (300, 4096, 200), (70, 768, 129), (64, 256, 9)])
 def test_gemm_block_sums_bit_exact(ctx, rows, cols, batch):
-    """Token 0's exact per-block integers inside the prefill GEMM (two-plane
-    MFMA sums and base-128 mins digits), on partial row and token tiles."""
+    """Token 0's exact per-block integers inside the f16 GEMM, on partial row and
+    token tiles."""
     say("gemm block sums", rows, cols, batch)
     w = _weights(DT.Q4_K, rows, cols, 900 + rows)
     x = randn(901 + batch, batch * cols).reshape(batch, cols)
@@ -766,7 +769,7 @@ def test_gemm_block_sums_bit_exact(ctx, rows, cols, batch):
 
 @pytest.mark.parametrize("level,split", [(69 / 127, False), (70 / 127, True), (1.0, True)])
 def test_gemm_exact_at_the_f32_bound(ctx, level, split):
-    """The GEMM sums sc*q*q8 in f32 chains, exact while every partial sum
+    """The f16 GEMM (block_sums) sums sc*q*q8 in f32 chains, exact while every partial sum
     stays below 2^24.  Weights of all +1 encode to sc = 63, q = 15 (sc*q =
     945, the largest); token 0's blocks hold one 1.0 and 255 values `level`,
     all of one sign (no cancellation): sum |q8| = 127 + 255 round(127 level).
@@ -861,10 +864,10 @@ def test_gemm_argmax_and_errors(ctx):
 
 
 def test_gemm_many_token_tiles(ctx):
-    """Seventeen and thirty-three token tiles: every token against the oracle
-    at 2100 tokens (a partial last tile), then a non-finite value in the last
-    of 4100 tokens, which every workgroup's scan of the records' flags must
-    reach: the call reports its column and element and writes nothing."""
+    """Many column tiles (of the int8 GEMM): every token against the oracle at
+    2100 tokens (a partial last tile), then a non-finite value in the last of
+    4100 tokens, which every workgroup's scan of the flags must reach: the call
+    reports its column and element and writes nothing."""
     rows, cols = 64, 4096
     w = _weights(DT.Q4_K, rows, cols, 91)
     W = rlq.Weights(ctx, DT.Q4_K, w, rows, cols)

@@ -2,8 +2,8 @@
 around the kernels' dispatch boundaries (the 16-row tile, partial last tiles,
 the balanced deal's 6144..16384 rows and just outside it), block counts from
 1 to 72 per row (the K splits of 4 and 16 and the shared-quantization kernel
-beyond 64 blocks), and batches 1..8 (one pass of the decode kernels) and 9 or
-12 (the prefill GEMM for Q4_K, passes of at most 8 columns otherwise).
+beyond 64 blocks), and batches 1..8 (the decode kernels, and for some shapes of
+two and more columns the int8 GEMM) and 9 or 12 (the GEMMs).
 
 Bars, as in test_gpu_parity: column 0's per-block integers bitwise (every
 batch for Q4_K, up to 8 columns otherwise), every column's f32 outputs within
@@ -58,8 +58,8 @@ def _cases(n=96, seed=0x5EED, batches=BATCHES, pooled=0.7):
 
 
 CASES = _cases()
-# a second draw: row counts mostly at random, batches of 13 to 33 (two to
-# five passes of the decode kernels; Q4_K's GEMM with one ragged token tile)
+# a second draw: row counts mostly at random, batches of 13 to 33 (one or two
+# ragged column tiles of the GEMMs)
 CASES_WIDE = _cases(48, seed=0xC0FFEE, batches=(1, 2, 5, 8, 13, 16, 17, 24, 31, 33), pooled=0.3)
 
 

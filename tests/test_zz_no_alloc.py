@@ -1,5 +1,5 @@
 """rlq_matmul_noalloc (the entry point that allocates nothing; its argmax
-keys and the prefill GEMM's activation image live in the library's static
+keys and the GEMMs' activation images live in the library's static
 device scratch) against rlq_matmul / rlq_matmul_argmax, which allocate their
 scratch in the context: the same kernels, so the outputs must be bitwise
 equal.  Two calls in a row, the second with a smaller input, so stale
@@ -43,7 +43,7 @@ def inputs(seed, batch, cols):
 
 
 @pytest.mark.parametrize("t,rows,cols,batches,with_argmax", [
-    (DT.Q4_K, 1000, 4096, (300, 40), True),     # prefill GEMM: activation image in the scratch
+    (DT.Q4_K, 1000, 4096, (300, 40), True),     # int8 GEMM: activation image in the scratch
     (DT.Q4_K, 1000, 4096, (300, 40), False),
     (DT.Q4_K, 2000, 2048, (7, 3), True),        # decode kernels: only the argmax keys in the scratch
     (DT.Q5_K, 1500, 4096, (8, 7), True),        # 7-8 columns: fused quantizer here, planes kernel in rlq_matmul
