@@ -158,6 +158,33 @@ def test_dealt_products(t, rows, nb, experts, tokens, counts):
         ctx.close()
 
 
+@pytest.mark.parametrize("t", TYPES, ids=lambda t: DT(t).name)
+def test_dealt_products_of_several_columns(t):
+    """MUL_MAT_ID whose slots take turns with a token's columns (slot s: column
+    s % 3 of the token's)."""
+    rows, experts, tokens, ncols, slots = 1500, 5, 70, 3, 6
+    cols = 768 - (96 if t == DT.Q8_0 else 0)
+    say("exact ids, several columns", DT(t).name)
+    data, w, w0 = blocks(t, experts * rows, cols, 9)
+    x = fitting_columns(t, w, w0, tokens * ncols, 7)
+    ids = torch.from_numpy(np.random.default_rng(8).integers(-1, experts, (tokens, slots)).astype(np.int32)).cuda()
+    ids[3] = -1  # (columns that no product uses)
+    ctx = rlq.Context(0)
+    try:
+        W = rlq.Weights(ctx, t, data.reshape(-1), rows, cols, experts)
+        y = ctx.mul_mat_id(W, x.view(tokens, ncols, cols), ids)
+        ctx.sync()
+        w, x = w.view(experts, rows, cols), x.view(tokens, ncols, cols)
+        want = torch.zeros_like(y)
+        for e in range(experts):
+            token, slot = (ids == e).nonzero(as_tuple=True)
+            want[token, slot] = exact(x[token, slot % ncols], w[e])
+        assert torch.equal(y, want)
+        W.close()
+    finally:
+        ctx.close()
+
+
 @pytest.mark.parametrize("packed", [False, True])
 @pytest.mark.parametrize("nb", [1, 3, 4])
 @pytest.mark.parametrize("t", TYPES, ids=lambda t: DT(t).name)
