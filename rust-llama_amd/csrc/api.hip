@@ -554,9 +554,10 @@ enum class Route { kDecode, kGemm, kIgemm };
 //    8192 (24.6 / 23.3; 5: 20.3 / 23.3); Q2_K three from 8192 above 4096 rows outside
 //    it (6000x8192 17.2 / 13.0; 2500x8192 11.2 / 11.4; 12288x8192 13.7 / 16.8);
 //  - Q8_0 whose parked terms no longer fit LDS (1000x14336, 3: 25.7 / 37.9, 5: 78 /
-//    39; 30000x8192, 8: 72 / 75, x14336, 5: 166 / 131), and of more tiles than CUs to
-//    16384 rows from 8192 values (9000x8192, 3: 41.9 / 37.1; 22000: 51 / 59) or eight
-//    columns from 4096 (6000x4096 26.9 / 17.2, 5: 12.8 / 17.0).
+//    39; 30000x8192, 8: 72 / 75, 28672x11264, 6: 81.5 / 92.9, 30000x14336, 5: 166 /
+//    131), and of more tiles than CUs to 16384 rows from 8192 values (9000x8192, 3:
+//    41.9 / 37.1; 22000: 51 / 59) or eight columns from 4096 (6000x4096 26.9 / 17.2,
+//    5: 12.8 / 17.0).
 // Not with an argmax, which the decode kernels finish in the same launch.
 // rlq_matmul applies the rule to 32768 rows, which is as far as it was swept, not
 // where the sides meet: above, the decode kernels stay, also where the GEMM is the
@@ -578,7 +579,7 @@ bool few_columns_igemm(uint32_t dtype, uint64_t rows, uint64_t cols, uint64_t ba
             if (deal) return batch == 8 && cols >= 8192;
             return batch >= 5 && cols >= (rows > 16384 ? 4096 : 2048);
         case kQ8_0:
-            if (blocks > (rows <= 24576 ? 1600 : 2100)) return true;
+            if (blocks > (rows <= 24576 ? 1600 : 2200)) return true;
             return rows > 4096 && rows <= 16384 && ((batch >= 3 && cols >= 8192) || (batch == 8 && cols >= 4096));
         default: return false;
     }

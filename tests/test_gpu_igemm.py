@@ -85,6 +85,25 @@ def test_many_columns(t, rows, cols, batch):
         ctx.close()
 
 
+@pytest.mark.parametrize("rows,cols,batch", [(24500, 10272, 5), (24500, 10208, 5), (24600, 11264, 6), (24600, 14336, 5)])
+def test_few_columns_of_long_rows(rows, cols, batch):
+    """Q8_0 on both sides of the lines between the decode kernels and the GEMM:
+    one f32 order, so bitwise the one-column products."""
+    say("few columns", rows, cols, batch)
+    gen = torch.Generator(device="cuda").manual_seed(cols)
+    ctx = rlq.Context(0)
+    try:
+        w = ctx.quantize(DT.Q8_0, torch.randn((rows, cols), generator=gen, device="cuda")).reshape(-1)
+        W = rlq.Weights(ctx, DT.Q8_0, w, rows, cols)
+        x = torch.randn((batch, cols), generator=gen, device="cuda")
+        y = ctx.matmul(W, x)
+        ctx.sync()
+        assert torch.equal(y, torch.cat([ctx.matmul(W, x[b:b + 1]) for b in range(batch)]))
+        W.close()
+    finally:
+        ctx.close()
+
+
 def test_flags_of_very_many_columns():
     """Past 8192 flags one launch folds them: slices of the result equal the
     slices' own products bit for bit, and the last column's error still
