@@ -771,10 +771,19 @@ int32_t rlq_mul_mat_id(rlq_context* ctx, const rlq_weights* w, uint32_t x_dtype,
     // once, with one launch and the padding of its tiles on top: from 80 MB of
     // matrices read again on it is the faster one (8 Q4_K experts of 14336x4096:
     // 8 pairs 50 us against 55, 16 pairs 95 against 71, 90 pairs 526 against 72;
-    // of 4096x2048: 16 pairs 20 against 26, 32 pairs 32 against 26).
+    // of 4096x2048: 16 pairs 20 against 26, 32 pairs 32 against 26).  Two exceptions:
+    // Q8_0 matrices of 32 to 100 MB with long rows while every wave of the decode
+    // launch has one tile (8 experts of 4096x14336: 12 pairs 105 against 122, 13 pairs
+    // 175 against 110; of 4096x8192: 12 pairs 68 against 72, 13 pairs 104 against 74),
+    // and Q5_K ones past 100 MB, from 170 MB on (4 of 28672x8192: 5 pairs 134 against
+    // 160).
+    const uint64_t mb = w->mat_bytes >> 20;
+    const bool one_tile = w->dtype == kQ8_0 && w->cols > 4096 && mb >= 32 && mb < 100 &&
+                          pairs * layout_tiles(w->rows) <= 12ull * (uint64_t)device_cus();
+    const uint64_t least = w->dtype == kQ5_K && mb >= 100 ? 170ull << 20 : 80ull << 20;
     const uint64_t again = (pairs - (pairs < w->n2 ? pairs : w->n2)) * w->mat_bytes;
     const IgRoute r{ids, (uint32_t)pairs, (uint32_t)w->n2, (uint32_t)columns, (uint32_t)slots, (uint32_t)ncols};
-    if (again >= (80ull << 20) && pairs <= 0x7fffffull && mm_igemm_takes(w->dtype, x_dtype, x) &&
+    if (again >= least && !one_tile && pairs <= 0x7fffffull && mm_igemm_takes(w->dtype, x_dtype, x) &&
         igemm_ids_takes(w->rows, w->cols, r)) {
         bool fits;
         HIP_TRY(ensure_image(ctx, igemm_ids_bytes(w->dtype, w->cols, r), s, &fits));

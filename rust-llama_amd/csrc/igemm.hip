@@ -1109,7 +1109,10 @@ static hipError_t ig_launch_few(IgArgs g, uint32_t tiles, hipStream_t s) {
 //    = 2688: 38.0 against 38.6), 2700 of Q5_K (59.3 against 80; 256 columns = 3584:
 //    76.8 against 67.4), 3500 of Q4_K (43.0 against 45.8; 53.0 against 56.1), and
 //    4000 where column tiles cannot be paired.  Q8_0 to 1024 (4096 rows, 256
-//    columns: 40 against 48; 384 = 1536: 56 against 50).
+//    columns: 40 against 48; 384 = 1536: 56 against 50; 14336 values a row, 256: 108
+//    against 137), and to 1800 tiles of MUL_MAT_ID, whose count includes unused ones
+//    (8 experts of 4096x14336, 10 products: 1152, 110 against 163; of 4096x4096, 79
+//    tokens: 1664, 45 against 53; 128 of 512x2048, 206 tokens: 2288, 64 against 58).
 //  - Beyond, two column tiles a wave, so that the weights it unpacks serve both
 //    (14336 rows, 512 columns, Q3_K / Q5_K / Q6_K: 87 / 116 / 109 against 124 / 147 /
 //    153), with K split in two to 3000 tiles (4096 rows, 512 columns: Q3_K 36.1
@@ -1120,7 +1123,7 @@ static hipError_t ig_launch(const IgArgs& g, uint32_t tiles, bool pairs, hipStre
     const uint64_t live = g.map.tile_mat ? tiles : (uint64_t)tiles / g.map.tpg * ((g.map.cpg + kIgTok - 1) / kIgTok);
     const uint64_t n = (uint64_t)((g.rows + 31) / 32) * live;
     if constexpr (T == kQ8_0) {
-        return n <= 1024 ? ig_launch_few<T, 8>(g, tiles, s) : ig_launch_one<T, 1, 1>(g, tiles, s);
+        return n <= (g.map.tile_mat ? 1800 : 1024) ? ig_launch_few<T, 8>(g, tiles, s) : ig_launch_one<T, 1, 1>(g, tiles, s);
     } else {
         constexpr uint64_t kFew = T == kQ2_K ? 2048 : (T == kQ4_K ? 3500 : (T == kQ5_K ? 2700 : 1700));
         if (n <= 160 && g.nchunk >= 16) return ig_launch_few<T, 16>(g, tiles, s);

@@ -361,3 +361,27 @@ def test_mul_mat_routes_of_few_columns(ctx, t, rows, cols, mats, ncols, packed):
             error = (y[0, i, c] - want).norm() / want.norm()
             assert float(error) <= (0.0 if t in EXACT else 2e-5), (i, c)
         W.close()
+
+
+@pytest.mark.parametrize("t,rows,cols,experts,pairs", [
+    (DT.Q8_0, 4096, 8192, 8, 12), (DT.Q8_0, 4096, 8192, 8, 13), (DT.Q5_K, 20000, 8192, 4, 5), (DT.Q5_K, 20000, 8192, 4, 6)],
+    ids=lambda v: DT(v).name if isinstance(v, DT) else str(v))
+def test_mul_mat_id_routes_of_few_pairs(ctx, t, rows, cols, experts, pairs):
+    """Pairs about the numbers where the GEMM and the decode launch take turns:
+    against the experts' products one by one."""
+    say("mul_mat_id routes", t, rows, cols, experts, pairs)
+    gen = torch.Generator(device="cuda").manual_seed(pairs)
+    w = ctx.quantize(t, torch.randn((experts * rows, cols), generator=gen, device="cuda") * 0.02).reshape(-1)
+    x = torch.randn((pairs, 1, cols), generator=gen, device="cuda")
+    ids = torch.randint(0, experts, (pairs, 1), generator=gen, device="cuda", dtype=torch.int32)
+    W = rlq.Weights(ctx, t, w, rows, cols, experts)
+    y = ctx.mul_mat_id(W, x, ids)
+    ctx.sync()
+    W.close()
+    for e, part in enumerate(w.reshape(experts, -1)):
+        W = rlq.Weights(ctx, t, part.contiguous(), rows, cols)
+        for i in (ids[:, 0] == e).nonzero()[:, 0].tolist():
+            want = ctx.matmul(W, x[i])[0]
+            error = (y[i, 0] - want).norm() / want.norm()
+            assert float(error) <= (0.0 if t in EXACT else 2e-5), i
+        W.close()

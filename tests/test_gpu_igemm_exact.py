@@ -158,6 +158,26 @@ def test_dealt_products(t, rows, nb, experts, tokens, counts):
         ctx.close()
 
 
+@pytest.mark.parametrize("rows,cols,tokens", [(4900, 832, 45), (4800, 832, 60), (4810, 832, 60)])
+def test_dealt_q8_0_products_about_the_line(rows, cols, tokens):
+    """Q8_0 products of 1694, 1800 and 1812 tiles (of which many are unused): the
+    few-tile kernel to 1800, the staged one past it."""
+    say("exact ids about the line", rows, cols, tokens)
+    data, w, w0 = blocks(DT.Q8_0, 8 * rows, cols, 9)
+    x = fitting_columns(DT.Q8_0, w, w0, tokens, 7)
+    ids = torch.from_numpy(np.random.default_rng(8).integers(0, 8, (tokens, 1)).astype(np.int32)).cuda()
+    ctx = rlq.Context(0)
+    try:
+        W = rlq.Weights(ctx, DT.Q8_0, data.reshape(-1), rows, cols, 8)
+        y = ctx.mul_mat_id(W, x.view(tokens, 1, cols), ids)
+        ctx.sync()
+        want = torch.stack([exact(x[i:i + 1], w.view(8, rows, cols)[int(e)])[0] for i, e in enumerate(ids[:, 0].tolist())])
+        assert torch.equal(y[:, 0], want)
+        W.close()
+    finally:
+        ctx.close()
+
+
 @pytest.mark.parametrize("t", TYPES, ids=lambda t: DT(t).name)
 def test_dealt_products_of_several_columns(t):
     """MUL_MAT_ID whose slots take turns with a token's columns (slot s: column
