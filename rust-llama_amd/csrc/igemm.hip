@@ -1107,12 +1107,14 @@ static hipError_t ig_launch_few(IgArgs g, uint32_t tiles, hipStream_t s) {
 //    against 36.3 and 38.1 against 40.1; 512 columns = 2048: 43.6 against 38.1 and
 //    47.2 against 42.0), 2048 of Q2_K (32.5 against 34.7; 14336 rows, 192 columns
 //    = 2688: 38.0 against 38.6), 2700 of Q5_K (59.3 against 80; 256 columns = 3584:
-//    76.8 against 67.4), 3500 of Q4_K (43.0 against 45.8; 53.0 against 56.1), and
-//    4000 where column tiles cannot be paired.  Q8_0 to 1024 (4096 rows, 256
+//    76.8 against 67.4), 3500 of Q4_K (43.0 against 45.8; 53.0 against 56.1), 2000
+//    of it with fewer chunks than waves (256 values a row: 2048 tiles 13.2 against
+//    11.2, 28672 rows, 96 columns = 2688: 17.7 against 12.5; 768 values: 19.0 against
+//    16.6), and 4000 where column tiles cannot be paired.  Q8_0 to 1024 (4096 rows, 256
 //    columns: 40 against 48; 384 = 1536: 56 against 50; 14336 values a row, 256: 108
 //    against 137), and to 1800 tiles of MUL_MAT_ID, whose count includes unused ones
 //    (8 experts of 4096x14336, 10 products: 1152, 110 against 163; of 4096x4096, 79
-//    tokens: 1664, 45 against 53; 128 of 512x2048, 206 tokens: 2288, 64 against 58).
+//    tokens: 1664, 45 against 53; 128 of 512x2048, 206 tokens: 2256, 64 against 58).
 //  - Beyond, two column tiles a wave, so that the weights it unpacks serve both
 //    (14336 rows, 512 columns, Q3_K / Q5_K / Q6_K: 87 / 116 / 109 against 124 / 147 /
 //    153), with K split in two to 3000 tiles (4096 rows, 512 columns: Q3_K 36.1
@@ -1128,7 +1130,8 @@ static hipError_t ig_launch(const IgArgs& g, uint32_t tiles, bool pairs, hipStre
         constexpr uint64_t kFew = T == kQ2_K ? 2048 : (T == kQ4_K ? 3500 : (T == kQ5_K ? 2700 : 1700));
         if (n <= 160 && g.nchunk >= 16) return ig_launch_few<T, 16>(g, tiles, s);
         if (n <= 512) return ig_launch_few<T, 8>(g, tiles, s);
-        if (n <= (pairs ? kFew : 4000)) return ig_launch_few<T, 4>(g, tiles, s);
+        const uint64_t few = !pairs ? 4000 : (T == kQ4_K && g.nchunk < 4 ? 2000 : kFew);
+        if (n <= few) return ig_launch_few<T, 4>(g, tiles, s);
         if (!pairs || (T == kQ2_K && n <= 4000)) return ig_launch_one<T, 1, 1>(g, tiles, s);
         if constexpr (T == kQ3_K || T == kQ6_K)
             if (n <= 3000) return ig_launch_one<T, 2, 2>(g, tiles, s);

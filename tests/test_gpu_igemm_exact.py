@@ -80,6 +80,10 @@ def shapes(t):
     for nb in (1, 2, 3, 4, 9):
         yield 8187, nb, 275
         yield 16390, nb, 275
+    yield 7990, 3, 256  # [2000], [2008], [2176]: Q4_K's lines below and from four chunks
+    yield 8010, 3, 256
+    yield 8010, 1, 270
+    yield 8010, 4, 256
     yield 66000, 3, 40
     yield 66000, 4, 64
     yield 131100, 3, 20
